@@ -10,34 +10,9 @@
 #include <stdint.h>
 
 #include "attn_params.h"
+#include "bf16_ops.h"
 
 namespace clef_hip {
-
-typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
-typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
-typedef __attribute__((ext_vector_type(8))) _Float16 f16x8;
-typedef __attribute__((ext_vector_type(2))) _Float16 f16x2;
-typedef __attribute__((ext_vector_type(4))) unsigned u32x4;
-typedef __attribute__((ext_vector_type(2))) unsigned u32x2;
-
-__device__ __forceinline__ float bf_lo(unsigned w) { return __uint_as_float(w << 16); }
-__device__ __forceinline__ float bf_hi(unsigned w) { return __uint_as_float(w & 0xffff0000u); }
-__device__ __forceinline__ float bf2f(uint16_t b) { return __uint_as_float((unsigned)b << 16); }
-
-// Round-to-nearest-even pair conversion (v_cvt_pk_bf16_f32 on gfx950).
-__device__ __forceinline__ unsigned pack_bf16(float a, float b) {
-    bf16x2 v = {(__bf16)a, (__bf16)b};
-    return __builtin_bit_cast(unsigned, v);
-}
-// Round-to-nearest-even pair conversion to f16 (the text path's Q and K operands).
-__device__ __forceinline__ unsigned pack_f16(float a, float b) {
-    f16x2 v = {(_Float16)a, (_Float16)b};
-    return __builtin_bit_cast(unsigned, v);
-}
-__device__ __forceinline__ uint16_t f2bf(float a) {
-    __bf16 v = (__bf16)a;
-    return __builtin_bit_cast(uint16_t, v);
-}
 
 // sigmoid(x) = 1 / (1 + 2^(-x log2 e)) with the hardware exp2 and reciprocal (~1 ulp each).
 __device__ __forceinline__ float sigmoidf(float x) {

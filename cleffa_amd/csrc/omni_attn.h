@@ -3,26 +3,31 @@
 // omni_attn_prep, omni_attention).
 //
 // The reference keeps the P.V accumulator as an FP32 hi/lo pair so that thousands of updates
-// do not round into one component. Here the P.V product runs on the FP64 matrix cores
-// (v_mfma_f64_16x16x4f64): P and V widened to FP64 give exact products and FP64 sums, which
-// covers the same need with no VALU compensation steps. The scores stay FP32 like the
-// reference's (v_mfma_f32_16x16x4f32).
+// do not round into one component. Here the P.V accumulators are FP64.
+//
+// Both products run on the bf16 matrix cores with every FP32 operand split into three bf16 parts
+// and six products per pair (split32.h). Bounds of the item loop, per 32-key tile and SIMD: 192
+// matrix instructions of 16 cycles against 128 FP32 ones of 32 cycles and 128 FP64 ones of 64 for
+// the same work before. At 16,344 tokens, 32 / 4 heads: 27.9 -> 10.7 ms, 53% of the cycles on the matrix cores at
+// 2.1 GHz; relative error against float64 3.2e-7 -> 1.8e-7 (most of it the FP32 output's
+// rounding: the scores take 8 full-size roundings instead of 32).
 //
 // Workgroup: one wave per q head of a GQA group (nh / nkv waves), all on the same 16 query
 // rows of one record, so one 32-key K/V tile in LDS serves the whole group.
-//   S^T = K . Q^T      f32 MFMA: A = 16 keys x 4 dims of K (LDS), B = the wave's Q (registers).
-//   O^T += V^T . P^T   f64 MFMA: A = 16 dims x 4 keys of V (LDS, widened), B = P (registers).
-// S^T's A rows take key 4(r%4) + r/4 for row r, so the four scores a lane holds are the keys of
-// four consecutive 4-key steps of the P.V product: P is the next product's B operand with no
-// shuffle. The f64 product's A rows take dim 32(r%4) + 8(r/4) + n in dim tile n, so a lane's
-// accumulators cover 32 consecutive dims of its query row and the epilogue stores whole runs.
+//   S^T = K . Q^T      A = 16 keys x 32 dims of K (LDS), B = the wave's Q (registers).
+//   O^T += V^T . P^T   A = 16 dims x 32 keys of V^T (LDS), B = P (registers); FP32 over the
+//                      tile's 32 keys (the full-size terms last, one rounding), FP64 across tiles.
+// The A rows are read in a permuted order (key / dim 8 (r / 4) + 4 t + r % 4 for row r of tile t of a
+// pair), so that a lane's scores are 8 consecutive keys, the B operand of the P.V product, and
+// its outputs runs of 8 dims.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <math.h>
 #include <stdint.h>
 
-#include <utility>
+#include <type_traits>
 
+#include "split32.h"
 
 namespace clef_hip {
 namespace omni {
@@ -30,7 +35,6 @@ namespace omni {
 constexpr int HD = 128;
 constexpr int BQ = 16;                  // query rows per block (every wave of the group)
 constexpr int BK = 32;                  // keys per LDS tile
-constexpr int TILE = BK * HD;           // floats per K or V tile (16 KB)
 constexpr int SLACK = 32;               // zero rows after each kv head's T rows
 
 typedef __attribute__((ext_vector_type(4))) float f32x4;
@@ -135,8 +139,6 @@ __global__ __launch_bounds__(256) void omni_prep_kernel(PrepParams p) {
     if (bad) atomicOr(p.status, 2u);
 }
 
-typedef __attribute__((address_space(3))) void lds_void;
-
 // max over the four 16-lane rows of a wave (permlane swaps, VALU only); every lane gets it
 __device__ __forceinline__ float xrow_max(float x) {
     auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
@@ -145,35 +147,73 @@ __device__ __forceinline__ float xrow_max(float x) {
     return fmaxf(__uint_as_float(q[0]), __uint_as_float(q[1]));
 }
 
-// 16-byte chunk swizzle of a 512-byte K / V row: distinct over the 16 keys one read touches
-__device__ __forceinline__ int swz(int key) { return (key & 15) ^ ((key >> 4) << 2); }
-
-template <int OFF>
-__device__ __forceinline__ f32x4 lds_read_f4(unsigned addr) {
-    f32x4 r;
-    asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(r) : "v"(addr), "i"(OFF) : "memory");
-    return r;
-}
-template <int N>
-__device__ __forceinline__ void lds_wait_f4(f32x4 &r) {
-    asm volatile("s_waitcnt lgkmcnt(%1)" : "+v"(r) : "i"(N));
-}
-
-template <typename F, int... I>
-__device__ __forceinline__ void sfor_impl(F &&f, std::integer_sequence<int, I...>) {
-    (f(std::integral_constant<int, I>{}), ...);
-}
-template <int N, typename F>
-__device__ __forceinline__ void sfor(F &&f) {
-    sfor_impl(f, std::make_integer_sequence<int, N>{});
+// The rows of a work item in plain FP32 (FP64 sums), for items whose K, V or Q hold values that have no bf16 parts
+// (infinities, magnitudes above bf16's overflow threshold): each wave runs its head's rows one by
+// one, a lane per key for the scores and two dims per lane for the output. Slow, and only a
+// pass that is not finite (status 2) or next to FP32's limit gets here.
+__device__ __noinline__ void omni_rows_plain(const AttnParams p, int q_row0, int nq, int q_pos0, int k_row0, int k_len, int h, int kh) {
+    const int lane = threadIdx.x & 63;
+    const float *kbase = p.k_plane + ((size_t)kh * p.kvT + k_row0) * HD;
+    const float *vbase = p.v_plane + ((size_t)kh * p.kvT + k_row0) * HD;
+    for (int r = 0; r < nq; r++) {
+        const float *q = p.q_plane + ((size_t)h * p.T + q_row0 + r) * HD;
+        const int keys = min(k_len, q_pos0 + r + 1);
+        float m = -INFINITY;
+        double l = 0.0, o0 = 0.0, o1 = 0.0;
+        for (int kb = 0; kb < keys; kb += 64) {
+            const int key = kb + lane;
+            const float *k = kbase + (size_t)min(key, keys - 1) * HD;
+            float s = 0.f;
+            for (int d = 0; d < HD; d++) s = fmaf(q[d], k[d], s);
+            const float x = key < keys ? s * p.scale : -INFINITY;
+            float mx = x;
+            for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
+            const float mn = fmaxf(m, mx);
+            const float alpha = m == mn ? 1.f : expf(m - mn);
+            const float pr = x == -INFINITY ? 0.f : expf(x - mn);
+            double rs = (double)pr;
+            for (int o = 32; o > 0; o >>= 1) rs += __shfl_xor(rs, o);
+            m = mn;
+            l = l * (double)alpha + rs;
+            o0 *= (double)alpha;
+            o1 *= (double)alpha;
+            for (int j = 0; j < 64 && kb + j < keys; j++) {
+                const double pj = (double)__shfl(pr, j);
+                const float2 v = *(const float2 *)(vbase + (size_t)(kb + j) * HD + 2 * lane);
+                o0 = fma(pj, (double)v.x, o0);
+                o1 = fma(pj, (double)v.y, o1);
+            }
+        }
+        const double il = l > 0.0 ? 1.0 / l : 0.0;
+        *(float2 *)(p.out + (size_t)(q_row0 + r) * p.nh * HD + (size_t)h * HD + 2 * lane) = make_float2((float)(o0 * il), (float)(o1 * il));
+    }
 }
 
 // Grid: one workgroup per (block, kv head); wave w is q head kh * W + w.
+//
+// K and V tiles of 32 keys are split into their bf16 parts once per workgroup, on the way from
+// HBM to LDS: each thread's loads go out one tile ahead into registers, are split
+// and stored as three bf16 planes (K rows, V transposed). LDS bytes of buffer b: K planes at
+// b BUF + 8 KB p, V^T planes at b BUF + KV + 8 KB p (p = h, m, l).
+//
+// A trip has two halves: the products (S(t), and P.V(t - 1): the P.V product lags one tile) and
+// the VALU work (softmax of S(t), splits of coming tiles), each closed by a barrier. With W = 8 (two
+// waves per SIMD, one workgroup per CU) waves 4-7 run half a trip behind waves 0-3, so that on
+// each SIMD one wave's products face the other's VALU work; in step, both waves wanted the matrix
+// cores and then both the VALU, and the times added up. That takes three buffers: V(t)
+// stages K(t + 2) and V(t + 1) while the later waves still read K(t) and V(t - 1). Smaller
+// groups keep one buffer, staged between the two barriers, so that several workgroups share a CU.
 template <int W>
-__global__ __launch_bounds__(64 * W) void omni_attn_kernel(AttnParams p) {
-    __shared__ __attribute__((aligned(16))) float smem[4 * TILE];   // K0 | K1 | V0 | V1
+__global__ __launch_bounds__(64 * W, W == 4 ? 2 : 1) void omni_attn_kernel(AttnParams p) {
+    constexpr bool PP = W == 8;                            // the two wave groups half a trip apart
+    constexpr int NB = PP ? 3 : 1, AH = PP ? 1 : 0;        // buffers; tiles staged ahead
+    constexpr int PL = BK * HD * 2;                        // bytes of one plane (8 KB)
+    constexpr int KV = 3 * PL, BUF = 2 * KV;               // K planes, then V^T planes
+    constexpr int NP = 8 / W;                              // 8-element pieces of K (and of V) per thread
+    __shared__ __attribute__((aligned(16))) uint8_t smem[NB * BUF];
     const int bi = blockIdx.x / p.nkv, kh = blockIdx.x % p.nkv;
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r16 = lane & 15, g = lane >> 4;
     const int h = kh * W + wave;
     const int32_t *blk = p.blocks + 8 * bi;
@@ -181,173 +221,298 @@ __global__ __launch_bounds__(64 * W) void omni_attn_kernel(AttnParams p) {
     const int n_tiles = (k_len + BK - 1) / BK;
     const bool q_valid = r16 < nq;
     const int qpos = q_pos0 + r16;
-
-    // ---- tile fills: a tile is 16 DMA groups of 1 KB (2 keys); wave w fills groups w*16/W ...
     const float *kbase = p.k_plane + ((size_t)kh * p.kvT + k_row0) * HD;
     const float *vbase = p.v_plane + ((size_t)kh * p.kvT + k_row0) * HD;
-    constexpr int PER = 16 / W;
-    unsigned fo[PER];
+    float amax = 0.f;
+    const split32::Weights wt;
+
+    // ---- tile staging. Piece e of a thread: K dims 8 c .. 8 c + 7 of one key, V keys
+    // 8 kg .. 8 kg + 7 of one dim.
+    float kr[NP][8], vr[NP][8];
+    auto load_k = [&](int kb) {
 #pragma unroll
-    for (int j = 0; j < PER; j++) {
-        const int grp = wave * PER + j, key = 2 * grp + (lane >> 5);
-        fo[j] = (unsigned)(key * HD + ((lane & 31) ^ swz(key)) * 4) * 4u;
-    }
-    auto fill = [&](int kb, float *Ks, float *Vs) {
-        const char *kt = (const char *)(kbase + (size_t)kb * HD), *vt = (const char *)(vbase + (size_t)kb * HD);
+        for (int e = 0; e < NP; e++) {
+            const int i = tid + 64 * W * e, key = i >> 4, c = i & 15;
+            const f32x4 *s = (const f32x4 *)(kbase + (size_t)(kb + key) * HD + 8 * c);
+            const f32x4 a = s[0], b = s[1];
 #pragma unroll
-        for (int j = 0; j < PER; j++)
-            __builtin_amdgcn_global_load_lds((const void *)(kt + fo[j]), (lds_void *)(Ks + (wave * PER + j) * 256), 16, 0, 0);
+            for (int j = 0; j < 4; j++) { kr[e][j] = a[j]; kr[e][4 + j] = b[j]; }
+        }
+    };
+    auto load_v = [&](int kb) {
 #pragma unroll
-        for (int j = 0; j < PER; j++)
-            __builtin_amdgcn_global_load_lds((const void *)(vt + fo[j]), (lds_void *)(Vs + (wave * PER + j) * 256), 16, 0, 0);
+        for (int e = 0; e < NP; e++) {
+            const int i = tid + 64 * W * e, d = i & 127, kg = i >> 7;
+            const float *s = vbase + (size_t)(kb + 8 * kg) * HD + d;
+#pragma unroll
+            for (int j = 0; j < 8; j++) vr[e][j] = s[j * HD];
+        }
+    };
+    auto put = [&](uint8_t *dst, const split32::Parts &s) {
+        *(bf16x8 *)dst = s.h;
+        *(bf16x8 *)(dst + PL) = s.m;
+        *(bf16x8 *)(dst + 2 * PL) = s.l;
+    };
+    // K chunk c of key 8a + 4t + b sits at position c ^ (4a + b): the 16 rows one operand read
+    // touches then hit 16 distinct 16-byte slots.
+    auto put_k = [&](uint8_t *buf) {
+#pragma unroll
+        for (int e = 0; e < NP; e++) {
+            const int i = tid + 64 * W * e, key = i >> 4, c = i & 15;
+            amax = split32::split_amax(amax, kr[e]);
+            put(buf + key * (2 * HD) + ((c ^ ((key & 3) | ((key >> 3) << 2))) * 16), split32::split8(kr[e], wt));
+        }
+    };
+    // V^T row d: its four 8-key chunks at position kg ^ (-(d / 8) % 4) ^ ((d / 4) % 2): the 16
+    // lanes one step of a ds_read_b128 or ds_write_b128 serves, consecutive or {0-3, 12-15, 20-27}
+    // and its like, hit 16 distinct 16-byte slots.
+    auto put_v = [&](uint8_t *buf) {
+#pragma unroll
+        for (int e = 0; e < NP; e++) {
+            const int i = tid + 64 * W * e, d = i & 127, kg = i >> 7;
+            amax = split32::split_amax(amax, vr[e]);
+            put(buf + KV + d * (2 * BK) + ((kg ^ (-(d >> 3) & 3) ^ ((d >> 2) & 1)) * 16), split32::split8(vr[e], wt));
+        }
+    };
+    // Keys past the item's range (slack, or another record's) become zeros: their zero probabilities
+    // then give zero products, and what lies there cannot send the item down the plain path.
+    auto clear_k = [&](int kb) {
+#pragma unroll
+        for (int e = 0; e < NP; e++)
+#pragma unroll
+            for (int j = 0; j < 8; j++) kr[e][j] = kb + ((tid + 64 * W * e) >> 4) < k_len ? kr[e][j] : 0.f;
+    };
+    auto clear_v = [&](int kb) {
+#pragma unroll
+        for (int e = 0; e < NP; e++) {
+            const int kg = (tid + 64 * W * e) >> 7;
+#pragma unroll
+            for (int j = 0; j < 8; j++) vr[e][j] = kb + 8 * kg + j < k_len ? vr[e][j] : 0.f;
+        }
     };
 
-    // ---- per-lane LDS byte addresses of the operand reads (buffer 0; buffer 1 at +TILE floats)
-    const unsigned base = (unsigned)(uintptr_t)(const __attribute__((address_space(3))) float *)smem;
-    unsigned ka[2];   // K row of S^T A row r16 in 16-key subtile u, chunk 8g (+ j via XOR below)
-    int kx[2];
+    // ---- per-lane LDS byte addresses of the operand reads (plane h of buffer 0)
+    const unsigned lds0 = split32::lds_offset(smem);
+    unsigned ka[4];   // 32-dim step c: K row of S^T A row r16 in subtile 0 (subtile 1: + 4 rows)
 #pragma unroll
-    for (int u = 0; u < 2; u++) {
-        const int key = 16 * u + 4 * (r16 & 3) + (r16 >> 2);
-        ka[u] = base + (unsigned)key * HD * 4u;
-        kx[u] = swz(key);
-    }
-    const int vd0 = 32 * (r16 & 3) + 8 * (r16 >> 2);   // first of the 8 dims this lane's V A rows take
+    for (int c = 0; c < 4; c++) ka[c] = lds0 + (8 * (r16 >> 2) + (r16 & 3)) * (2 * HD) + (((4 * c + g) ^ r16) * 16);
+    unsigned va[2];   // V^T row of O^T A row r16 in dim tiles 0 and 1 (tiles 2u + w: + 32 u rows)
+#pragma unroll
+    for (int w = 0; w < 2; w++)
+        va[w] = lds0 + KV + (8 * (r16 >> 2) + 4 * w + (r16 & 3)) * (2 * BK) + ((g ^ (-(r16 >> 2) & 3) ^ w) * 16);
 
-    // ---- Q: lane holds Q[row r16][32 g + c], c = 0..31 (the B operand of step c)
-    float qf[32];
+    if (n_tiles > 0) {
+        load_k(0);
+        load_v(0);
+    }
+    // ---- Q: lane holds Q[row r16][32 c + 8 g + j], the B operand of step c, scaled by
+    // scale * log2 e (the scores then are exponents of 2)
+    bf16x8 qh[4], qm[4], ql[4];
     {
-        const int qr = q_valid ? r16 : 0;
-        const f32x4 *qs = (const f32x4 *)(p.q_plane + ((size_t)h * p.T + q_row0 + qr) * HD + 32 * g);
+        const float sl2 = p.scale * 1.4426950408889634f;
+        const float *qs = p.q_plane + ((size_t)h * p.T + q_row0 + (q_valid ? r16 : 0)) * HD + 8 * g;
 #pragma unroll
-        for (int j = 0; j < 8; j++) {
-            const f32x4 v = qs[j];
-            qf[4 * j] = v.x; qf[4 * j + 1] = v.y; qf[4 * j + 2] = v.z; qf[4 * j + 3] = v.w;
+        for (int c = 0; c < 4; c++) {
+            const f32x4 a = *(const f32x4 *)(qs + 32 * c), b = *(const f32x4 *)(qs + 32 * c + 4);
+            float x[8];
+#pragma unroll
+            for (int j = 0; j < 4; j++) { x[j] = a[j] * sl2; x[4 + j] = b[j] * sl2; }
+            amax = split32::split_amax(amax, x);
+            const split32::Parts s = split32::split8(x, wt);
+            qh[c] = s.h; qm[c] = s.m; ql[c] = s.l;
         }
     }
-    if (n_tiles > 0) fill(0, smem, smem + 2 * TILE);
-    __builtin_amdgcn_s_waitcnt(0);
-    __syncthreads();
+    // tile t's operands live in buffer t % NB; registers hold the tiles staged next
+    if (n_tiles > 0) {
+        if (BK > k_len) clear_k(0);
+        put_k(smem);
+        if (n_tiles > 1) load_k(BK);
+        if constexpr (PP) {
+            if (BK > k_len) clear_v(0);
+            put_v(smem);
+            if (n_tiles > 1) {
+                load_v(BK);
+                if (2 * BK > k_len) clear_k(BK);
+                put_k(smem + BUF);
+                if (n_tiles > 2) load_k(2 * BK);
+            }
+        }
+    }
+    // every LDS access of the half trip is done; the loads in flight stay so
+    auto half_barrier = [&]() {
+        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    half_barrier();
 
     f64x4 o[8];
 #pragma unroll
     for (int n = 0; n < 8; n++) o[n] = f64x4{0.0, 0.0, 0.0, 0.0};
-    float m_run = -INFINITY;
+    // the running maximum starts at the lowest finite value: a row that has seen no key yet then
+    // needs no case of its own (its probabilities are 2^-inf = 0)
+    float m_run = -3.4028235e38f;
     double l_run = 0.0;
+    bf16x8 ph, pm, pl;   // P of the previous tile
 
-    auto tile = [&](const int t, auto BUF) {
-        constexpr int buf = decltype(BUF)::value;
-        const int kb = t * BK;
-        if (t + 1 < n_tiles) fill(kb + BK, smem + (buf ^ 1) * TILE, smem + 2 * TILE + (buf ^ 1) * TILE);
-        // S^T: two 16-key subtiles, 32 four-dim steps each
-        f32x4 s[2];
+    // The products of a trip: S^T of the tile at kbuf (two 16-key subtiles, four 32-dim steps; the hh
+    // terms in one accumulator, the smaller ones in another), and O^T += V^T . P^T of the tile at
+    // vbuf (pairs of 16-dim tiles, FP32 over the tile's 32 keys, then into the FP64
+    // accumulators). Every step is six operand reads and twelve products.
+    auto products = [&](unsigned kbuf, unsigned vbuf, auto S, auto PV, float (&x)[8]) {
+        constexpr int n_s = decltype(S)::value ? 4 : 0, n = n_s + (decltype(PV)::value ? 4 : 0);
+        constexpr int LOOK = W == 4 ? 1 : 2;   // steps the reads run ahead (two waves of W = 4 share a SIMD's registers with 16 staged values more)
+        split32::Six ring[LOOK];
+        auto read = [&](auto I) {
+            constexpr int i = decltype(I)::value;
+            if constexpr (i < n_s) split32::read6<0, PL>(ring[i % LOOK], ka[i] + kbuf, ka[i] + kbuf + 4 * 2 * HD);
+            else split32::read6<32 * (i - n_s) * 2 * BK, PL>(ring[i % LOOK], va[0] + vbuf, va[1] + vbuf);
+        };
+        f32x4 s[2], sx[2], acc[2][2];
 #pragma unroll
-        for (int u = 0; u < 2; u++) {
-            f32x4 a[8];
-            sfor<8>([&](auto J) {
-                constexpr int j = decltype(J)::value;
-                a[j] = lds_read_f4<buf * TILE * 4>(ka[u] + (unsigned)(((8 * g + j) ^ kx[u]) * 16));
-            });
-            s[u] = f32x4{0.f, 0.f, 0.f, 0.f};
-            sfor<8>([&](auto J) {
-                constexpr int j = decltype(J)::value;
-                lds_wait_f4<7 - j>(a[j]);
+        for (int u = 0; u < 2; u++) s[u] = sx[u] = f32x4{0.f, 0.f, 0.f, 0.f};
+        read(std::integral_constant<int, 0>{});
+        if constexpr (LOOK > 1 && n > 1) read(std::integral_constant<int, 1>{});
+        // what step i - 1 left to the VALU, in six parts between step i's products: placed right
+        // after their own chain's end the sums would wait for it, and the products behind them
+        auto rest = [&](auto I, auto J) {
+            constexpr int i = decltype(I)::value, j = decltype(J)::value;
+            if constexpr (i == n_s && n_s > 0) {
+                if constexpr (j >= 2) {
 #pragma unroll
-                for (int e = 0; e < 4; e++)
-                    s[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j][e], qf[4 * j + e], s[u], 0, 0, 0);
-            });
-        }
-        // Online softmax. s[u][v] is the score of key kb + 16u + 4v + g for query row r16.
-        float x[2][4], mx = -INFINITY;
-#pragma unroll
-        for (int u = 0; u < 2; u++)
-#pragma unroll
-            for (int v = 0; v < 4; v++) {
-                const int key = kb + 16 * u + 4 * v + g;
-                const bool ok = q_valid && key < k_len && key <= qpos;
-                x[u][v] = ok ? s[u][v] * p.scale : -INFINITY;
-                mx = fmaxf(mx, x[u][v]);
-            }
-        const float mn = fmaxf(m_run, xrow_max(mx));
-        double pd[2][4];
-        float alpha = 1.f, rs = 0.f;
-        if (mn != -INFINITY) {
-            alpha = (m_run == -INFINITY) ? 0.f : expf(m_run - mn);
-#pragma unroll
-            for (int u = 0; u < 2; u++)
-#pragma unroll
-                for (int v = 0; v < 4; v++) {
-                    const float pv = x[u][v] == -INFINITY ? 0.f : expf(x[u][v] - mn);
-                    pd[u][v] = (double)pv;
-                    rs += pv;
+                    for (int e = 2 * (j - 2); e < 2 * (j - 1); e++) x[e] = s[e >> 2][e & 3] + sx[e >> 2][e & 3];
                 }
+            } else if constexpr (i > n_s && j >= 2) {
+                constexpr int k = i - 1 - n_s;
+#pragma unroll
+                for (int e = 2 * (j - 2); e < 2 * (j - 1); e++) o[2 * k + (e >> 2)][e & 3] += (double)acc[k & 1][e >> 2][e & 3];
+            }
+        };
+        split32::sfor<n>([&](auto I) {
+            constexpr int i = decltype(I)::value;
+            split32::wait6<(LOOK > 1 && i + 1 < n ? 6 : 0)>(ring[i % LOOK]);
+            const split32::Six a = ring[i % LOOK];
+            if constexpr (i < n_s) {
+                split32::mma6_apart(s, sx, a, qh[i], qm[i], ql[i]);
+            } else {
+                constexpr int k = i - n_s;
+                f32x4(&c)[2] = acc[k & 1];
+                c[0] = c[1] = f32x4{0.f, 0.f, 0.f, 0.f};
+                __builtin_amdgcn_sched_barrier(0);
+                split32::sfor<6>([&](auto J) {
+                    constexpr int j = decltype(J)::value;
+                    split32::mma6_term<j>(c[0], c[1], a, ph, pm, pl);
+                    rest(I, J);
+                    __builtin_amdgcn_sched_barrier(0);
+                });
+            }
+            if constexpr (i + LOOK < n) read(std::integral_constant<int, i + LOOK>{});
+        });
+        if constexpr (n > n_s) {
+#pragma unroll
+            for (int e = 0; e < 8; e++) o[6 + (e >> 2)][e & 3] += (double)acc[1][e >> 2][e & 3];
         } else {
 #pragma unroll
-            for (int u = 0; u < 2; u++)
+            for (int e = 0; e < 8; e++) x[e] = s[e >> 2][e & 3] + sx[e >> 2][e & 3];
+        }
+    };
+    // One trip (FIRST: no P.V yet). EDGE: some key of the tile lies past a row's position, or the
+    // tiles it stages may reach past the record's end.
+    int bt = 0;   // t % NB
+    auto trip = [&](const int t, auto FIRST, auto EDGE) {
+        constexpr bool first = decltype(FIRST)::value, edge = decltype(EDGE)::value;
+        const int kb = t * BK;
+        const int b_next = bt + 1 < NB ? bt + 1 : 0, b_prev = bt > 0 ? bt - 1 : NB - 1;
+        float x[8];
+        // the wave in its products goes first where both of a SIMD's waves want to issue (2.5% at
+        // 16,344 tokens; the other way round 1% slower)
+        if constexpr (PP) __builtin_amdgcn_s_setprio(1);
+        products(bt * BUF, b_prev * BUF, std::true_type{}, std::integral_constant<bool, !first>{}, x);
+        if constexpr (PP) __builtin_amdgcn_s_setprio(0);
+        half_barrier();
+        // stage K(t + 1 + AH) and V(t + AH), then load the tiles after them
+        if (!edge || t + 1 + AH < n_tiles) {
+            if (edge && kb + (2 + AH) * BK > k_len) clear_k(kb + (1 + AH) * BK);
+            put_k(smem + (PP ? b_prev : 0) * BUF);
+        }
+        if (!edge || t + 2 + AH < n_tiles) load_k(min(t + 2 + AH, n_tiles - 1) * BK);
+        if (!edge || t + AH < n_tiles) {
+            if (edge && kb + (1 + AH) * BK > k_len) clear_v(kb + AH * BK);
+            put_v(smem + (PP ? b_next : 0) * BUF);
+        }
+        if (!edge || t + 1 + AH < n_tiles) load_v(min(t + 1 + AH, n_tiles - 1) * BK);
+        // x[4 u + v] is the score (exponent of 2) of key kb + 8g + 4u + v for row r16
+        if constexpr (edge) {
+            const int lim = min(k_len - 1, qpos) - kb - 8 * g;
 #pragma unroll
-                for (int v = 0; v < 4; v++) pd[u][v] = 0.0;
+            for (int j = 0; j < 8; j++) x[j] = j <= lim ? x[j] : -INFINITY;
+        }
+        float mx = x[0];
+#pragma unroll
+        for (int j = 1; j < 8; j++) mx = fmaxf(mx, x[j]);
+        const float mn = fmaxf(m_run, xrow_max(mx));
+        const float alpha = __builtin_amdgcn_exp2f(m_run - mn);
+        float rs = 0.f;
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            x[j] = __builtin_amdgcn_exp2f(x[j] - mn);   // a masked key's -inf gives 0
+            rs += x[j];
         }
         m_run = mn;
         l_run = l_run * (double)alpha + (double)rs;
-        if (__any(alpha != 1.f)) {
-            const double ad = (double)alpha;
+        const split32::Parts pp = split32::split8(x, wt);
+        ph = pp.h; pm = pp.m; pl = pp.l;
+        if constexpr (!first) {
+            if (__any(alpha != 1.f)) {
+                // in place (as plain C++ the other path of this branch copied all 64 registers)
+                const double ad = (double)alpha;
 #pragma unroll
-            for (int n = 0; n < 8; n++) o[n] *= ad;
+                for (int n = 0; n < 8; n++)
+#pragma unroll
+                    for (int v = 0; v < 4; v++) {
+                        double d = o[n][v];
+                        asm("v_mul_f64 %0, %0, %1" : "+v"(d) : "v"(ad));
+                        o[n][v] = d;
+                    }
+            }
         }
-        // O^T += V^T . P^T: 8 four-key steps (u, v), each 8 dim tiles
-        f32x4 vb[2][2];
-        auto vread = [&](auto U, auto V, f32x4 *dst) {
-            constexpr int u = decltype(U)::value, v = decltype(V)::value;
-            const int key = 16 * u + 4 * v + g;
-            const unsigned row = base + (unsigned)(2 * TILE + key * HD) * 4u;
-            const int x = swz(key);
-            dst[0] = lds_read_f4<buf * TILE * 4>(row + (unsigned)((((vd0 >> 2)) ^ x) * 16));
-            dst[1] = lds_read_f4<buf * TILE * 4>(row + (unsigned)((((vd0 >> 2) + 1) ^ x) * 16));
-        };
-        vread(std::integral_constant<int, 0>{}, std::integral_constant<int, 0>{}, vb[0]);
-        sfor<8>([&](auto S) {
-            constexpr int st = decltype(S)::value, u = st >> 2, v = st & 3, cur = st & 1;
-            if constexpr (st + 1 < 8)
-                vread(std::integral_constant<int, ((st + 1) >> 2)>{}, std::integral_constant<int, (st + 1) & 3>{}, vb[cur ^ 1]);
-            if constexpr (st + 1 < 8) {
-                lds_wait_f4<2>(vb[cur][0]);
-                lds_wait_f4<2>(vb[cur][1]);
-            } else {
-                lds_wait_f4<0>(vb[cur][0]);
-                lds_wait_f4<0>(vb[cur][1]);
-            }
-            const double b = pd[u][v];
-#pragma unroll
-            for (int n = 0; n < 8; n++) {
-                const float a = n < 4 ? vb[cur][0][n] : vb[cur][1][n - 4];
-                o[n] = __builtin_amdgcn_mfma_f64_16x16x4f64((double)a, b, o[n], 0, 0, 0);
-            }
-        });
-        __builtin_amdgcn_s_waitcnt(0);
-        __syncthreads();
+        half_barrier();
+        bt = b_next;
     };
-    for (int t = 0; t < n_tiles; t += 2) {
-        tile(t, std::integral_constant<int, 0>{});
-        if (t + 1 < n_tiles) tile(t + 1, std::integral_constant<int, 1>{});
+    using T = std::true_type;
+    using F = std::false_type;
+    // trips whose tile every row sees whole, with the tiles they stage inside the record
+    const int n_inner = min((q_pos0 + 1) / BK, k_len / BK - AH - 1);
+    if (n_tiles > 0) {
+        const bool late = PP && wave >= W / 2;
+        if (late) half_barrier();
+        int t = 0;
+        if (n_inner > 0) trip(t++, T{}, F{});
+        else trip(t++, T{}, T{});
+        for (; t < n_inner; t++) trip(t, F{}, F{});
+        for (; t < n_tiles; t++) trip(t, F{}, T{});
+        if (PP && !late) half_barrier();
+        float none[8];
+        products(0, (bt > 0 ? bt - 1 : NB - 1) * BUF, F{}, T{}, none);
     }
 
-    // ---- epilogue: O = O^T / l; lane holds dims 32 g + 8 v + n of row r16 (accumulator n, entry v)
+    // ---- epilogue: O = O^T / l; lane holds dims 32 u + 8 g + 4 w + v of row r16 (tile 2u + w, entry v)
     double l_row = l_run;
     l_row += __shfl_xor(l_row, 16);
     l_row += __shfl_xor(l_row, 32);
+    if (__syncthreads_or(split32::split_bad(amax))) {
+        omni_rows_plain(p, q_row0, nq, q_pos0, k_row0, k_len, h, kh);
+        return;
+    }
     if (q_valid) {
         const double il = l_row > 0.0 ? 1.0 / l_row : 0.0;
-        float *dst = p.out + (size_t)(q_row0 + r16) * p.nh * HD + (size_t)h * HD + 32 * g;
+        float *dst = p.out + (size_t)(q_row0 + r16) * p.nh * HD + (size_t)h * HD + 8 * g;
 #pragma unroll
-        for (int v = 0; v < 4; v++) {
-            f32x4 w0, w1;
+        for (int n = 0; n < 8; n++) {
+            f32x4 w;
 #pragma unroll
-            for (int n = 0; n < 4; n++) {
-                w0[n] = (float)(o[n][v] * il);
-                w1[n] = (float)(o[n + 4][v] * il);
-            }
-            *(f32x4 *)(dst + 8 * v) = w0;
-            *(f32x4 *)(dst + 8 * v + 4) = w1;
+            for (int v = 0; v < 4; v++) w[v] = (float)(o[n][v] * il);
+            *(f32x4 *)(dst + 32 * (n >> 1) + 4 * (n & 1)) = w;
         }
     }
 }

@@ -1,0 +1,127 @@
+// FP32 products on the bf16 matrix cores of CDNA4 (gfx950).
+//
+// An FP32 value is the exact sum of three bf16 values: h = bf16(x), m = bf16(x - h),
+// l = bf16(x - h - m), each rounded to nearest even, so |m| <= 2^-9 |x| and |l| <= 2^-18 |x|. A product a . b then
+// takes the six terms hh, hm, mh, hl, lh, mm; the three left out (ml, lm, ll) are at most 2^-26 |a b| together, below the
+// rounding of one FP32 product (2^-24 |a b|). The terms run on v_mfma_f32_16x16x32_bf16 with FP32
+// accumulation, the small ones first or into accumulators of their own, so that the full-size sum
+// is rounded once per 32-deep step, where v_mfma_f32_16x16x4f32 rounds it once per 4. Six bf16
+// products cost 6 / 16 of the FP32 matrix instructions' time (2.5 PFLOP/s against 157 TFLOP/s).
+//
+// The split is exact for finite |x| below bf16's overflow threshold (0x7f7f8000) whose parts stay
+// clear of the subnormals (|x| above about 2^-108; below, an absolute 2^-133 is lost). Larger and infinite
+// values give infinite or NaN parts: kernels note the largest magnitude they split
+// (split_amax / split_bad) and recompute such work items with plain FP32 arithmetic. A NaN gives NaN.
+#pragma once
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+#include <utility>
+
+#include "bf16_ops.h"
+
+namespace clef_hip {
+namespace split32 {
+
+typedef __attribute__((ext_vector_type(4))) float f32x4;
+
+// The parts of eight consecutive contraction elements: one 16x16x32 operand each.
+struct Parts {
+    bf16x8 h, m, l;
+};
+
+// x - h of one element of a packed pair: v_dot2_f32_bf16 with weights (-1, 0) or (0, -1), one instruction
+// for the widening and the subtraction. The difference is exact, so the instruction's own rounding does not
+// enter (checked over the exponent range against the two-instruction form). The weights sit in
+// registers the compiler cannot see through: as constants it encoded (-1, 0) wrongly.
+struct Weights {
+    unsigned lo, hi;
+    __device__ __forceinline__ Weights() : lo(0x0000bf80u), hi(0xbf800000u) { asm("" : "+s"(lo), "+s"(hi)); }
+};
+__device__ __forceinline__ float minus_lo(unsigned pair, const Weights &w, float x) {
+    return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, pair), __builtin_bit_cast(bf16x2, w.lo), x, false);
+}
+__device__ __forceinline__ float minus_hi(unsigned pair, const Weights &w, float x) {
+    return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, pair), __builtin_bit_cast(bf16x2, w.hi), x, false);
+}
+
+__device__ __forceinline__ Parts split8(const float (&x)[8], const Weights &w) {
+    u32x4 h, m, l;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const float a = x[2 * i], b = x[2 * i + 1];
+        h[i] = pack_bf16(a, b);
+        const float a1 = minus_lo(h[i], w, a), b1 = minus_hi(h[i], w, b);
+        m[i] = pack_bf16(a1, b1);
+        l[i] = pack_bf16(minus_lo(m[i], w, a1), minus_hi(m[i], w, b1));
+    }
+    return {__builtin_bit_cast(bf16x8, h), __builtin_bit_cast(bf16x8, m), __builtin_bit_cast(bf16x8, l)};
+}
+
+// Largest magnitude of a running maximum and eight values (a NaN does not count: its parts are NaN).
+__device__ __forceinline__ float split_amax(float amax, const float (&x)[8]) {
+#pragma unroll
+    for (int i = 0; i < 8; i += 2) asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(amax) : "v"(x[i]), "v"(x[i + 1]));
+    return amax;
+}
+// whether a value of that magnitude has no finite parts
+__device__ __forceinline__ bool split_bad(float amax) { return amax >= __uint_as_float(0x7f7f8000u); }
+
+template <typename F, int... I>
+__device__ __forceinline__ void sfor_impl(F &&f, std::integer_sequence<int, I...>) {
+    (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, typename F>
+__device__ __forceinline__ void sfor(F &&f) {
+    sfor_impl(f, std::make_integer_sequence<int, N>{});
+}
+
+// Operand reads run ahead of their products: six ds_read_b128 (the h, m, l parts of two operands) as
+// one asm statement, and a wait that names them before their use.
+__device__ __forceinline__ unsigned lds_offset(const void *p) { return (unsigned)(uintptr_t)(const __attribute__((address_space(3))) void *)p; }
+struct Six {
+    bf16x8 h0, m0, l0, h1, m1, l1;
+};
+// operands at a + O and b + O, their parts PL bytes apart
+template <int O, int PL>
+__device__ __forceinline__ void read6(Six &r, unsigned a, unsigned b) {
+    asm volatile("ds_read_b128 %0, %6 offset:%8\n\tds_read_b128 %3, %7 offset:%8\n\t"
+                 "ds_read_b128 %1, %6 offset:%9\n\tds_read_b128 %4, %7 offset:%9\n\t"
+                 "ds_read_b128 %2, %6 offset:%10\n\tds_read_b128 %5, %7 offset:%10"
+                 : "=&v"(r.h0), "=&v"(r.m0), "=&v"(r.l0), "=&v"(r.h1), "=&v"(r.m1), "=&v"(r.l1)
+                 : "v"(a), "v"(b), "i"(O), "i"(O + PL), "i"(O + 2 * PL) : "memory");
+}
+template <int N>   // until at most N LDS operations are outstanding
+__device__ __forceinline__ void wait6(Six &r) {
+    asm volatile("s_waitcnt lgkmcnt(%6)" : "+v"(r.h0), "+v"(r.m0), "+v"(r.l0), "+v"(r.h1), "+v"(r.m1), "+v"(r.l1) : "i"(N) : "memory");
+}
+
+__device__ __forceinline__ f32x4 mma(bf16x8 a, bf16x8 b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0); }
+
+// Two products of split operands against one split operand: hh into big, the five smaller terms
+// into small (the caller may pass one accumulator for both: the small terms then come first).
+__device__ __forceinline__ void mma6_apart(f32x4 (&big)[2], f32x4 (&small)[2], const Six &a, bf16x8 bh, bf16x8 bm, bf16x8 bl) {
+    small[0] = mma(a.l0, bh, small[0]);
+    small[1] = mma(a.l1, bh, small[1]);
+    big[0] = mma(a.h0, bh, big[0]);
+    big[1] = mma(a.h1, bh, big[1]);
+    small[0] = mma(a.h0, bl, small[0]);
+    small[1] = mma(a.h1, bl, small[1]);
+    small[0] = mma(a.m0, bm, small[0]);
+    small[1] = mma(a.m1, bm, small[1]);
+    small[0] = mma(a.m0, bh, small[0]);
+    small[1] = mma(a.m1, bh, small[1]);
+    small[0] = mma(a.h0, bm, small[0]);
+    small[1] = mma(a.h1, bm, small[1]);
+}
+// term j of the six, smallest first, of two products into one accumulator each
+template <int J>
+__device__ __forceinline__ void mma6_term(f32x4 &c0, f32x4 &c1, const Six &a, bf16x8 bh, bf16x8 bm, bf16x8 bl) {
+    constexpr int A[6] = {2, 0, 1, 1, 0, 0}, B[6] = {0, 2, 1, 0, 1, 0};   // parts: 0 h, 1 m, 2 l
+    const bf16x8 b = B[J] == 0 ? bh : B[J] == 1 ? bm : bl;
+    c0 = mma(A[J] == 0 ? a.h0 : A[J] == 1 ? a.m0 : a.l0, b, c0);
+    c1 = mma(A[J] == 0 ? a.h1 : A[J] == 1 ? a.m1 : a.l1, b, c1);
+}
+
+}  // namespace split32
+}  // namespace clef_hip

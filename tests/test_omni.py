@@ -214,3 +214,82 @@ def test_omni_long_flat():
         assert np.abs(got - want[None, None, :]).max() < 6e-8, "long accumulation lost constant values"
         res.append(got.copy())
     assert np.array_equal(res[0].view(np.uint32), res[1].view(np.uint32))
+
+
+def _planes(T, nh, nkv, seed):
+    """Q, K, V planes [heads][T][128] as the prologue leaves them (RMS-normalised rows), f32."""
+    rng = np.random.default_rng(seed)
+    Q, K, V = (rng.standard_normal((n, T, 128)).astype(np.float32) for n in (nh, nkv, nkv))
+    return [x / np.sqrt((x.astype(np.float64) ** 2).mean(-1, keepdims=True)).astype(np.float32) for x in (Q, K)] + [V]
+
+
+def _attend(Q, K, V, cu):
+    """The attention kernel on given planes (slack rows and rows between records as they come)."""
+    nh, T, _ = Q.shape
+    nkv = K.shape[0]
+    att, plan = OmniAttention(nh, nkv), OmniPlan(cu)
+    q, k, v = att.planes(T)
+    q.copy_(torch.from_numpy(Q))
+    for dst, src in ((k, K), (v, V)):
+        dst.zero_()
+        dst[:, :T].copy_(torch.from_numpy(src))
+    out = torch.full((T, nh * 128), float("nan"), device="cuda")
+    att.attention(q, k, v, plan, out=out)
+    torch.cuda.synchronize()
+    return out.cpu().numpy()
+
+
+def _reference(Q, K, V, cu):
+    with np.errstate(all="ignore"):
+        return oracle.attention(*[x.astype(np.float64) for x in (Q, K, V)], np.asarray(cu, np.int32), None, True, 128 ** -0.5, None)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nh,nkv", [(8, 1), (8, 2), (6, 3), (3, 3)])
+def test_omni_group_widths_and_tile_edges(nh, nkv):
+    """Every group width (8, 4, 2, 1 heads) over records that end on, before and after 32-key
+    tiles. Bound: the scores' FP32 rounding (|s| up to ~40 in exponents of 2, 8 roundings of 2^-24
+    each: 2e-5 of P at most, averaged over keys) leaves outputs of size ~1 within 3e-6, as the
+    reference's tests ask."""
+    print(f"[omni] widths {nh}/{nkv}", flush=True)
+    lens = [1, 16, 17, 31, 32, 33, 48, 63, 64, 65, 95, 96, 97, 130, 257]
+    cu = np.concatenate([[0], np.cumsum(lens)])
+    Q, K, V = _planes(int(cu[-1]), nh, nkv, seed=nh)
+    got, want = _attend(Q, K, V, cu), _reference(Q, K, V, cu)
+    assert np.abs(got - want).max() < 3e-6
+    alone = _attend(Q[:, :lens[0]], K[:, :lens[0]], V[:, :lens[0]], [0, lens[0]])
+    assert np.array_equal(alone.view(np.uint32), got[:lens[0]].view(np.uint32))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nh,nkv", [(8, 1), (4, 1)])
+@pytest.mark.parametrize("which", ["v_inf", "v_big", "v_small", "k_minus", "q_big"])
+def test_omni_values_without_bf16_parts(nh, nkv, which):
+    """Infinities and magnitudes above bf16's overflow threshold (3.39e38) have no bf16 parts: such
+    items run in plain FP32, and records beside them stay bit for bit what they are alone."""
+    print(f"[omni] values {which} {nh}/{nkv}", flush=True)
+    lens = [40, 70, 21]
+    cu = np.concatenate([[0], np.cumsum(lens)])
+    Q, K, V = _planes(int(cu[-1]), nh, nkv, seed=5)
+    row = 40 + 33
+    if which == "v_inf":
+        V[0, row, 5], V[0, row + 20, 9] = np.inf, -np.inf
+    elif which == "v_big":       # finite in FP32, above bf16's largest
+        V[0, row, 5] = np.float32(3.395e38)
+    elif which == "v_small":     # parts near the subnormals: relative to V, not to the others
+        V[:] *= np.float32(1e-28)
+    elif which == "k_minus":     # scores of minus infinity for that key: no weight
+        Q[:, :, 7], K[0, row, 7] = np.abs(Q[:, :, 7]) + np.float32(0.1), -np.inf
+    else:
+        Q[1, row, 3], K[0, :, 3] = np.float32(3.395e38), np.float32(1e-38)
+    got, want = _attend(Q, K, V, cu), _reference(Q, K, V, cu)
+    fine = np.isfinite(want)
+    assert np.array_equal(got[~fine], want[~fine].astype(np.float32), equal_nan=True)
+    scale = np.abs(V[np.isfinite(V) & (np.abs(V) < 1e30)]).max() if which != "v_big" else 1.0
+    big = np.maximum(np.abs(want[fine]), scale)
+    assert (np.abs(got[fine] - want[fine]) / big).max() < 3e-6
+    for r in (0, 2):             # the clean records
+        a, b = cu[r], cu[r + 1]
+        if which in ("v_inf", "v_big"):
+            alone = _attend(Q[:, a:b], K[:, a:b], V[:, a:b], [0, b - a])
+            assert np.array_equal(alone.view(np.uint32), got[a:b].view(np.uint32))
