@@ -462,7 +462,7 @@ def main():
         core_ms = statistics.median(rounds["core"])
         achieved = flops / (core_ms * 1e-3) / 1e12
         peak = PEAK_F32_MFMA if a.fp32 else PEAK_BF16_TFLOPS
-        kname = f"attn_text_f32_kernel<{info['nh'] // w['nkv']}>" if a.fp32 else "attn_text_kernel<64>"
+        kname = "attn_text_f32_kernel" if a.fp32 else "attn_text_kernel<64>"
         res["roofline"] = {"bound": "mfma", "kernel": kname,
                            "achieved": round(achieved, 2), "peak": peak, "unit": "TFLOP/s",
                            "frac": round(achieved / peak, 4),

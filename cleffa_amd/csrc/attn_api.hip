@@ -184,16 +184,6 @@ bool vis_run(const clef_hip_vis_args *a, uint16_t *q_plane, uint16_t *k_plane, u
     return launch_ok("attn_vis", err, errlen);
 }
 
-// The FP32 core over the (16-row sub-block, kv head, head chunk) items (the kernel's LDS allows
-// one workgroup per CU): a chunk of W <= 6 heads runs two waves per head, each on half of the
-// head dims, so that the waves spread evenly over the four SIMDs (12 for the 6 q heads of a
-// 24 / 4 model); 7 and 8 heads run one wave per head.
-template <int W>
-void launch_f32(const text32::Params &p, long grid, hipStream_t s) {
-    constexpr int X = W <= 6 ? 2 : 1;
-    hipLaunchKernelGGL((text32::attn_text_f32_kernel<W, X>), dim3((unsigned)grid), dim3(64 * W * X), 0, s, p);
-}
-
 bool core_f32(const clef_hip_attn_args *a, void *stream, char *err, size_t errlen) {
     text32::Params p;
     p.qkv = (const float *)a->qkv; p.q_norm = a->q_norm; p.pos3 = a->pos3; p.inv_freq = a->inv_freq;
@@ -203,32 +193,20 @@ bool core_f32(const clef_hip_attn_args *a, void *stream, char *err, size_t errle
     p.row = a->row; p.kvT = a->kvT; p.nh = a->nh; p.nkv = a->nkv; p.n_rot = a->n_rot;
     p.causal = a->causal ? 1 : 0; p.gate = a->gate ? 1 : 0; p.out_type = a->out_type;
     p.eps = a->eps; p.scale = a->scale; p.f16_lim = f16_limit(a->f16_lim);
-    // a kv group of G q heads runs as ceil(G / 8) chunks of W = ceil(G / chunks) heads
     const int group = a->nh / a->nkv;
-    p.n_chunks = (group + 7) / 8;
-    const int W = (group + p.n_chunks - 1) / p.n_chunks;
-    p.n_blk = a->n_blk;
-    const long n_items = (long)a->n_blk * text32::SUB * a->nkv * p.n_chunks;
-    if (n_items > 0x7fffffffL) return fail(err, errlen, "grid too large");
-    // One workgroup per item, dispatched in the items' longest-first order: the hardware hands
-    // each free CU the next item, which balanced C1 better (594 us) than a persistent grid of
-    // one workgroup per CU over a static snake order (660 us; C2 within 1%).
-    // CLEF_HIP_F32_PERSISTENT=1 selects the persistent grid.
-    long grid = n_items;
-    const char *ge = getenv("CLEF_HIP_F32_PERSISTENT");
     const long cus = device_cus();
-    if (ge && ge[0] == '1' && cus > 0 && cus < n_items) grid = cus;
-    hipStream_t s = (hipStream_t)stream;
-    switch (W) {
-        case 1: launch_f32<1>(p, grid, s); break;
-        case 2: launch_f32<2>(p, grid, s); break;
-        case 3: launch_f32<3>(p, grid, s); break;
-        case 4: launch_f32<4>(p, grid, s); break;
-        case 5: launch_f32<5>(p, grid, s); break;
-        case 6: launch_f32<6>(p, grid, s); break;
-        case 7: launch_f32<7>(p, grid, s); break;
-        default: launch_f32<8>(p, grid, s); break;
-    }
+    auto items = [&](int slots) {
+        const text32::Shape f = text32::f32_shape(slots, group);
+        return (long)a->n_blk * (text32::BLK / (16 * f.R)) * (group / f.k) * a->nkv;
+    };
+    // Eight waves of 16 rows share each K / V tile's split; a pass that gives them too few items to
+    // fill the CUs runs items of four such waves, the others only helping with the splits.
+    p.slots = items(8) >= cus ? 8 : 4;
+    // one workgroup per item, dispatched in the items' longest-first order: the hardware hands
+    // each free CU the next item
+    const long n_items = items(p.slots);
+    if (n_items > 0x7fffffffL) return fail(err, errlen, "grid too large");
+    hipLaunchKernelGGL(text32::attn_text_f32_kernel, dim3((unsigned)n_items), dim3(64 * text32::NW), 0, (hipStream_t)stream, p);
     return launch_ok("attn_text_f32", err, errlen);
 }
 

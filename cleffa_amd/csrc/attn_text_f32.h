@@ -10,50 +10,53 @@
 //   sigmoid(gate) (the second half of the head's row), written through act16 (bf16, or f16
 //   that saturates and flags the record) or as f32.
 //
-// Everything is FP32: the products run on v_mfma_f32_16x16x4f32 (FP32 operands, FP32
-// accumulation), the softmax in FP32 VALU (exp2 domain). Key tiles start at the record's first key, so a
-// record's arithmetic does not depend on what is packed with it.
+// Everything is held in FP32; the products run on the bf16 matrix cores with every operand split
+// into three bf16 parts and six products per pair (split32.h), FP32 accumulation, the softmax in FP32
+// VALU (exp2 domain). Key tiles start at the record's first key, so a record's arithmetic does not
+// depend on what is packed with it.
 //
-// Workgroup: a chunk of W <= 8 q heads of the GQA group (a group of more than 8 heads runs as
-// several chunks), X = 1 or 2 waves per head, all on the same 16 query rows, so one 32-key K / V
-// tile in LDS (64 KB, double buffered: 128 KB) serves the chunk. With two waves per head each
-// takes half of the head dims (see attn_text_f32_kernel).
-//   S^T = K . Q^T      A = 16 keys x 4 dims of K (LDS), B = the wave's Q (registers).
-//   O^T += V^T . P^T   A = 16 dims x 4 keys of V (LDS), B = P (registers).
-// Lane l = 16 g + r. S^T's A row r takes key 4(r % 4) + r / 4 of the 16-key subtile, so the four
-// scores a lane holds (accumulator rows 4g + v) are keys 4v + g: the B operand of the four 4-key
-// steps of the P.V product, with no shuffle. In S^T, lane (g, r) reads chunks 16g + j of its
-// key's K row (dims 64g + 4j + e); the K rows are padded to 1,040 bytes so those 16 rows fall in
-// distinct banks. In the P.V product, read j of lane r takes chunk 16j + r of its key's V row: a
-// read's 16 lanes cover 256 contiguous bytes. The A row r of dim tile 4j + e is then dim
-// 64j + 4r + e, and accumulator v of lane (g, r) in tile 4j + e holds dim 64j + 16g + 4v + e of
-// query row r. Every LDS read is a per-lane base register plus an immediate offset.
+// Workgroup: NW waves of 16 query rows, R row groups x k heads of one kv group (f32_shape), so one
+// 32-key K / V tile in LDS (three bf16 planes each, 96 KB) serves up to 128 rows.
+//   S^T = K . Q^T      A = 16 keys x 32 dims of K (LDS), B = the wave's Q (registers, 96 of them).
+//   O^T += V^T . P^T   A = 16 dims x 32 keys of V^T (LDS), B = P (registers).
+// The A rows are read in a permuted order (key / dim 8 (r / 4) + 4 t + r % 4 for row r of tile t of
+// a pair), so that a lane's scores are 8 consecutive keys, the B operand of the P.V product, and
+// its outputs runs of 8 dims.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <math.h>
 #include <stdint.h>
 
-#include <utility>
+#include <type_traits>
 
 #include "attn_kernels.h"
 #include "clef_hip_attn.h"
+#include "split32.h"
 
 namespace clef_hip {
 namespace text32 {
 
 constexpr int HD = 256;
-constexpr int BQ = 16;                  // query rows per workgroup
-constexpr int SUB = 128 / BQ;           // workgroups per 128-row plan block
+constexpr int BLK = 128;                // query rows of a plan block
 constexpr int BK = 32;                  // keys per LDS tile
-constexpr int ROW = HD + 4;             // LDS floats per key row: 1,040 bytes, so the 16 rows
-                                        // one K read touches start 16 bytes apart in the banks
-constexpr int TILE = BK * ROW;          // floats per K or V tile (32.5 KB)
-constexpr int TB = TILE * 4;            // bytes per tile
-constexpr int RUN = 4;                  // K chunks read ahead of their products
-constexpr int NRUN = 16 / RUN;
+constexpr int NW = 8;                   // waves per workgroup
 
 typedef __attribute__((ext_vector_type(4))) float f32x4;
-typedef __attribute__((address_space(3))) void lds_void;
+
+// Row groups of 16 rows and heads of a full item of `slots` waves, for kv groups of `group` heads: two
+// heads where the group is even (a causal item's last tiles are masked for its first rows, so
+// fewer rows waste less), one otherwise.
+struct Shape {
+    int R, k;
+};
+__host__ __device__ inline Shape f32_shape(int slots, int group) { return group % 2 == 0 ? Shape{slots / 2, 2} : Shape{slots, 1}; }
+// Heads of an item that holds only `rows` rows: the largest divisor of the group that fits.
+__host__ __device__ inline int f32_heads(int slots, int rows, int group) {
+    const int wph = (rows + 15) / 16;
+    for (int k = slots / wph; k > 1; k--)
+        if (group % k == 0) return k;
+    return 1;
+}
 
 struct PrepParams {
     const float *qkv;           // [T][row]
@@ -78,7 +81,7 @@ struct Params {
     void *out;
     int32_t *ovf;
     int row, kvT, nh, nkv, n_rot, causal, gate, out_type;
-    int n_blk, n_chunks;        // plan blocks; head chunks per kv group (ceil(group / 8))
+    int slots;                  // waves of an item that hold rows: 8, or 4 (the others only stage tiles)
     float eps, scale, f16_lim;
 };
 
@@ -137,346 +140,376 @@ __device__ __forceinline__ float xrow_max(float x) {
     return fmaxf(__uint_as_float(q[0]), __uint_as_float(q[1]));
 }
 
-template <int OFF>
-__device__ __forceinline__ f32x4 lds_read_f4(unsigned addr) {
-    f32x4 r;
-    asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(r) : "v"(addr), "i"(OFF) : "memory");
-    return r;
-}
-template <int N>
-__device__ __forceinline__ void lds_wait_f4(f32x4 &r) {
-    asm volatile("s_waitcnt lgkmcnt(%1)" : "+v"(r) : "i"(N));
+// The rows of a wave in plain FP32, for items whose Q, K or V hold values that have no bf16 parts
+// (infinities, magnitudes above bf16's overflow threshold): one row after the other, a lane per key
+// for the scores and four dims per lane for q and the output.
+__device__ __noinline__ void text_rows_plain(const Params p, int q_row0, int nq, int q_pos0, int k_row0, int k_len, int h, int kh, int32_t *flag) {
+    const int lane = threadIdx.x & 63;
+    const float *kbase = p.k_plane + ((size_t)kh * p.kvT + k_row0) * HD;
+    const float *vbase = p.v_plane + ((size_t)kh * p.kvT + k_row0) * HD;
+    for (int r = 0; r < nq; r++) {
+        const int t = q_row0 + r;
+        const float *src = p.qkv + (size_t)t * p.row + (size_t)h * 2 * HD + 4 * lane;
+        f32x4 q = *(const f32x4 *)src;
+        if (p.q_norm) {
+            float ss = q.x * q.x + q.y * q.y + q.z * q.z + q.w * q.w;
+            for (int o = 32; o > 0; o >>= 1) ss += __shfl_xor(ss, o);
+            const float inv = 1.0f / sqrtf(ss / (float)HD + p.eps);
+            const f32x4 w = *(const f32x4 *)(p.q_norm + 4 * lane);
+            for (int e = 0; e < 4; e++) q[e] = q[e] * inv * w[e];
+        }
+        if (p.n_rot) {   // dims i (lanes 0-7) and i + 32 (lanes 8-15)
+            for (int e = 0; e < 4; e++) {
+                const float other = __shfl_xor(q[e], 8);
+                if (lane < 16) {
+                    float c, s;
+                    rope_cs_f32(p.pos3, p.inv_freq, t, (4 * lane + e) & 31, &c, &s);
+                    q[e] = lane < 8 ? q[e] * c - other * s : q[e] * c + other * s;
+                }
+            }
+        }
+        const int keys = p.causal ? min(k_len, q_pos0 + r + 1) : k_len;
+        float m = -INFINITY, l = 0.f;
+        f32x4 o = {0.f, 0.f, 0.f, 0.f};
+        for (int kb = 0; kb < keys; kb += 64) {
+            const int key = kb + lane;
+            const float *k = kbase + (size_t)min(key, keys - 1) * HD;
+            float s = 0.f;
+            for (int c = 0; c < 64; c++) {
+                const f32x4 kv = *(const f32x4 *)(k + 4 * c);
+                for (int e = 0; e < 4; e++) s = fmaf(__shfl(q[e], c), kv[e], s);
+            }
+            const float x = key < keys ? s * p.scale : -INFINITY;
+            float mx = x;
+            for (int i = 32; i > 0; i >>= 1) mx = fmaxf(mx, __shfl_xor(mx, i));
+            const float mn = fmaxf(m, mx);
+            const float alpha = m == mn ? 1.f : expf(m - mn);
+            const float pr = x == -INFINITY ? 0.f : expf(x - mn);
+            float rs = pr;
+            for (int i = 32; i > 0; i >>= 1) rs += __shfl_xor(rs, i);
+            m = mn;
+            l = l * alpha + rs;
+            o *= alpha;
+            for (int j = 0; j < 64 && kb + j < keys; j++) {
+                const float pj = __shfl(pr, j);
+                const f32x4 v = *(const f32x4 *)(vbase + (size_t)(kb + j) * HD + 4 * lane);
+                for (int e = 0; e < 4; e++) o[e] = fmaf(pj, v[e], o[e]);
+            }
+        }
+        const float il = l > 0.f ? 1.0f / l : 0.f;
+        f32x4 w;
+        for (int e = 0; e < 4; e++) w[e] = o[e] * il;
+        if (p.gate) {
+            const f32x4 gv = *(const f32x4 *)(src + HD);
+            for (int e = 0; e < 4; e++) w[e] = w[e] * sigmoidf(gv[e]);
+        }
+        store_out4(p.out, (size_t)t * p.nh * HD + (size_t)h * HD + 4 * lane, w, p.out_type, p.f16_lim, flag);
+    }
 }
 
-template <typename F, int... I>
-__device__ __forceinline__ void sfor_impl(F &&f, std::integer_sequence<int, I...>) {
-    (f(std::integral_constant<int, I>{}), ...);
-}
-template <int N, typename F>
-__device__ __forceinline__ void sfor(F &&f) {
-    sfor_impl(f, std::make_integer_sequence<int, N>{});
-}
-
-// Work items are (16-row sub-block, kv head, head chunk): the kv group's G = nh / nkv q heads
-// split into n_chunks chunks of at most W <= 8 heads, X waves per head (a chunk's spare waves
-// fill tiles and take barriers but compute nothing). With X = 2 the two waves of a head split
-// its 256 dims: wave (slot s, half x), wave id s + W x, holds Q steps c = 4j + e of the chunks
-// j in {4x .. 4x + 3, 8 + 4x .. 8 + 4x + 3} (so a rotary pair (i, i + 32) stays in one wave)
-// and O for dims 128x .. 128x + 127; the halves' partial scores meet through LDS and each wave
-// adds its partner's to its own (the same sum in both, bitwise), then both run the softmax. Six
-// q heads then fill twelve waves, three per SIMD, where six waves left two SIMDs with one. Items run in the plan's longest-first
-// block order, each block's last 16 rows (its longest causal rows) first. With G workgroups,
-// workgroup b takes items b, then 2G - 1 - b, ... (snake order, so long and short items mix;
-// one item each when G is the item count); while an item's epilogue runs, the next item's
-// first K / V tile loads into the idle LDS buffers.
-template <int W, int X>
-__global__ __launch_bounds__(64 * W * X) void attn_text_f32_kernel(Params p) {
-    static_assert(X == 1 || X == 2, "one or two waves per head");
-    constexpr int NW = W * X;           // waves
-    constexpr int QN = 64 / X;          // Q steps (and B registers) per wave
-    __shared__ __attribute__((aligned(16))) float smem[4 * TILE];   // K0 | K1 | V0 | V1
-    // partial scores of the two halves: slot (wave, lane) holds its two 16-key subtiles
-    __shared__ __attribute__((aligned(16))) f32x4 xch[X > 1 ? NW * 64 * 2 : 1];
+// Work items are (block, R x 16 rows of it, k heads of a kv group, kv head), the plan's longest-first
+// blocks outermost, each block's last rows first, kv heads innermost (an XCD then streams the K / V
+// of few of them), one workgroup each. An item of few rows runs more heads (f32_heads), and the
+// items of the heads it took are empty.
+//
+// Per 32-key tile: barrier; S(t) while V(t) is split into LDS; barrier; softmax; P.V(t) while
+// K(t + 1) is split. The operand staged beside a product is the one the product does not read, so
+// one buffer each is enough; its loads go out a phase ahead into registers that K and V share.
+__global__ __launch_bounds__(64 * NW) void attn_text_f32_kernel(Params p) {
+    constexpr int PL = BK * HD * 2, KV = 3 * PL;           // bytes of one bf16 plane; the V^T planes
+    __shared__ __attribute__((aligned(16))) uint8_t smem[2 * KV];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int slot = X == 1 ? wave : wave % W, half = X == 1 ? 0 : wave / W;   // head slot in the chunk, dim half
     const int r16 = lane & 15, g = lane >> 4;
     const int group = p.nh / p.nkv;
-    const int n_items = p.n_blk * SUB * p.nkv * p.n_chunks;
-    const int G = gridDim.x;
-    struct Item {
-        int nq, q_row0, q_pos0, k_row0, k_len, n_tiles, kh, h;
-        bool live;   // this wave has a head in the item's chunk
-        int32_t *flag;
-    };
-    // the k-th item of this workgroup, or nq = 0 past the end
-    auto item_at = [&](int k, Item &it) {
-        const int j = k * G + ((k & 1) ? G - 1 - (int)blockIdx.x : (int)blockIdx.x);
-        it.nq = 0;
-        if (j >= n_items) return false;
-        const int chunk = j % p.n_chunks, rest = j / p.n_chunks;
-        it.kh = rest % p.nkv;
-        const int sb = rest / p.nkv, bi = sb / SUB, sub = SUB - 1 - sb % SUB;
-        const int32_t *blk = p.blocks + 8 * bi;
-        it.nq = min(BQ, blk[1] - BQ * sub);
-        if (it.nq <= 0) { it.nq = 0; return true; }      // a sub-block past the block's rows
-        it.q_row0 = blk[0] + BQ * sub;
-        it.q_pos0 = blk[2] + BQ * sub;
-        it.k_row0 = blk[3];
-        it.k_len = p.causal ? min(blk[4], it.q_pos0 + it.nq) : blk[4];
-        it.n_tiles = (it.k_len + BK - 1) / BK;
-        it.flag = p.ovf ? p.ovf + blk[5] : nullptr;
-        const int hw = chunk * W + slot;
-        it.live = hw < group;
-        it.h = it.kh * group + (it.live ? hw : 0);
-        return true;
-    };
-    // next item with rows, from ordinal k on; false past the end
-    auto advance = [&](int &k, Item &it) {
-        while (item_at(k, it)) {
-            if (it.nq > 0) return true;
-            k++;
-        }
-        return false;
-    };
+    const Shape shape = f32_shape(p.slots, group);
+    const int span = 16 * shape.R, n_sub = BLK / span, n_ch = group / shape.k;
+    const split32::Weights wt;
+    // per-lane LDS byte addresses of the operand reads (plane h)
+    const unsigned lds0 = split32::lds_offset(smem);
+    unsigned ka[4];   // 32-dim step c, c % 4: K row of S^T A row r16 in subtile 0 (+ 256 c / 4; subtile 1: + 4 rows)
+#pragma unroll
+    for (int c = 0; c < 4; c++) ka[c] = lds0 + (8 * (r16 >> 2) + (r16 & 3)) * (2 * HD) + (((4 * c + g) ^ r16) * 16);
+    unsigned va[2];   // V^T row of O^T A row r16 in dim tiles 0 and 1 (tiles 2u + w: + 32 u rows)
+#pragma unroll
+    for (int w = 0; w < 2; w++)
+        va[w] = lds0 + KV + (8 * (r16 >> 2) + 4 * w + (r16 & 3)) * (2 * BK) + ((g ^ (-(r16 >> 2) & 3) ^ w) * 16);
 
-    // ---- tile fills: one 1 KB DMA group per key row; wave w fills rows w, w + NW, ...
-    auto fill = [&](const Item &it, int kb, float *Ks, float *Vs) {
-        const float *kbase = p.k_plane + ((size_t)it.kh * p.kvT + it.k_row0) * HD;
-        const float *vbase = p.v_plane + ((size_t)it.kh * p.kvT + it.k_row0) * HD;
-        for (int r = wave; r < BK; r += NW) {
-            const size_t off = (size_t)(kb + r) * HD + 4 * lane;
-            __builtin_amdgcn_global_load_lds((const void *)(kbase + off), (lds_void *)(Ks + r * ROW), 16, 0, 0);
-            __builtin_amdgcn_global_load_lds((const void *)(vbase + off), (lds_void *)(Vs + r * ROW), 16, 0, 0);
-        }
-    };
-    // Rows past the keys (not written by this pass, possibly not finite) -> 0 in V, so that the
-    // zero probabilities of masked keys give exact zero products.
-    auto clear_tail = [&](const Item &it, int kb, float *Vs) {
-        if (kb + BK <= it.k_len) return;                  // workgroup-uniform
-        for (int r = wave; r < BK; r += NW)
-            if (kb + r >= it.k_len) *(f32x4 *)(Vs + r * ROW + 4 * lane) = f32x4{0.f, 0.f, 0.f, 0.f};
-    };
+    {
+        const int item = blockIdx.x;
+        const int kh = item % p.nkv, ic = item / p.nkv % n_ch, ib = item / p.nkv / n_ch;
+        const int32_t *blk = p.blocks + 8 * (ib / n_sub);
+        const int r0 = span * (n_sub - 1 - ib % n_sub), rows = min(span, blk[1] - r0);
+        if (rows <= 0) return;
+        const int kk = f32_heads(p.slots, rows, group), wph = (rows + 15) / 16;
+        if (ic * kk >= group) return;
+        const int slot = wave / wph;
+        const bool live = slot < kk;
+        const int h = kh * group + ic * kk + (live ? slot : 0);
+        const int q_row0 = blk[0] + r0 + (live ? 16 * (wave - slot * wph) : 0), q_pos0 = blk[2] + q_row0 - blk[0];
+        const int nq = live ? min(16, blk[0] + r0 + rows - q_row0) : 0;
+        const int k_row0 = blk[3], k_len = p.causal ? min(blk[4], blk[2] + r0 + rows) : blk[4];
+        int32_t *const flag = p.ovf ? p.ovf + blk[5] : nullptr;
+        const int n_tiles = (k_len + BK - 1) / BK;
+        // keys this wave's rows see, and the tiles it runs
+        const int my_len = live ? (p.causal ? min(k_len, q_pos0 + nq) : k_len) : 0;
+        const bool q_valid = r16 < nq;
+        const float *const kbase = p.k_plane + ((size_t)kh * p.kvT + k_row0) * HD;
+        const float *const vbase = p.v_plane + ((size_t)kh * p.kvT + k_row0) * HD;
+        float amax = 0.f;
 
-    const unsigned lds0 = (unsigned)(uintptr_t)(const __attribute__((address_space(3))) float *)smem;
-    // K: row 4(r16 % 4) + r16 / 4 of subtile 0, chunk 16g (+ 4 half); V: row g, chunk r16
-    // (+ 32 half) (buffer 0)
-    const unsigned ka = lds0 + (unsigned)(4 * (r16 & 3) + (r16 >> 2)) * ROW * 4u + 256u * g + 64u * half;
-    const unsigned va = lds0 + 2u * TB + (unsigned)g * ROW * 4u + 16u * r16 + 512u * half;
-    // the K chunk (of 16 per 64 dims) of this wave's chunk step q4
-    auto kchunk = [](int q4) { return X == 1 ? q4 : (q4 < 4 ? q4 : q4 + 4); };
+        // ---- tile staging, two pieces a thread. Piece e: K dims 8 c .. 8 c + 7
+        // of one key, V keys 8 kg .. 8 kg + 7 of one dim; each load is a uniform base plus a
+        // 32-bit lane offset. Keys past the item's range become zeros: their zero probabilities
+        // then give zero products, and what lies there cannot flag the item.
+        float raw[2][8];
+        const unsigned ko = 32u * tid, vo = (tid >> 8) * (8u * HD * 4u) + (tid & 255) * 4u;
+        auto load_k = [&](int kb) {
+#pragma unroll
+            for (int e = 0; e < 2; e++) {
+                const char *s = (const char *)(kbase + (size_t)(kb + 2 * NW * e) * HD);
+                const f32x4 a = *(const f32x4 *)(s + ko), b = *(const f32x4 *)(s + ko + 16);
+#pragma unroll
+                for (int j = 0; j < 4; j++) { raw[e][j] = a[j]; raw[e][4 + j] = b[j]; }
+            }
+        };
+        auto load_v = [&](int kb) {
+#pragma unroll
+            for (int e = 0; e < 2; e++)
+#pragma unroll
+                for (int j = 0; j < 8; j++) {
+                    const char *s = (const char *)(vbase + (size_t)(kb + 2 * NW * e + j) * HD);
+                    raw[e][j] = *(const float *)(s + vo);
+                }
+        };
+        // K chunk c of key 8a + 4t + b sits at position c ^ (4a + b), V^T chunk kg of dim d at
+        // kg ^ (-(d / 8) % 4) ^ ((d / 4) % 2): the lanes one step of a read or write serves hit
+        // distinct 16-byte slots.
+        const unsigned dk = (tid >> 5) * (2 * HD) + (((tid & 31) ^ (((tid >> 5) & 3) | (((tid >> 5) >> 3) << 2))) * 16);
+        const unsigned dv = KV + (tid & 255) * (2 * BK) + (((tid >> 8) ^ (-((tid & 255) >> 3) & 3) ^ ((tid >> 2) & 1)) * 16);
+        // piece e lies 2 NW e keys on, or NW e / 4 chunks: no carry into the bits of the thread's own
+        auto dst_k = [&](int e) { return smem + (dk ^ (unsigned)(((2 * NW * e) >> 3 << 2) * 16)) + 2 * NW * e * (2 * HD); };
+        auto dst_v = [&](int e) { return smem + (dv ^ (unsigned)((NW / 4 * e) * 16)); };
+        auto put = [&](auto DST) {
+#pragma unroll
+            for (int e = 0; e < 2; e++) {
+                amax = split32::split_amax(amax, raw[e]);
+                const split32::Parts x = split32::split8(raw[e], wt);
+                uint8_t *const dst = DST(e);
+                *(bf16x8 *)dst = x.h;
+                *(bf16x8 *)(dst + PL) = x.m;
+                *(bf16x8 *)(dst + 2 * PL) = x.l;
+            }
+        };
+        auto put_k = [&](int kb) {
+            if (kb + BK > k_len) {
+#pragma unroll
+                for (int e = 0; e < 2; e++)
+#pragma unroll
+                    for (int j = 0; j < 8; j++) raw[e][j] = kb + (tid >> 5) + 2 * NW * e < k_len ? raw[e][j] : 0.f;
+            }
+            put(dst_k);
+        };
+        auto put_v = [&](int kb) {
+            if (kb + BK > k_len) {
+#pragma unroll
+                for (int e = 0; e < 2; e++)
+#pragma unroll
+                    for (int j = 0; j < 8; j++) raw[e][j] = kb + 8 * (tid >> 8) + 2 * NW * e + j < k_len ? raw[e][j] : 0.f;
+            }
+            put(dst_v);
+        };
 
-    int k = 0;
-    Item cur;
-    if (!advance(k, cur)) return;
-    if (cur.n_tiles > 0) fill(cur, 0, smem, smem + 2 * TILE);
-    for (;;) {
-        const bool q_valid = r16 < cur.nq;
-        const int qpos = cur.q_pos0 + r16;
-        const int t = cur.q_row0 + (q_valid ? r16 : 0);
-        const int h = cur.h;
-        const int k_len = cur.k_len, n_tiles = cur.n_tiles;
-
-        // ---- Q prologue: lane holds Q[row r16][64 g + c(q)] for the wave's QN steps q, with
-        // c(q) = 4 kchunk(q / 4) + q % 4 + 16 half: normalised (the sum of squares over the
-        // whole row) and rotated, FP32. Rotary pair i < 32 / X of the wave is (qv[i], qv[i + NP]),
-        // dims 16 half + i and 32 + 16 half + i (lanes g = 0).
-        constexpr int NP = 32 / X;
-        constexpr int RX = X == 1 ? RUN : 2;   // K chunks per run (two per run in the split layout, for registers)
-        float qv[QN];
+        load_k(0);
+        // ---- Q prologue: lane holds Q[row r16][32 c + 8 g + j], the B operand of step c:
+        // normalised, rotated (pair i < 32 is chunks 0 and 1 of the lane) and scaled by
+        // scale * log2 e (the scores then are exponents of 2), in FP32, then split
+        bf16x8 qh[8], qm[8], ql[8];
         {
-            float ss = 0.f;
-            {
-                // the wave's own QN elements of the lane's 64 (the chunks kchunk(q4) + 4 half)
-                const float *qs = p.qkv + (size_t)t * p.row + (size_t)h * 2 * HD + 64 * g + 16 * half;
+            // every load goes out before the first is used
+            const int t = q_row0 + (q_valid ? r16 : 0);
+            const float *qs = p.qkv + (size_t)t * p.row + (size_t)h * 2 * HD + 8 * g;
+            float x[8][8];
+            f32x4 w[8][2], cs[4];
 #pragma unroll
-                for (int q4 = 0; q4 < QN / 4; q4++) {
-                    const f32x4 v = *(const f32x4 *)(qs + 4 * kchunk(q4));
-                    qv[4 * q4] = v.x; qv[4 * q4 + 1] = v.y; qv[4 * q4 + 2] = v.z; qv[4 * q4 + 3] = v.w;
-                }
-                if (p.q_norm) {
+            for (int c = 0; c < 8; c++) {
+                const f32x4 a = *(const f32x4 *)(qs + 32 * c), b = *(const f32x4 *)(qs + 32 * c + 4);
 #pragma unroll
-                    for (int q = 0; q < QN; q++) ss += qv[q] * qv[q];
+                for (int j = 0; j < 4; j++) { x[c][j] = a[j]; x[c][4 + j] = b[j]; }
+            }
+            // without norms or a table, the pass's own rows stand in (loaded, not used)
+            const float *ws = p.q_norm ? p.q_norm + 8 * g : qs, *ts = p.rope_cs ? p.rope_cs + (size_t)t * 64 + 16 * g : qs;
+#pragma unroll
+            for (int c = 0; c < 8; c++)
+#pragma unroll
+                for (int i = 0; i < 2; i++) w[c][i] = *(const f32x4 *)(ws + 32 * c + 4 * i);
+#pragma unroll
+            for (int q = 0; q < 4; q++) cs[q] = *(const f32x4 *)(ts + 4 * q);   // cos, sin of pairs 8g + 2q, 8g + 2q + 1
+            if (p.n_rot && !p.rope_cs) {
+                // no table: the wave evaluates its rows' angles into LDS (the V^T region is free)
+                float2 *tab = (float2 *)(smem + KV) + 16 * 32 * wave;
+                for (int i = lane; i < 16 * 32; i += 64) {
+                    const int row = i >> 5;
+                    float c, s;
+                    rope_cs_f32(p.pos3, p.inv_freq, q_row0 + (row < nq ? row : 0), i & 31, &c, &s);
+                    tab[i] = make_float2(c, s);
                 }
+#pragma unroll
+                for (int q = 0; q < 4; q++) cs[q] = *(const f32x4 *)(tab + 32 * r16 + 8 * g + 2 * q);
             }
             if (p.q_norm) {
+                float ss = 0.f;
+#pragma unroll
+                for (int c = 0; c < 8; c++)
+#pragma unroll
+                    for (int j = 0; j < 8; j++) ss += x[c][j] * x[c][j];
                 ss += __shfl_xor(ss, 16);
                 ss += __shfl_xor(ss, 32);
-                if constexpr (X > 1) {
-                    // the two halves' sums of squares meet through LDS: the row's sum is the same
-                    // in both (own + partner's); the nop covers a VALU result read by the LDS write
-                    float *xs = (float *)xch;
-                    asm volatile("s_nop 1\n\tds_write_b32 %0, %1\n\ts_waitcnt lgkmcnt(0)\n\ts_barrier"
-                                 : : "v"((unsigned)(uintptr_t)(const __attribute__((address_space(3))) float *)(xs + wave * 64 + lane)), "v"(ss) : "memory");
-                    float o;
-                    asm volatile("ds_read_b32 %0, %1\n\ts_waitcnt lgkmcnt(0)"
-                                 : "=v"(o) : "v"((unsigned)(uintptr_t)(const __attribute__((address_space(3))) float *)(xs + (half ? wave - W : wave + W) * 64 + lane)) : "memory");
-                    ss = half ? o + ss : ss + o;
-                }
                 const float inv = 1.0f / sqrtf(ss / (float)HD + p.eps);
-                const float *w = p.q_norm + 64 * g + 16 * half;
 #pragma unroll
-                for (int q4 = 0; q4 < QN / 4; q4++) {
-                    const f32x4 wv = *(const f32x4 *)(w + 4 * kchunk(q4));
+                for (int c = 0; c < 8; c++)
 #pragma unroll
-                    for (int e = 0; e < 4; e++) qv[4 * q4 + e] = qv[4 * q4 + e] * inv * wv[e];
+                    for (int j = 0; j < 8; j++) x[c][j] = x[c][j] * inv * w[c][j >> 2][j & 3];
+            }
+            if (p.n_rot) {
+#pragma unroll
+                for (int j = 0; j < 8; j++) {
+                    const float c = cs[j >> 1][2 * (j & 1)], s = cs[j >> 1][2 * (j & 1) + 1];
+                    const float x0 = x[0][j], x1 = x[1][j];
+                    x[0][j] = x0 * c - x1 * s;
+                    x[1][j] = x1 * c + x0 * s;
                 }
             }
-            if (p.n_rot && g == 0) {
-#pragma unroll
-                for (int i = 0; i < NP; i++) {
-                    const int i0 = NP * half + i;
-                    float c, s;
-                    if (p.rope_cs) {
-                        const float2 cs = *(const float2 *)(p.rope_cs + ((size_t)t * 32 + i0) * 2);
-                        c = cs.x; s = cs.y;
-                    } else {
-                        rope_cs_f32(p.pos3, p.inv_freq, t, i0, &c, &s);
-                    }
-                    const float x0 = qv[i], x1 = qv[i + NP];
-                    qv[i] = x0 * c - x1 * s;
-                    qv[i + NP] = x1 * c + x0 * s;
-                }
-            }
-            // the scores in the exp2 domain: scale * log2 e folded into Q
             const float sl2 = p.scale * 1.4426950408889634f;
 #pragma unroll
-            for (int q = 0; q < QN; q++) qv[q] *= sl2;
+            for (int c = 0; c < 8; c++) {
+#pragma unroll
+                for (int j = 0; j < 8; j++) x[c][j] *= sl2;
+                amax = split32::split_amax(amax, x[c]);
+                const split32::Parts s = split32::split8(x[c], wt);
+                qh[c] = s.h; qm[c] = s.m; ql[c] = s.l;
+            }
         }
-        __builtin_amdgcn_s_waitcnt(0);
-        if (n_tiles > 0) clear_tail(cur, 0, smem + 2 * TILE);
-        __syncthreads();
+        // the previous item's last reads are behind its closing barrier
+        put_k(0);
+        load_v(0);
 
-        constexpr int NO = 16 / X;   // dim tiles 4j + e of this wave (j < 4 / X)
-        f32x4 o[NO];
+        f32x4 o[16];
 #pragma unroll
-        for (int n = 0; n < NO; n++) o[n] = f32x4{0.f, 0.f, 0.f, 0.f};
-        float m_run = -INFINITY, l_run = 0.f;
-
-        auto tile = [&](const int ti, auto BUF) {
-            constexpr int buf = decltype(BUF)::value;
-            const int kb = ti * BK;
-            if (ti + 1 < n_tiles) fill(cur, kb + BK, smem + (buf ^ 1) * TILE, smem + 2 * TILE + (buf ^ 1) * TILE);
-            // S^T: two 16-key subtiles, QN four-dim steps each, their products interleaved (two
-            // independent accumulator chains); K read in runs of RX chunks per subtile
-            f32x4 s[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
-            if (cur.live) {   // wave-uniform: a spare wave of the last head chunk only fills
-                sfor<16 / X / RX>([&](auto H) {
-                    constexpr int hh = decltype(H)::value;
-                    f32x4 a[2][RX];
-                    sfor<RX>([&](auto J) {
-                        constexpr int j = decltype(J)::value;
-                        constexpr int ch = X == 1 ? RX * hh + j : (RX * hh + j < 4 ? RX * hh + j : RX * hh + j + 4);
-                        a[0][j] = lds_read_f4<buf * TB + ch * 16>(ka);
-                        a[1][j] = lds_read_f4<buf * TB + 16 * ROW * 4 + ch * 16>(ka);
-                    });
-                    sfor<RX>([&](auto J) {
-                        constexpr int j = decltype(J)::value;
-                        lds_wait_f4<2 * (RX - 1 - j) + 1>(a[0][j]);
-                        lds_wait_f4<2 * (RX - 1 - j)>(a[1][j]);
+        for (int n = 0; n < 16; n++) o[n] = f32x4{0.f, 0.f, 0.f, 0.f};
+        // the running maximum starts at the lowest finite value: a row that has seen no key yet
+        // then needs no case of its own
+        float m_run = -3.4028235e38f, l_run = 0.f;
+        // every LDS access of the phase is done; the loads in flight stay so
+        auto phase_barrier = [&]() {
+            __builtin_amdgcn_sched_barrier(0);
+            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        for (int t = 0; t < n_tiles; t++) {
+            const int kb = t * BK;
+            const bool mine = kb < my_len;   // wave-uniform
+            phase_barrier();                 // K(t) is in place; V(t - 1) has been read
+            // S^T: two 16-key subtiles, eight 32-dim steps; the hh terms in one accumulator, the
+            // smaller ones in another
+            split32::Ring ring;
+            f32x4 s[2], sx[2];
 #pragma unroll
-                        for (int e = 0; e < 4; e++) {
-                            s[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[0][j][e], qv[4 * (RX * hh + j) + e], s[0], 0, 0, 0);
-                            s[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[1][j][e], qv[4 * (RX * hh + j) + e], s[1], 0, 0, 0);
-                        }
-                    });
+            for (int u = 0; u < 2; u++) s[u] = sx[u] = f32x4{0.f, 0.f, 0.f, 0.f};
+            if (mine) split32::ring_start<PL, 0, 4 * 2 * HD>(ring, ka[0], ka[0]);
+            const bool more = t + 1 < n_tiles;
+            put_v(kb);
+            if (more) load_k(kb + BK);
+            if (mine) {
+                split32::sfor<8>([&](auto I) {
+                    constexpr int i = decltype(I)::value, n = i + 1, o8 = 256 * (n / 4);
+                    split32::ring_step<PL, (n < 8), o8, o8 + 4 * 2 * HD>(ring, ka[n % 4], ka[n % 4], s[0], s[1], sx[0], sx[1], qh[i], qm[i], ql[i]);
                 });
             }
-            if constexpr (X > 1) {
-                // the halves' partial scores meet: write this wave's, barrier, add the partner's
-                const unsigned xa = (unsigned)(uintptr_t)(const __attribute__((address_space(3))) f32x4 *)(xch + 2 * (wave * 64 + lane));
-                // (the wait states cover an MFMA result read by the LDS write: the compiler does
-                // not see inside the statement)
-                asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 4\n\tds_write_b128 %0, %1\n\tds_write_b128 %0, %2 offset:16" : : "v"(xa), "v"(s[0]), "v"(s[1]) : "memory");
-                asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-                const unsigned pa = xa + (half ? -1 : 1) * (unsigned)(W * 64 * 32);
-                f32x4 t0, t1;
-                asm volatile("ds_read_b128 %0, %2\n\tds_read_b128 %1, %2 offset:16\n\ts_waitcnt lgkmcnt(0)" : "=&v"(t0), "=&v"(t1) : "v"(pa) : "memory");
-                s[0] += t0;
-                s[1] += t1;
+            phase_barrier();                 // V(t) is in place; K(t) has been read
+            if (mine) split32::ring_start<PL, 0, 0>(ring, va[0], va[1]);
+            if (more) {
+                put_k(kb + BK);
+                load_v(kb + BK);
             }
-            if (cur.live) {
-                // V chunk j of step st = (u, v): key 16u + 4v + g, chunk 16j + r16 of its row
-                auto vread = [&](auto ST, auto J) {
-                    constexpr int st = decltype(ST)::value, u = st >> 2, v = st & 3, j = decltype(J)::value;
-                    return lds_read_f4<buf * TB + (16 * u + 4 * v) * ROW * 4 + 256 * j>(va);
-                };
-                constexpr int NJ = 4 / X;   // V chunks per step of this wave
-                f32x4 vb[NJ];   // step 0's chunks load while the softmax runs
-                sfor<NJ>([&](auto J) { vb[decltype(J)::value] = vread(std::integral_constant<int, 0>{}, J); });
-                // Online softmax. s[u][v] is the score of key kb + 16u + 4v + g for query row r16.
-                float x[2][4], mx = -INFINITY;
+            if (mine) {
+                // x[4 u + v] is the score (exponent of 2) of key kb + 8g + 4u + v for row r16
+                float x[8], mx, rs = 0.f;
 #pragma unroll
-                for (int u = 0; u < 2; u++)
+                for (int j = 0; j < 8; j++) x[j] = s[j >> 2][j & 3] + sx[j >> 2][j & 3];
+                if (kb + BK > k_len || (p.causal && kb + BK - 1 > q_pos0)) {
+                    const int lim = (p.causal ? min(k_len - 1, q_pos0 + r16) : k_len - 1) - kb - 8 * g;
 #pragma unroll
-                    for (int v = 0; v < 4; v++) {
-                        const int key = kb + 16 * u + 4 * v + g;
-                        const bool ok = q_valid && key < k_len && (!p.causal || key <= qpos);
-                        x[u][v] = ok ? s[u][v] : -INFINITY;
-                        mx = fmaxf(mx, x[u][v]);
-                    }
+                    for (int j = 0; j < 8; j++) x[j] = j <= lim ? x[j] : -INFINITY;
+                }
+                mx = x[0];
+#pragma unroll
+                for (int j = 1; j < 8; j++) mx = fmaxf(mx, x[j]);
                 const float mn = fmaxf(m_run, xrow_max(mx));
-                float pv[2][4];
-                float alpha = 1.f, rs = 0.f;
-                if (mn != -INFINITY) {
-                    alpha = (m_run == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(m_run - mn);
+                const float alpha = __builtin_amdgcn_exp2f(m_run - mn);
 #pragma unroll
-                    for (int u = 0; u < 2; u++)
-#pragma unroll
-                        for (int v = 0; v < 4; v++) {
-                            pv[u][v] = x[u][v] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(x[u][v] - mn);
-                            rs += pv[u][v];
-                        }
-                } else {
-#pragma unroll
-                    for (int u = 0; u < 2; u++)
-#pragma unroll
-                        for (int v = 0; v < 4; v++) pv[u][v] = 0.f;
+                for (int j = 0; j < 8; j++) {
+                    x[j] = __builtin_amdgcn_exp2f(x[j] - mn);   // a masked key's -inf gives 0
+                    rs += x[j];
                 }
                 m_run = mn;
                 l_run = l_run * alpha + rs;
-                const float alpha_o = alpha;
-                // O^T += V^T . P^T: 8 four-key steps (u, v), each 16 dim tiles. The V chunks roll
-                // through four registers: chunk j of the next step is read as soon as the current
-                // step's chunk j has fed its four products, so three reads are always in flight.
+                if (__any(alpha != 1.f)) {   // in place (as plain C++ the other path copies the registers)
 #pragma unroll
-                for (int n = 0; n < NO; n++) o[n] *= alpha_o;
-                sfor<8>([&](auto S) {
-                    constexpr int st = decltype(S)::value, u = st >> 2, v = st & 3;
-                    const float b = pv[u][v];
-                    sfor<NJ>([&](auto J) {
-                        constexpr int j = decltype(J)::value;
-                        if constexpr (st + 1 < 8) lds_wait_f4<NJ - 1>(vb[j]);
-                        else lds_wait_f4<NJ - 1 - j>(vb[j]);
+                    for (int n = 0; n < 16; n++)
 #pragma unroll
-                        for (int e = 0; e < 4; e++)
-                            o[4 * j + e] = __builtin_amdgcn_mfma_f32_16x16x4f32(vb[j][e], b, o[4 * j + e], 0, 0, 0);
-                        if constexpr (st + 1 < 8) vb[j] = vread(std::integral_constant<int, st + 1>{}, J);
-                    });
+                        for (int v = 0; v < 4; v++) {
+                            float d = o[n][v];
+                            asm("v_mul_f32 %0, %1, %0" : "+v"(d) : "v"(alpha));
+                            o[n][v] = d;
+                        }
+                }
+                const split32::Parts pp = split32::split8(x, wt);
+                // O^T += V^T . P^T: pairs of 16-dim tiles, the six terms smallest first
+                split32::sfor<8>([&](auto I) {
+                    constexpr int i = decltype(I)::value, o8 = 32 * (i + 1) * 2 * BK;
+                    split32::ring_step<PL, (i + 1 < 8), o8, o8>(ring, va[0], va[1], o[2 * i], o[2 * i + 1], o[2 * i], o[2 * i + 1], pp.h, pp.m, pp.l);
                 });
             }
-            __builtin_amdgcn_s_waitcnt(0);
-            if (ti + 1 < n_tiles) clear_tail(cur, kb + BK, smem + 2 * TILE + (buf ^ 1) * TILE);
-            __syncthreads();
-        };
-        for (int ti = 0; ti < n_tiles; ti += 2) {
-            tile(ti, std::integral_constant<int, 0>{});
-            if (ti + 1 < n_tiles) tile(ti + 1, std::integral_constant<int, 1>{});
         }
 
-        // ---- the next item's first tile loads into the buffers the key loop has left (every
-        // wave passed its closing barrier) while this item's epilogue runs
-        const Item done = cur;
-        k++;
-        const bool more = advance(k, cur);
-        if (more && cur.n_tiles > 0) fill(cur, 0, smem, smem + 2 * TILE);
-
-        // ---- epilogue: O = O^T / l, times sigmoid(gate). Accumulator n = 4j + e, entry v of lane
-        // (g, r16) is dim 64j + 16g + 4v + e of row r16.
+        // ---- epilogue: O = O^T / l, times sigmoid(gate). Tiles 2u, 2u + 1 of lane (g, r16) are
+        // dims 32 u + 8 g .. + 7 of row r16.
         float l_row = l_run;
         l_row += __shfl_xor(l_row, 16);
         l_row += __shfl_xor(l_row, 32);
-        if (q_valid && done.live) {
+        if (__syncthreads_or(split32::split_bad(amax))) {   // also: the tiles' last reads are done
+            if (live) text_rows_plain(p, q_row0, nq, q_pos0, k_row0, k_len, h, kh, flag);
+        } else if (q_valid) {
             const float il = l_row > 0.f ? 1.0f / l_row : 0.f;
-            const float *grow = p.qkv + (size_t)t * p.row + (size_t)h * 2 * HD + HD;
-            const size_t obase = (size_t)t * p.nh * HD + (size_t)h * HD;
+            const size_t t = (size_t)(q_row0 + r16);
+            const size_t obase = t * p.nh * HD + (size_t)h * HD + 8 * g;
+            if (p.gate) {   // every gate load goes out before the first store
+                const float *grow = p.qkv + t * p.row + (size_t)h * 2 * HD + HD + 8 * g;
+                f32x4 gv[16];
 #pragma unroll
-            for (int v = 0; v < 4; v++)
+                for (int n = 0; n < 16; n++) gv[n] = *(const f32x4 *)(grow + 32 * (n >> 1) + 4 * (n & 1));
 #pragma unroll
-                for (int j = 0; j < 4 / X; j++) {
-                    const int d = 64 * (j + (4 / X) * half) + 16 * g + 4 * v;
-                    f32x4 w;
+                for (int n = 0; n < 16; n++)
 #pragma unroll
-                    for (int e = 0; e < 4; e++) w[e] = o[4 * j + e][v] * il;
-                    if (p.gate) {
-                        const f32x4 gv = *(const f32x4 *)(grow + d);
+                    for (int v = 0; v < 4; v++) o[n][v] = o[n][v] * il * sigmoidf(gv[n][v]);
+            } else {
 #pragma unroll
-                        for (int e = 0; e < 4; e++) w[e] = w[e] * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-gv[e] * 1.4426950408889634f));
-                    }
-                    store_out4(p.out, obase + d, w, p.out_type, p.f16_lim, done.flag);
+                for (int n = 0; n < 16; n++) o[n] *= il;
+            }
+            auto store = [&](const int type) {
+#pragma unroll
+                for (int u = 0; u < 8; u++) {
+                    float w[8];
+#pragma unroll
+                    for (int j = 0; j < 8; j++) w[j] = o[2 * u + (j >> 2)][j & 3];
+                    store_out8(p.out, obase + 32 * u, w, type, p.f16_lim, flag);
                 }
+            };
+            if (p.out_type == CLEF_HIP_OUT_F32) store(CLEF_HIP_OUT_F32);
+            else if (p.out_type == CLEF_HIP_OUT_BF16) store(CLEF_HIP_OUT_BF16);
+            else store(CLEF_HIP_OUT_F16);
         }
-        if (!more) break;
     }
 }
 

@@ -45,23 +45,29 @@ __device__ __forceinline__ float minus_hi(unsigned pair, const Weights &w, float
     return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, pair), __builtin_bit_cast(bf16x2, w.hi), x, false);
 }
 
+// the parts of one pair of elements, as packed words
+__device__ __forceinline__ void split2(float a, float b, const Weights &w, unsigned &h, unsigned &m, unsigned &l) {
+    h = pack_bf16(a, b);
+    const float a1 = minus_lo(h, w, a), b1 = minus_hi(h, w, b);
+    m = pack_bf16(a1, b1);
+    l = pack_bf16(minus_lo(m, w, a1), minus_hi(m, w, b1));
+}
 __device__ __forceinline__ Parts split8(const float (&x)[8], const Weights &w) {
     u32x4 h, m, l;
 #pragma unroll
     for (int i = 0; i < 4; i++) {
-        const float a = x[2 * i], b = x[2 * i + 1];
-        h[i] = pack_bf16(a, b);
-        const float a1 = minus_lo(h[i], w, a), b1 = minus_hi(h[i], w, b);
-        m[i] = pack_bf16(a1, b1);
-        l[i] = pack_bf16(minus_lo(m[i], w, a1), minus_hi(m[i], w, b1));
+        unsigned a, b, c;
+        split2(x[2 * i], x[2 * i + 1], w, a, b, c);
+        h[i] = a; m[i] = b; l[i] = c;
     }
     return {__builtin_bit_cast(bf16x8, h), __builtin_bit_cast(bf16x8, m), __builtin_bit_cast(bf16x8, l)};
 }
 
 // Largest magnitude of a running maximum and eight values (a NaN does not count: its parts are NaN).
+__device__ __forceinline__ void split_amax2(float &amax, float a, float b) { asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(amax) : "v"(a), "v"(b)); }
 __device__ __forceinline__ float split_amax(float amax, const float (&x)[8]) {
 #pragma unroll
-    for (int i = 0; i < 8; i += 2) asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(amax) : "v"(x[i]), "v"(x[i + 1]));
+    for (int i = 0; i < 8; i += 2) split_amax2(amax, x[i], x[i + 1]);
     return amax;
 }
 // whether a value of that magnitude has no finite parts
@@ -76,9 +82,12 @@ __device__ __forceinline__ void sfor(F &&f) {
     sfor_impl(f, std::make_integer_sequence<int, N>{});
 }
 
-// Operand reads run ahead of their products: six ds_read_b128 (the h, m, l parts of two operands) as
-// one asm statement, and a wait that names them before their use.
+__device__ __forceinline__ f32x4 mma(bf16x8 a, bf16x8 b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0); }
+
 __device__ __forceinline__ unsigned lds_offset(const void *p) { return (unsigned)(uintptr_t)(const __attribute__((address_space(3))) void *)p; }
+
+// Operand reads two steps ahead of their products, for kernels with the registers for it: six
+// ds_read_b128 (the h, m, l parts of two operands) as one asm statement, and a wait that names them.
 struct Six {
     bf16x8 h0, m0, l0, h1, m1, l1;
 };
@@ -95,8 +104,6 @@ template <int N>   // until at most N LDS operations are outstanding
 __device__ __forceinline__ void wait6(Six &r) {
     asm volatile("s_waitcnt lgkmcnt(%6)" : "+v"(r.h0), "+v"(r.m0), "+v"(r.l0), "+v"(r.h1), "+v"(r.m1), "+v"(r.l1) : "i"(N) : "memory");
 }
-
-__device__ __forceinline__ f32x4 mma(bf16x8 a, bf16x8 b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0); }
 
 // Two products of split operands against one split operand: hh into big, the five smaller terms
 // into small (the caller may pass one accumulator for both: the small terms then come first).
@@ -121,6 +128,56 @@ __device__ __forceinline__ void mma6_term(f32x4 &c0, f32x4 &c1, const Six &a, bf
     const bf16x8 b = B[J] == 0 ? bh : B[J] == 1 ? bm : bl;
     c0 = mma(A[J] == 0 ? a.h0 : A[J] == 1 ? a.m0 : a.l0, b, c0);
     c1 = mma(A[J] == 0 ? a.h1 : A[J] == 1 ? a.m1 : a.l1, b, c1);
+}
+
+// Products of a pair of 16-row A operands (two 16-key subtiles of K, two 16-dim tiles of V^T) with
+// one B operand: six ds_read_b128 and twelve products a step, as a stream whose reads roll one step
+// ahead through the same 24 registers: a part's two registers take the next step's read as soon as their
+// last product has issued. Reads, waits and products come in the order l, m, h, so that at each wait the four
+// newest reads may stay in flight.
+template <int OA, int OB>
+__device__ __forceinline__ void read_pair(bf16x8 (&r)[2], unsigned a, unsigned b) {
+    static_assert(OA < 65536 && OB < 65536, "16-bit offsets");
+    asm volatile("ds_read_b128 %0, %2 offset:%4\n\tds_read_b128 %1, %3 offset:%5"
+                 : "=&v"(r[0]), "=&v"(r[1]) : "v"(a), "v"(b), "i"(OA), "i"(OB) : "memory");
+}
+template <int N>   // until at most N LDS operations are outstanding
+__device__ __forceinline__ void wait_pair(bf16x8 (&r)[2]) {
+    asm volatile("s_waitcnt lgkmcnt(%2)" : "+v"(r[0]), "+v"(r[1]) : "i"(N) : "memory");
+}
+struct Ring {
+    bf16x8 l[2], m[2], h[2];
+};
+// AT: OA, OB (byte offsets of the two operands' h parts) and the addresses they add to; the m and l
+// parts lie PL and 2 PL behind.
+template <int PL, int OA, int OB>
+__device__ __forceinline__ void ring_start(Ring &r, unsigned a, unsigned b) {
+    read_pair<OA + 2 * PL, OB + 2 * PL>(r.l, a, b);
+    read_pair<OA + PL, OB + PL>(r.m, a, b);
+    read_pair<OA, OB>(r.h, a, b);
+}
+// One step: the products of the operands in the ring with (bh, bm, bl), hh into big and the smaller terms into
+// small (which may be the same accumulators), and the reads of the next step's operands
+// (MORE) at OA, OB.
+template <int PL, bool MORE, int OA, int OB>
+__device__ __forceinline__ void ring_step(Ring &r, unsigned a, unsigned b, f32x4 &big0, f32x4 &big1, f32x4 &small0, f32x4 &small1,
+                                          bf16x8 bh, bf16x8 bm, bf16x8 bl) {
+    auto pair = [&](const bf16x8 (&x)[2], bf16x8 y, f32x4 &c0, f32x4 &c1) {
+        c0 = mma(x[0], y, c0);
+        c1 = mma(x[1], y, c1);
+    };
+    wait_pair<4>(r.l);
+    pair(r.l, bh, small0, small1);
+    if constexpr (MORE) read_pair<OA + 2 * PL, OB + 2 * PL>(r.l, a, b);
+    wait_pair<(MORE ? 4 : 2)>(r.m);
+    pair(r.m, bm, small0, small1);
+    pair(r.m, bh, small0, small1);
+    if constexpr (MORE) read_pair<OA + PL, OB + PL>(r.m, a, b);
+    wait_pair<(MORE ? 4 : 0)>(r.h);
+    pair(r.h, bl, small0, small1);
+    pair(r.h, bm, small0, small1);
+    pair(r.h, bh, big0, big1);
+    if constexpr (MORE) read_pair<OA, OB>(r.h, a, b);
 }
 
 }  // namespace split32

@@ -145,9 +145,10 @@ typedef struct {
                                  CLEF_HIP_QKV_F32 (1): the FP32 path (clef_metal.m:1330-1413,
                                  attn_prep + attention_prefetch_64 and kin): f32 rows, f32 K and V
                                  planes, FP32 products and softmax, for the per-record rerun after
-                                 an overflow (clef.c:526-550) and CLEF_ATTN_TU=0. In FP32 mode any
-                                 nh / nkv works (groups above 8 heads run as several head
-                                 chunks), sched and trace are ignored, and only the output (f16
+                                 an overflow (clef.c:526-550) and CLEF_ATTN_TU=0 (the products run
+                                 as six bf16 products of operands split exactly in three, at the
+                                 error of FP32 ones or below). In FP32 mode any nh / nkv works,
+                                 sched and trace are ignored, and only the output (f16
                                  out_type) can flag. Other values are rejected */
     const int32_t *tok_kv;    /* [T] device int32: the plan's pass row -> plane row map (the inverse
                                  of kv_tok); the bf16 K/V prologue runs over pass rows with it */

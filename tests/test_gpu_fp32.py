@@ -191,3 +191,72 @@ def test_fp32_random_pass(seed):
     w = _fp32(w)
     out, _ = _run(w)
     _check_fp32(out.cpu().numpy(), w, what=f"random {seed}")
+
+
+@pytest.mark.parametrize("which", ["v_inf", "v_big", "v_small", "q_big", "k_minus"])
+def test_fp32_values_without_bf16_parts(which):
+    """Infinities and magnitudes above bf16's overflow threshold (3.39e38) have no bf16 parts: items
+    that hold one run in plain FP32, against float64 (infinite and NaN outputs included); records
+    beside them stay bit for bit what they are alone. Values of 1e-28 keep their relative precision."""
+    _say(f"[fp32] values {which}")
+    lengths, nh, nkv, hd = [40, 70, 21], 8, 2, 256
+    plain = which in ("q_big", "k_minus")
+    w = workloads.text_inputs(lengths, nh, nkv, n_rot=0 if plain else 64, seed=9, norm=not plain, outlier_frac=0)
+    w = _fp32(dict(w, gate=True, theta=1e7))
+    q = w["qkv"].clone()
+    kcol, vcol, row = 2 * nh * hd, (2 * nh + nkv) * hd, 40 + 33
+    if which == "v_inf":
+        q[row, vcol + 5], q[row + 20, vcol + hd + 9] = float("inf"), float("-inf")
+    elif which == "v_big":
+        q[row, vcol + 5] = 3.395e38
+    elif which == "v_small":
+        q[:, vcol:] *= 1e-28
+    elif which == "q_big":      # head 1 (kv head 0), against keys near 0 in that dim: finite scores
+        q[row, 2 * hd + 3] = 3.395e38
+        q[:, kcol + 3] = 1e-38
+    else:                       # scores of minus infinity for one key: no weight
+        for h in range(nh // nkv):
+            q[:, 2 * h * hd + 7] = q[:, 2 * h * hd + 7].abs() + 0.1
+        q[row, kcol + 7] = float("-inf")
+    w = dict(w, qkv=q)
+    got = _run(w)[0].cpu().numpy()
+    with np.errstate(all="ignore"):
+        want = oracle_text(w)
+    fine = np.isfinite(want)
+    assert np.array_equal(got[~fine], want[~fine].astype(np.float32), equal_nan=True)
+    unit = 1e-28 if which == "v_small" else 1.0
+    assert (np.abs(got[fine] - want[fine]) / np.maximum(np.abs(want[fine]), unit)).max() < 2e-5
+    cu = w["cu_seqlens"]
+    for r in (0, 2):
+        a, b = int(cu[r]), int(cu[r + 1])
+        alone, _ = _run(dict(w, qkv=q[a:b].clone(), pos3=w["pos3"][a:b].clone(), cu_seqlens=np.array([0, b - a], np.int32)))
+        assert np.array_equal(alone.cpu().numpy().view(np.uint32), got[a:b].view(np.uint32))
+
+
+@pytest.mark.parametrize("nh,nkv", [(24, 4), (15, 3), (16, 2)])
+def test_fp32_item_sizes_agree_bitwise(nh, nkv):
+    """A record gives the same bits in a pass large enough for eight-wave items as in a small pass, whose
+    items hold rows in four waves (and packed with short records, whose items take more heads)."""
+    _say(f"[fp32] item sizes {nh}/{nkv}")
+    lengths = [300, 5, 17, 40, 81, 97, 128] + [257] * 30
+    w = _fp32(dict(workloads.text_inputs(lengths, nh, nkv, seed=2), gate=True, theta=1e7))
+    packed, _ = _run(w)
+    cu = w["cu_seqlens"]
+    for r in range(8):
+        a, b = int(cu[r]), int(cu[r + 1])
+        alone, _ = _run(dict(w, qkv=w["qkv"][a:b].clone(), pos3=w["pos3"][a:b].clone(), cu_seqlens=np.array([0, b - a], np.int32)))
+        assert torch.equal(alone.view(torch.int32), packed[a:b].view(torch.int32)), f"record {r}"
+
+
+def test_fp32_without_rope_table():
+    """The core evaluates the angles itself when no cos / sin table is given: the same bits."""
+    _say("[fp32] no rope table")
+    w = _fp32(dict(workloads.text_inputs([200, 33], 8, 2, seed=12), gate=True, theta=1e7))
+    att, plan = TextAttention(8, 2, 256, 64, rope_theta=1e7), AttnPlan(w["cu_seqlens"])
+    d = [w[k].cuda() for k in ("qkv", "q_norm", "k_norm", "pos3")]
+    kp, vp = att.planes(plan.kvT, fp32=True)
+    kw = dict(out_dtype="f32", k_plane=kp, vt_plane=vp, kvT=plan.kvT)
+    with_table = att.forward(*d, plan, rope_cs=att.rope_table(plan.T), **kw)
+    without = att.forward(*d, plan, stage="core", **kw)
+    torch.cuda.synchronize()
+    assert torch.equal(with_table.view(torch.int32), without.view(torch.int32))
