@@ -226,6 +226,15 @@ KvRows kv_rows_params(const clef_hip_attn_args *a, const int32_t *tok_kv) {
     return r;
 }
 
+// The bf16 K/V prologue as its own launch: K waves of 4 pass rows, then V waves of (kv head, 64 rows,
+// 16 dims); 4 waves per workgroup.
+bool prep_kv_bf16(const clef_hip_attn_args *a, const int32_t *tok_kv, void *stream, char *err, size_t errlen) {
+    const long waves = (long)(a->T + 3) / 4 + (long)a->nkv * ((a->T + 63) / 64) * 16;
+    hipLaunchKernelGGL(text_prep_direct_kernel, dim3((unsigned)((waves + 3) / 4)), dim3(kPrepDirectThreads), 0, (hipStream_t)stream,
+                       (const uint16_t *)a->qkv, a->row, kv_rows_params(a, tok_kv));
+    return launch_ok("text_prep_direct", err, errlen);
+}
+
 }  // namespace
 
 extern "C" {
@@ -507,11 +516,7 @@ bool clef_hip_attn_prep_kv(const clef_hip_attn_args *a, void *stream, char *err,
         return launch_ok("text_prep_kv_f32", err, errlen);
     }
     if (!a->tok_kv) return fail(err, errlen, "the K/V prologue needs tok_kv (the plan's pass row -> plane row map)");
-    // K waves of 4 pass rows, then V waves of (kv head, 64 rows, 16 dims); 4 waves per workgroup
-    const long waves = (long)(a->T + 3) / 4 + (long)a->nkv * ((a->T + 63) / 64) * 16;
-    hipLaunchKernelGGL(text_prep_direct_kernel, dim3((unsigned)((waves + 3) / 4)), dim3(kPrepDirectThreads), 0, (hipStream_t)stream,
-                       (const uint16_t *)a->qkv, a->row, kv_rows_params(a, a->tok_kv));
-    return launch_ok("text_prep_direct", err, errlen);
+    return prep_kv_bf16(a, a->tok_kv, stream, err, errlen);
 }
 
 bool clef_hip_attn_core(const clef_hip_attn_args *a, void *stream, char *err, size_t errlen) {
@@ -570,22 +575,46 @@ bool clef_hip_qkv_gemm(int H, const uint16_t *X, const uint16_t *W, const clef_h
     memset(&p, 0, sizeof(p));
     p.X = X; p.W = W; p.Y = (uint16_t *)a->qkv;
     p.T = a->T; p.N = (int)N; p.K = H; p.ldy = a->row;
-    p.n_tiles = (int)(N / gemm::BN);
-    p.n_per_xcd = (p.n_tiles + 7) / 8;
     p.r.T = a->T; p.r.nh = a->nh; p.r.nkv = a->nkv;
     if (tok_kv) {
         p.kv = 1;
         p.r = kv_rows_params(a, tok_kv);
     }
-    // 256 x 256 tiles, 8 waves of 128 x 64, 64-deep K slices double-buffered (128 KB of LDS):
-    // 128-row tiles moved 1.5x the operand bytes per product and ran fill-bound (0.59 against
-    // 0.53 ms at 4096 x 14336 x 5120); 32-deep slices four deep and 64 x 128 wave blocks measured
-    // no better
-    using C = gemm::Cfg<256, 128, 64, 64, 2>;
-    p.m_tiles = (a->T + C::BM - 1) / C::BM;
-    const long grid = 8L * p.n_per_xcd * p.m_tiles;
-    hipLaunchKernelGGL(gemm::qkv_gemm_kernel<C>, dim3((unsigned)grid), dim3(C::THREADS), 0, (hipStream_t)stream, p);
-    return launch_ok("qkv_gemm", err, errlen);
+    // The tile by its rounds over the 32 CUs of an XCD (tile_of deals N tiles to XCDs), times what a
+    // round takes relative to one of 256 x 256 tiles (us at 14336 x 5120 with T = 61 / 512 / 1024):
+    //   256 x 256 (111 / 137 / 138): the fewest operand bytes per product; 128-row tiles move 1.5 times as many
+    //             and run fill-bound on whole rounds (0.59 against 0.53 ms at T = 4096).
+    //   128 x 256 (75 / 87 / 161): twice the tiles, for passes that leave half the CUs without a 256-row one.
+    //   128 x 64, 64 x 64 (41, 38 / 154, 201 / -): few rows, where reading W is the work: 56 tiles of 256
+    //             columns pull 147 MB through 56 CUs, 224 narrow ones, six to eight slices deep, at 4 TB/s.
+    //             They hold no whole head, so the prologue follows as a launch (in these times).
+    // Each element's sum runs over k in the same order in all of them: the bits do not depend on the tile.
+    auto rounds = [&](int bm, int bn) {
+        const long n_per_xcd = (N / bn + 7) / 8, m = (a->T + bm - 1) / bm;
+        return (m * n_per_xcd + 31) / 32;
+    };
+    const long cost[4] = {100 * rounds(256, 256), 63 * rounds(128, 256), 38 * rounds(128, 64), 33 * rounds(64, 64)};
+    const int best = (int)(std::min_element(cost, cost + 4) - cost);
+    const bool kv = p.kv;
+    if (best >= 2) p.kv = 0;
+    auto launch = [&](auto CFG) {
+        using C = decltype(CFG);
+        p.n_tiles = (int)(N / C::BN);
+        p.n_per_xcd = (p.n_tiles + 7) / 8;
+        p.m_tiles = (a->T + C::BM - 1) / C::BM;
+        const long grid = 8L * p.n_per_xcd * p.m_tiles;
+        hipLaunchKernelGGL(gemm::qkv_gemm_kernel<C>, dim3((unsigned)grid), dim3(C::THREADS), 0, (hipStream_t)stream, p);
+        return launch_ok("qkv_gemm", err, errlen);
+    };
+    switch (best) {
+        // 8 waves of 128 x 64, 64-deep K slices double-buffered (128 KB of LDS); 32-deep slices four
+        // deep and 64 x 128 wave blocks measured no better
+        case 0: return launch(gemm::Cfg<256, 256, 128, 64, 64, 2>{});
+        case 1: return launch(gemm::Cfg<128, 256, 64, 64, 64, 3>{});
+        case 2: if (!launch(gemm::Cfg<128, 64, 64, 32, 64, 6>{})) return false; break;
+        default: if (!launch(gemm::Cfg<64, 64, 32, 32, 64, 8>{})) return false; break;
+    }
+    return !kv || prep_kv_bf16(a, tok_kv, stream, err, errlen);
 }
 
 bool clef_hip_attn_prefill(const clef_hip_attn_args *a, void *stream, char *err, size_t errlen) {

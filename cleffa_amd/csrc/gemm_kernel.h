@@ -3,11 +3,13 @@
 // them; f32 accumulation), the role of clef_metal_gemm (clef_metal.m:463-499) at its QKV call
 // (clef_metal.m:1326).
 //
-// Tiles of BM (256) rows x 256 columns, one per workgroup of 8 waves (2 per SIMD). A 256-column
-// tile of the QKV output is exactly one head's slice (a query or gate half of a q head, one K
+// Tiles of BM rows x BN columns, one per workgroup (clef_hip_qkv_gemm chooses by the number of tiles; 256 x
+// 256 with 8 waves, 2 per SIMD, for large passes). A 256-column tile of the QKV output is exactly one
+// head's slice (a query or gate half of a q head, one K
 // head or one V head), so the epilogue of a K tile holds whole key rows: it runs the RMSNorm,
 // rotary and f16 split of the K/V prologue on them and writes the K plane rows; a V tile writes
-// its V^T plane entries. Every output tile also leaves its bf16 rows in the qkv buffer.
+// its V^T plane entries. Every output tile also leaves its bf16 rows in the qkv buffer. Narrower
+// tiles write the rows only, and the prologue kernel follows.
 //   k loop:   BK-deep K slices of X and W stream global -> LDS with global_load_lds (16 bytes a
 //             lane), STAGES deep, into unpadded rows whose 16-byte chunks are XOR-swizzled, so
 //             the ds_read_b128 operand reads of 16 consecutive rows hit distinct banks. The
@@ -33,8 +35,7 @@ namespace gemm {
 
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 
-constexpr int BN = 256, HD = 256;
-constexpr int CS = 2 * BN + 16;                      // C-tile row stride in LDS (bytes)
+constexpr int HD = 256;                              // a head's columns: the N tile of the fused prologue
 constexpr int KALIGN = 64;                           // K must be a multiple of this
 
 struct Params {
@@ -77,11 +78,12 @@ __device__ __forceinline__ bool tile_of(const Params &p, int b, int *tm, int *tn
     return true;
 }
 
-// Kernel configuration: WM x WN output block per wave ((BM / WM) x (BN / WN) waves), K slices
-// of BK (32 or 64) staged STAGES deep in LDS.
-template <int BM_, int WM_, int WN_, int BK_, int STAGES_>
+// Kernel configuration: BM x BN output tile, WM x WN output block per wave ((BM / WM) x (BN / WN)
+// waves), K slices of BK (32 or 64) staged STAGES deep in LDS.
+template <int BM_, int BN_, int WM_, int WN_, int BK_, int STAGES_>
 struct Cfg {
-    static constexpr int BM = BM_, WM = WM_, WN = WN_, BK = BK_, STAGES = STAGES_;
+    static constexpr int BM = BM_, BN = BN_, WM = WM_, WN = WN_, BK = BK_, STAGES = STAGES_;
+    static constexpr int CS = 2 * BN + 16;                           // C-tile row stride in LDS (bytes)
     static constexpr int WAVES = (BM / WM) * (BN / WN), THREADS = 64 * WAVES;
     static constexpr int MT = WM / 16, NT = WN / 16, FR = MT + NT;   // 16-row / 16-column fragments
     static constexpr int KS = BK / 32;                               // 32-deep product steps per slice
@@ -112,29 +114,36 @@ __device__ __forceinline__ void read_frags(bf16x8 (&r)[NT + MT], unsigned wk, un
 // fragments, so that no copy or use of them can be placed between their reads and the wait.
 template <int N, int F>
 __device__ __forceinline__ void wait_frags(bf16x8 (&r)[F]) {
-    static_assert(F == 8 || F == 12, "fragment counts of the wave layouts");
-    if constexpr (F == 8)
+    static_assert(F == 4 || F == 6 || F == 8 || F == 12, "fragment counts of the wave layouts");
+    if constexpr (F == 4)
+        asm volatile("s_waitcnt lgkmcnt(%4)" : "+v"(r[0]), "+v"(r[1]), "+v"(r[2]), "+v"(r[3]) : "i"(N) : "memory");
+    else if constexpr (F == 6)
+        asm volatile("s_waitcnt lgkmcnt(%6)" : "+v"(r[0]), "+v"(r[1]), "+v"(r[2]), "+v"(r[3]), "+v"(r[4]), "+v"(r[5]) : "i"(N) : "memory");
+    else if constexpr (F == 8)
         asm volatile("s_waitcnt lgkmcnt(%8)" : "+v"(r[0]), "+v"(r[1]), "+v"(r[2]), "+v"(r[3]), "+v"(r[4]), "+v"(r[5]), "+v"(r[6]), "+v"(r[7]) : "i"(N) : "memory");
     else
         asm volatile("s_waitcnt lgkmcnt(%12)" : "+v"(r[0]), "+v"(r[1]), "+v"(r[2]), "+v"(r[3]), "+v"(r[4]), "+v"(r[5]), "+v"(r[6]), "+v"(r[7]), "+v"(r[8]), "+v"(r[9]), "+v"(r[10]), "+v"(r[11]) : "i"(N) : "memory");
 }
-// s_waitcnt vmcnt(b * FILLS) for a run-time b in [0, 4], then the workgroup barrier
+// s_waitcnt vmcnt(b * FILLS) for a run-time b in [0, 6], then the workgroup barrier
 template <int FILLS>
 __device__ __forceinline__ void wait_fills_barrier(int b) {
+    constexpr auto n = [](int k) { return k * FILLS < 63 ? k * FILLS : 63; };
     switch (b) {
         case 0: asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory"); break;
-        case 1: asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"i"(FILLS) : "memory"); break;
-        case 2: asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"i"(2 * FILLS) : "memory"); break;
-        case 3: asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"i"(3 * FILLS) : "memory"); break;
-        default: asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"i"(4 * FILLS) : "memory"); break;
+        case 1: asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"i"(n(1)) : "memory"); break;
+        case 2: asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"i"(n(2)) : "memory"); break;
+        case 3: asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"i"(n(3)) : "memory"); break;
+        case 4: asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"i"(n(4)) : "memory"); break;
+        case 5: asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"i"(n(5)) : "memory"); break;
+        default: asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"i"(n(6)) : "memory"); break;
     }
 }
 
 template <typename C>
 __global__ __launch_bounds__(C::THREADS, 1) void qkv_gemm_kernel(Params p) {
     constexpr int MT = C::MT, NT = C::NT, FR = C::FR, FILLS = C::FILLS, A_FILLS = C::A_FILLS, B_FILLS = C::B_FILLS;
-    constexpr int BM = C::BM, BK = C::BK, STAGES = C::STAGES, KS = C::KS, RS = 2 * BK;   // RS: LDS row bytes
-    static_assert(FILLS * (STAGES - 2) <= 63, "vmcnt range");
+    constexpr int BM = C::BM, BN = C::BN, CS = C::CS, BK = C::BK, STAGES = C::STAGES, KS = C::KS, RS = 2 * BK;   // RS: LDS row bytes
+    static_assert(FILLS * (STAGES - 2) <= 63 && STAGES <= 8, "vmcnt range");
     __shared__ __attribute__((aligned(1024))) uint8_t lds[C::LDS_BYTES];
     int tm, tn;
     if (!tile_of(p, blockIdx.x, &tm, &tn)) return;
@@ -246,11 +255,11 @@ __global__ __launch_bounds__(C::THREADS, 1) void qkv_gemm_kernel(Params p) {
     __syncthreads();
 #pragma unroll
     for (int i = 0; i < BM * BN * 2 / 16 / C::THREADS; i++) {
-        const int id = tid + C::THREADS * i, row = id >> 5, c16 = id & 31;
+        const int id = tid + C::THREADS * i, row = id / (BN / 8), c16 = id % (BN / 8);
         if (m0 + row < p.T)
             *(u32x4 *)(p.Y + (size_t)(m0 + row) * p.ldy + n0 + 8 * c16) = *(const u32x4 *)(lds + row * CS + 16 * c16);
     }
-    if (p.kv) {
+    if (BN == HD && p.kv) {
         const int kcol = 2 * p.r.nh * HD;
         float2 *table = (float2 *)(lds + BM * CS);
         if (n0 >= kcol && n0 < kcol + p.r.nkv * HD) k_rows<C::THREADS, BM>(p.r, lds, CS, m0, (n0 - kcol) / HD, table);

@@ -131,3 +131,28 @@ def test_fused_step_matches_oracle():
          "nh": 24, "nkv": 4, "hd": 256, "n_rot": 64, "gate": True, "theta": 1e7}
     rows = np.sort(np.random.default_rng(0).choice(int(cu[-1]), 256, replace=False))
     assert_close(out.float().cpu().numpy()[rows], oracle_text(w, rows=rows), what="fused step")
+
+
+@pytest.mark.parametrize("nh,nkv,H", [(24, 4, 64), (8, 2, 192), (16, 4, 576)])
+def test_rows_do_not_depend_on_the_pass_size(nh, nkv, H):
+    """The tile changes with the pass's rows (64 x 64, 128 x 64, 128 x 256, 256 x 256): a row's
+    projection and its planes keep their bits, at the edges of every tile, also where H gives fewer
+    slices than the pipeline is deep."""
+    q_norm, k_norm, pos3, cu = _plan_inputs([2100], nh, 4)
+    X, W = _operands(2100, H, nh, nkv, 6)
+    att = TextAttention(nh, nkv, 256, 64)
+
+    def run(T):
+        plan = AttnPlan(np.array([0, T], np.int32), causal=True)
+        kp, vp = att.planes(2112)
+        cs = att.rope_table(T)
+        qkv = att.project(X[:T].contiguous(), W, plan, q_norm, k_norm, pos3[:T].contiguous(), k_plane=kp, vt_plane=vp, kvT=2112, rope_cs=cs)
+        torch.cuda.synchronize()
+        return qkv, kp[:, :T], vp[:, :, :T], cs[:T]
+
+    full = run(2100)
+    for T in (1, 63, 64, 65, 128, 129, 255, 256, 257, 500, 700, 1024, 1025):
+        _say(f"[qkv_gemm] pass size {T} heads {nh}/{nkv} H={H}")
+        got = run(T)
+        for a, b in zip(got, (full[0][:T], full[1][:, :T], full[2][:, :, :T], full[3][:T])):
+            assert torch.equal(a.contiguous().view(torch.int16), b.contiguous().view(torch.int16)), T
