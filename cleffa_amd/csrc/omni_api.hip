@@ -117,9 +117,17 @@ bool clef_hip_omni_attention(const clef_hip_omni_attn_args *a, void *stream, cha
     p.q_plane = a->q_plane; p.k_plane = a->k_plane; p.v_plane = a->v_plane; p.blocks = a->blocks;
     p.out = a->out; p.nh = a->nh; p.nkv = a->nkv; p.T = a->T; p.kvT = a->kvT; p.n_blk = a->n_blk;
     p.scale = a->scale;
-    const long grid = (long)a->n_blk * a->nkv;
+    int w = a->nh / a->nkv, parts = 1;
+    // A group of 8 heads whose pass leaves half the CUs idle runs as two workgroups of 4 heads: one wave
+    // instead of two on each SIMD for every tile of the chain (401 tokens at 32 / 4 heads: 49.8 -> 42.5 us; 512: 58.9 -> 50.6).
+    int dev = 0, cus = 0;
+    if (w == 8 && hipGetDevice(&dev) == hipSuccess && hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess &&
+        2L * a->n_blk * a->nkv <= cus) {
+        w = 4;
+        parts = 2;
+    }
+    const long grid = (long)a->n_blk * a->nkv * parts;
     if (grid > 0x7fffffffL) return fail(err, errlen, "grid too large");
-    const int w = a->nh / a->nkv;
     const dim3 g((unsigned)grid), b(64 * w);
     hipStream_t s = (hipStream_t)stream;
     switch (w) {

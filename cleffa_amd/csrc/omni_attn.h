@@ -189,7 +189,7 @@ __device__ __noinline__ void omni_rows_plain(const AttnParams p, int q_row0, int
     }
 }
 
-// Grid: one workgroup per (block, kv head); wave w is q head kh * W + w.
+// Grid: one workgroup per (block, kv head, W heads of its group); wave w is head w of those.
 //
 // K and V tiles of 32 keys are split into their bf16 parts once per workgroup, on the way from
 // HBM to LDS: each thread's loads go out one tile ahead into registers, are split
@@ -211,11 +211,11 @@ __global__ __launch_bounds__(64 * W, W == 4 ? 2 : 1) void omni_attn_kernel(AttnP
     constexpr int KV = 3 * PL, BUF = 2 * KV;               // K planes, then V^T planes
     constexpr int NP = 8 / W;                              // 8-element pieces of K (and of V) per thread
     __shared__ __attribute__((aligned(16))) uint8_t smem[NB * BUF];
-    const int bi = blockIdx.x / p.nkv, kh = blockIdx.x % p.nkv;
+    const int n_parts = p.nh / p.nkv / W, kh = blockIdx.x % p.nkv, part = blockIdx.x / p.nkv % n_parts, bi = blockIdx.x / p.nkv / n_parts;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r16 = lane & 15, g = lane >> 4;
-    const int h = kh * W + wave;
+    const int h = (kh * n_parts + part) * W + wave;
     const int32_t *blk = p.blocks + 8 * bi;
     const int q_row0 = blk[0], nq = blk[1], q_pos0 = blk[2], k_row0 = blk[3], k_len = blk[4];
     const int n_tiles = (k_len + BK - 1) / BK;

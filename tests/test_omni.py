@@ -293,3 +293,20 @@ def test_omni_values_without_bf16_parts(nh, nkv, which):
         if which in ("v_inf", "v_big"):
             alone = _attend(Q[:, a:b], K[:, a:b], V[:, a:b], [0, b - a])
             assert np.array_equal(alone.view(np.uint32), got[a:b].view(np.uint32))
+
+
+@pytest.mark.gpu
+def test_omni_split_groups_agree_bitwise():
+    """A small pass runs a group of 8 heads as two workgroups of 4: a record's bytes are those it
+    has in a pass large enough for one workgroup per group, at both sides of the rule (2 x 16-row
+    blocks x kv heads against 256 CUs)."""
+    nh, nkv = 32, 4
+    lens = [33, 495, 512, 513] + [200] * 12
+    cu = np.concatenate([[0], np.cumsum(lens)])
+    Q, K, V = _planes(int(cu[-1]), nh, nkv, seed=11)
+    packed = _attend(Q, K, V, cu)
+    for r in range(4):
+        print(f"[omni] split groups, {lens[r]} tokens", flush=True)
+        a, b = cu[r], cu[r + 1]
+        alone = _attend(Q[:, a:b], K[:, a:b], V[:, a:b], [0, b - a])
+        assert np.array_equal(alone.view(np.uint32), packed[a:b].view(np.uint32))
