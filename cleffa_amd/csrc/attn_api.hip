@@ -587,14 +587,16 @@ bool clef_hip_qkv_gemm(int H, const uint16_t *X, const uint16_t *W, const clef_h
     //   128 x 256 (75 / 87 / 161): twice the tiles, for passes that leave half the CUs without a 256-row one.
     //   128 x 64, 64 x 64 (41, 38 / 154, 201 / -): few rows, where reading W is the work: 56 tiles of 256
     //             columns pull 147 MB through 56 CUs, 224 narrow ones, six to eight slices deep, at 4 TB/s.
-    //             They hold no whole head, so the prologue follows as a launch (in these times).
+    //   128 x 128 (52 / 108 / 194): in between, where it is one round and the others more or emptier (T = 160:
+    //             55 against 75 and 81; at 10240 x 4096 T = 384: 42 against 59 and 61).
+    //             The last three hold no whole head, so the prologue follows as a launch (in these times).
     // Each element's sum runs over k in the same order in all of them: the bits do not depend on the tile.
     auto rounds = [&](int bm, int bn) {
         const long n_per_xcd = (N / bn + 7) / 8, m = (a->T + bm - 1) / bm;
         return (m * n_per_xcd + 31) / 32;
     };
-    const long cost[4] = {100 * rounds(256, 256), 63 * rounds(128, 256), 38 * rounds(128, 64), 33 * rounds(64, 64)};
-    const int best = (int)(std::min_element(cost, cost + 4) - cost);
+    const long cost[5] = {100 * rounds(256, 256), 63 * rounds(128, 256), 38 * rounds(128, 64), 33 * rounds(64, 64), 48 * rounds(128, 128)};
+    const int best = (int)(std::min_element(cost, cost + 5) - cost);
     const bool kv = p.kv;
     if (best >= 2) p.kv = 0;
     auto launch = [&](auto CFG) {
@@ -612,7 +614,8 @@ bool clef_hip_qkv_gemm(int H, const uint16_t *X, const uint16_t *W, const clef_h
         case 0: return launch(gemm::Cfg<256, 256, 128, 64, 64, 2>{});
         case 1: return launch(gemm::Cfg<128, 256, 64, 64, 64, 3>{});
         case 2: if (!launch(gemm::Cfg<128, 64, 64, 32, 64, 6>{})) return false; break;
-        default: if (!launch(gemm::Cfg<64, 64, 32, 32, 64, 8>{})) return false; break;
+        case 3: if (!launch(gemm::Cfg<64, 64, 32, 32, 64, 8>{})) return false; break;
+        default: if (!launch(gemm::Cfg<128, 128, 64, 32, 64, 4>{})) return false; break;
     }
     return !kv || prep_kv_bf16(a, tok_kv, stream, err, errlen);
 }

@@ -135,7 +135,7 @@ def test_fused_step_matches_oracle():
 
 @pytest.mark.parametrize("nh,nkv,H", [(24, 4, 64), (8, 2, 192), (16, 4, 576)])
 def test_rows_do_not_depend_on_the_pass_size(nh, nkv, H):
-    """The tile changes with the pass's rows (64 x 64, 128 x 64, 128 x 256, 256 x 256): a row's
+    """The tile changes with the pass's rows (64 x 64, 128 x 64, 128 x 128, 128 x 256, 256 x 256): a row's
     projection and its planes keep their bits, at the edges of every tile, also where H gives fewer
     slices than the pipeline is deep."""
     q_norm, k_norm, pos3, cu = _plan_inputs([2100], nh, 4)
@@ -151,7 +151,7 @@ def test_rows_do_not_depend_on_the_pass_size(nh, nkv, H):
         return qkv, kp[:, :T], vp[:, :, :T], cs[:T]
 
     full = run(2100)
-    for T in (1, 63, 64, 65, 128, 129, 255, 256, 257, 500, 700, 1024, 1025):
+    for T in (1, 63, 64, 65, 128, 129, 255, 256, 257, 385, 500, 700, 1024, 1025):
         _say(f"[qkv_gemm] pass size {T} heads {nh}/{nkv} H={H}")
         got = run(T)
         for a, b in zip(got, (full[0][:T], full[1][:, :T], full[2][:, :, :T], full[3][:T])):
