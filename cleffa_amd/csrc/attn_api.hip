@@ -1,6 +1,7 @@
 // C ABI of the prefill attention path: argument checks, the host-side plan builder and the
 // kernel launches. Declarations and layouts are documented in include/clef_hip_attn.h.
 #include <hip/hip_runtime.h>
+#include <limits.h>
 #include <stdarg.h>
 #include <stdio.h>
 #include <stdlib.h>
@@ -589,16 +590,21 @@ bool clef_hip_qkv_gemm(int H, const uint16_t *X, const uint16_t *W, const clef_h
     //             columns pull 147 MB through 56 CUs, 224 narrow ones, six to eight slices deep, at 4 TB/s.
     //   128 x 128 (52 / 108 / 194): in between, where it is one round and the others more or emptier (T = 160:
     //             55 against 75 and 81; at 10240 x 4096 T = 384: 42 against 59 and 61).
-    //             The last three hold no whole head, so the prologue follows as a launch (in these times).
+    //             The three narrower than 256 columns hold no whole head, so the prologue follows as a
+    //             launch (in these times).
+    //   256 x 256, its last round as halves (226 at T = 1300 with the layer's attention, 250 without): where
+    //             that round fills at most half of the CUs (qkv_gemm_halved_kernel).
     // Each element's sum runs over k in the same order in all of them: the bits do not depend on the tile.
     auto rounds = [&](int bm, int bn) {
         const long n_per_xcd = (N / bn + 7) / 8, m = (a->T + bm - 1) / bm;
         return (m * n_per_xcd + 31) / 32;
     };
-    const long cost[5] = {100 * rounds(256, 256), 63 * rounds(128, 256), 38 * rounds(128, 64), 33 * rounds(64, 64), 48 * rounds(128, 128)};
-    const int best = (int)(std::min_element(cost, cost + 5) - cost);
+    const int most = (int)((N / 256 + 7) / 8 * ((a->T + 255L) / 256)), whole = gemm::whole_tiles(most);   // 256 x 256 tiles of an XCD
+    const long cost[6] = {100 * rounds(256, 256), 63 * rounds(128, 256), 38 * rounds(128, 64), 33 * rounds(64, 64), 48 * rounds(128, 128),
+                          whole == most ? LONG_MAX : 100L * (whole / gemm::XCD_CUS) + 63};
+    const int best = (int)(std::min_element(cost, cost + 6) - cost);
     const bool kv = p.kv;
-    if (best >= 2) p.kv = 0;
+    if (best >= 2 && best != 5) p.kv = 0;
     auto launch = [&](auto CFG) {
         using C = decltype(CFG);
         p.n_tiles = (int)(N / C::BN);
@@ -615,7 +621,20 @@ bool clef_hip_qkv_gemm(int H, const uint16_t *X, const uint16_t *W, const clef_h
         case 1: return launch(gemm::Cfg<128, 256, 64, 64, 64, 3>{});
         case 2: if (!launch(gemm::Cfg<128, 64, 64, 32, 64, 6>{})) return false; break;
         case 3: if (!launch(gemm::Cfg<64, 64, 32, 32, 64, 8>{})) return false; break;
-        default: if (!launch(gemm::Cfg<128, 128, 64, 32, 64, 4>{})) return false; break;
+        case 4: if (!launch(gemm::Cfg<128, 128, 64, 32, 64, 4>{})) return false; break;
+        default: {
+            p.n_tiles = (int)(N / 256);
+            p.n_per_xcd = (p.n_tiles + 7) / 8;
+            p.m_tiles = (a->T + 255) / 256;
+            int wgs = 0;   // of the XCD with the most; some own one N tile less
+            for (int x = 0; x < 8; x++) {
+                const int n = (p.n_tiles - x + 7) / 8 * p.m_tiles;
+                wgs = std::max(wgs, 2 * n - gemm::whole_tiles(n));
+            }
+            hipLaunchKernelGGL((gemm::qkv_gemm_halved_kernel<gemm::Cfg<256, 256, 128, 64, 64, 2>, gemm::Cfg<128, 256, 64, 64, 64, 3>>),
+                               dim3(8u * (unsigned)wgs), dim3(512), 0, (hipStream_t)stream, p);
+            return launch_ok("qkv_gemm", err, errlen);
+        }
     }
     return !kv || prep_kv_bf16(a, tok_kv, stream, err, errlen);
 }

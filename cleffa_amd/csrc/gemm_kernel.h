@@ -4,7 +4,7 @@
 // (clef_metal.m:1326).
 //
 // Tiles of BM rows x BN columns, one per workgroup (clef_hip_qkv_gemm chooses by the number of tiles; 256 x
-// 256 with 8 waves, 2 per SIMD, for large passes). A 256-column tile of the QKV output is exactly one
+// 256 with 8 waves, 2 per SIMD, for large passes, a last round of few as halves). A 256-column tile of the QKV output is exactly one
 // head's slice (a query or gate half of a q head, one K
 // head or one V head), so the epilogue of a K tile holds whole key rows: it runs the RMSNorm,
 // rotary and f16 split of the K/V prologue on them and writes the K plane rows; a V tile writes
@@ -139,14 +139,12 @@ __device__ __forceinline__ void wait_fills_barrier(int b) {
     }
 }
 
+// One BM x BN output tile (row of tiles tm, column of tiles tn) by the whole workgroup.
 template <typename C>
-__global__ __launch_bounds__(C::THREADS, 1) void qkv_gemm_kernel(Params p) {
+__device__ __forceinline__ void gemm_tile(const Params &p, uint8_t *lds, int tm, int tn) {
     constexpr int MT = C::MT, NT = C::NT, FR = C::FR, FILLS = C::FILLS, A_FILLS = C::A_FILLS, B_FILLS = C::B_FILLS;
     constexpr int BM = C::BM, BN = C::BN, CS = C::CS, BK = C::BK, STAGES = C::STAGES, KS = C::KS, RS = 2 * BK;   // RS: LDS row bytes
     static_assert(FILLS * (STAGES - 2) <= 63 && STAGES <= 8, "vmcnt range");
-    __shared__ __attribute__((aligned(1024))) uint8_t lds[C::LDS_BYTES];
-    int tm, tn;
-    if (!tile_of(p, blockIdx.x, &tm, &tn)) return;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int m0 = tm * BM, n0 = tn * BN;
@@ -264,6 +262,41 @@ __global__ __launch_bounds__(C::THREADS, 1) void qkv_gemm_kernel(Params p) {
         float2 *table = (float2 *)(lds + BM * CS);
         if (n0 >= kcol && n0 < kcol + p.r.nkv * HD) k_rows<C::THREADS, BM>(p.r, lds, CS, m0, (n0 - kcol) / HD, table);
         else if (n0 >= kcol + p.r.nkv * HD) v_rows<C::WAVES, BM>(p.r, lds, CS, m0, (n0 - kcol - p.r.nkv * HD) / HD);
+    }
+}
+
+template <typename C>
+__global__ __launch_bounds__(C::THREADS, 1) void qkv_gemm_kernel(Params p) {
+    __shared__ __attribute__((aligned(1024))) uint8_t lds[C::LDS_BYTES];
+    int tm, tn;
+    if (!tile_of(p, blockIdx.x, &tm, &tn)) return;
+    gemm_tile<C>(p, lds, tm, tn);
+}
+
+// C's tiles for the whole rounds of each XCD's CUs (one workgroup a CU: LDS), and a last round that fills at
+// most half of them as twice as many tiles H of half the rows, for the CUs that would idle. A tile's time
+// is its LDS fills, 48 KB of X and W a slice against 64 KB for half the products, so that
+// round takes 0.63 of a full one (not 0.5), and a round filled beyond half stays whole (two rounds of H
+// take 1.26). QKV projection and attention layer at 14336 x 5120, before and after: one record of 1,300 tokens
+// (1.3 rounds) 250 -> 226 us, 2,500 (2.2) 421 -> 393, 4,096 (3.5) 704 -> 690; 2,048 at 10240 x 4096 (1.25)
+// 228 -> 209. m_tiles and n_tiles count C's tiles.
+constexpr int XCD_CUS = 32;
+// tiles of an XCD with n of them that stay whole
+__host__ __device__ inline int whole_tiles(int n) { return n % XCD_CUS <= XCD_CUS / 2 ? n - n % XCD_CUS : n; }
+template <typename C, typename H>
+__global__ __launch_bounds__(C::THREADS, 1) void qkv_gemm_halved_kernel(Params p) {
+    static_assert(C::THREADS == H::THREADS && C::BM == 2 * H::BM && C::BN == H::BN, "halves of a tile");
+    __shared__ __attribute__((aligned(1024))) uint8_t lds[C::LDS_BYTES > H::LDS_BYTES ? C::LDS_BYTES : H::LDS_BYTES];
+    const int x = blockIdx.x & 7, j = blockIdx.x >> 3;
+    const int whole = whole_tiles(((p.n_tiles - x + 7) >> 3) * p.m_tiles);
+    int tm, tn;
+    if (j < whole) {
+        if (tile_of(p, 8 * j + x, &tm, &tn)) gemm_tile<C>(p, lds, tm, tn);
+    } else {
+        const int r = j - whole;
+        if (!tile_of(p, 8 * (whole + (r >> 1)) + x, &tm, &tn)) return;
+        tm = 2 * tm + (r & 1);
+        if (tm * H::BM < p.T) gemm_tile<H>(p, lds, tm, tn);
     }
 }
 

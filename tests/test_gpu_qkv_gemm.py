@@ -156,3 +156,30 @@ def test_rows_do_not_depend_on_the_pass_size(nh, nkv, H):
         got = run(T)
         for a, b in zip(got, (full[0][:T], full[1][:, :T], full[2][:, :, :T], full[3][:T])):
             assert torch.equal(a.contiguous().view(torch.int16), b.contiguous().view(torch.int16)), T
+
+
+@pytest.mark.parametrize("nh,nkv,T", [(24, 4, 1153), (24, 4, 1280), (24, 4, 2400), (16, 2, 1700), (16, 2, 1793), (60, 4, 520), (60, 4, 640)])
+def test_halved_last_round(nh, nkv, T):
+    """Passes whose last round of 256 x 256 tiles is at most half full run it as 128-row tiles (three to
+    sixteen tiles of an XCD, XCDs that own a tile less, a last half past the rows): each row's projection and planes
+    have the bits of a pass of 60 rows, which takes 64-column tiles."""
+    q_norm, k_norm, pos3, cu = _plan_inputs([T], nh, 8)
+    X, W = _operands(T, 128, nh, nkv, 9)
+    att = TextAttention(nh, nkv, 256, 64)
+
+    def run(a, b):
+        plan = AttnPlan(np.array([0, b - a], np.int32), causal=True)
+        kp, vp = att.planes(-(-(b - a) // 64) * 64)
+        cs = att.rope_table(b - a)
+        qkv = att.project(X[a:b].contiguous(), W, plan, q_norm, k_norm, pos3[a:b].contiguous(), k_plane=kp, vt_plane=vp,
+                          kvT=kp.shape[1], rope_cs=cs)
+        torch.cuda.synchronize()
+        return qkv, kp[:, :b - a], vp[:, :, :b - a], cs[:b - a]
+
+    _say(f"[qkv_gemm] halved last round {T} rows, heads {nh}/{nkv}")
+    got = run(0, T)
+    for a in range(0, T, 60):
+        b = min(a + 60, T)
+        want = run(a, b)
+        for g, w in zip((got[0][a:b], got[1][:, a:b], got[2][:, :, a:b], got[3][a:b]), want):
+            assert torch.equal(g.contiguous().view(torch.int16), w.contiguous().view(torch.int16)), (a, b)
