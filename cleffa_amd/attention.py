@@ -138,10 +138,7 @@ class AttnPlan:
         self.n_blk = n_blk.value
         self.kv_rows = kv_rows.value
         self.blocks_host = blocks[: self.n_blk].copy()
-        # the last pass row and kv row that the blocks reach: what each call is checked against
-        b = self.blocks_host
-        self.q_end = int((b[:, 0] + b[:, 1]).max()) if self.n_blk else 0
-        self.k_end = int((b[:, 3] + b[:, 4]).max()) if self.n_blk else 0
+        self._set_bounds()
         self.tok_kv_host = tok_kv[: self.T].copy()
         self.kv_tok_host = kv_tok[: self.kv_rows].copy()
         self.device = _device(device)
@@ -154,6 +151,17 @@ class AttnPlan:
         # a key that leaves f16's range
         seq_start = np.repeat(cu_q[:-1], np.diff(cu_q)).astype(np.int32)
         self.seq_start = torch.from_numpy(np.ascontiguousarray(seq_start if self.T else np.zeros(1, np.int32))).to(self.device)
+
+    def _set_bounds(self):
+        """The last pass row and kv row that the blocks reach: what each call is checked against."""
+        b = self.blocks_host
+        self.q_end = int((b[:, 0] + b[:, 1]).max()) if self.n_blk else 0
+        self.k_end = int((b[:, 3] + b[:, 4]).max()) if self.n_blk else 0
+
+    def __setstate__(self, state):   # copies and saved plans, whose state may hold neither bounds nor schedules
+        self.__dict__.update(state)
+        self.__dict__.setdefault("_sched", {})
+        self._set_bounds()
 
     def schedule(self, nh, nkv, n_wg):
         """Per-workgroup item lists of the attention core over n_wg workgroups (device int32,

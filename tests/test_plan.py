@@ -1,5 +1,7 @@
 """Host-side plan builder (clef_hip_attn_plan, the block list of clef_metal.m:1243-1257 and the
 packing of clef.c:470-497): coverage, key ranges, order and kv-row layout. Runs on the CPU."""
+import pickle
+
 import numpy as np
 import pytest
 
@@ -245,3 +247,14 @@ def test_plan_fingerprint():
     assert len(seen) == 5
     # FNV-1a known answer: the empty input hashes to the offset basis
     assert _fnv_fingerprint(np.zeros((0, 8), np.int32)) == np.int32(np.uint32(2166136261 | 1).view(np.int32))
+
+
+def test_saved_plan_without_bounds_is_restored():
+    """A plan saved without the bounds and schedules that calls read gets them when it is loaded."""
+    plan = AttnPlan(np.array([0, 37, 300], np.int32), device="cpu")
+    state = {k: v for k, v in plan.__dict__.items() if k not in ("q_end", "k_end", "_sched")}
+    old = AttnPlan.__new__(AttnPlan)
+    old.__setstate__(state)
+    assert (old.q_end, old.k_end, old._sched) == (plan.q_end, plan.k_end, {})
+    again = pickle.loads(pickle.dumps(plan))
+    assert (again.q_end, again.k_end) == (300, plan.k_end) and np.array_equal(again.blocks_host, plan.blocks_host)
