@@ -190,7 +190,9 @@ bool clef_hip_attn_schedule(const int32_t *blocks, int n_blk, int nh, int nkv, i
  * plane row map, [T]) != NULL: every K head's rows are normalised, rotated and written to the K
  * plane and every V head's to the V^T plane, bitwise what clef_hip_attn_prep_kv writes from the
  * same qkv rows (with the same flags and rope_cs), so clef_hip_attn_core may follow directly;
- * NULL: the product only. H must be a multiple of 64; X and W at most 4 GiB each. */
+ * NULL: the product only. Passes of few rows take tiles narrower than a head and launch the
+ * prologue after the product, with the same results. H must be a multiple of 64; X and W at most
+ * 4 GiB each. */
 bool clef_hip_qkv_gemm(int H, const uint16_t *X, const uint16_t *W, const clef_hip_attn_args *a, const int32_t *tok_kv,
                        void *stream, char *err, size_t errlen);
 
