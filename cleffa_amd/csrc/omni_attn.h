@@ -147,8 +147,8 @@ __device__ __forceinline__ float xrow_max(float x) {
     return fmaxf(__uint_as_float(q[0]), __uint_as_float(q[1]));
 }
 
-// The rows of a work item in plain FP32 (FP64 sums), for items whose K, V or Q hold values that have no bf16 parts
-// (infinities, magnitudes above bf16's overflow threshold): each wave runs its head's rows one by
+// The rows of a work item in plain FP32 (FP64 sums), for items whose K, V or Q hold infinities or magnitudes whose
+// FP32 sum over a tile could overflow (split_bad: from 2^121): each wave runs its head's rows one by
 // one, a lane per key for the scores and two dims per lane for the output. Slow, and only a
 // pass that is not finite (status 2) or next to FP32's limit gets here.
 __device__ __noinline__ void omni_rows_plain(const AttnParams p, int q_row0, int nq, int q_pos0, int k_row0, int k_len, int h, int kh) {

@@ -10,8 +10,9 @@
 //
 // The split is exact for finite |x| below bf16's overflow threshold (0x7f7f8000) whose parts stay
 // clear of the subnormals (|x| above about 2^-108; below, an absolute 2^-133 is lost). Larger and infinite
-// values give infinite or NaN parts: kernels note the largest magnitude they split
-// (split_amax / split_bad) and recompute such work items with plain FP32 arithmetic. A NaN gives NaN.
+// values give infinite or NaN parts, and sums of values next to that threshold are infinite: kernels note
+// the largest magnitude they split (split_amax / split_bad) and recompute such work items with
+// plain FP32 arithmetic. A NaN gives NaN.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -70,8 +71,9 @@ __device__ __forceinline__ float split_amax(float amax, const float (&x)[8]) {
     for (int i = 0; i < 8; i += 2) split_amax2(amax, x[i], x[i + 1]);
     return amax;
 }
-// whether a value of that magnitude has no finite parts
-__device__ __forceinline__ bool split_bad(float amax) { return amax >= __uint_as_float(0x7f7f8000u); }
+// Whether a value of that magnitude is left to plain arithmetic: from 2^121 on. Its parts are finite up to
+// 0x7f7f8000 (3.39e38), but the sum over a tile's 32 keys, with probabilities up to 1, has to be as well.
+__device__ __forceinline__ bool split_bad(float amax) { return amax >= 0x1p121f; }
 
 template <typename F, int... I>
 __device__ __forceinline__ void sfor_impl(F &&f, std::integer_sequence<int, I...>) {

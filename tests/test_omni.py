@@ -296,6 +296,23 @@ def test_omni_values_without_bf16_parts(nh, nkv, which):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("nh,nkv", [(8, 1), (4, 1)])
+@pytest.mark.parametrize("big", [1e36, 1.1e37, 2e37, 1e38, 3.3e38])
+def test_omni_sums_of_large_values_stay_finite(nh, nkv, big):
+    """Equal scores over values whose plain sum leaves FP32's range: the output is their mean, finite.
+    Bound: FP32 sums of 32 equally signed values (32 roundings of 2^-24 at most), FP64 across tiles,
+    one rounding of the output: 33 x 2^-24 = 2e-6 of the largest value."""
+    print(f"[omni] values of {big:g} {nh}/{nkv}", flush=True)
+    T = 100
+    Q, K, V = _planes(T, nh, nkv, seed=3)
+    Q[:] = 0
+    V = (big * np.random.default_rng(1).uniform(0.9, 1.0, V.shape)).astype(np.float32)
+    got, want = _attend(Q, K, V, [0, 33, T]), _reference(Q, K, V, [0, 33, T])
+    assert np.isfinite(got).all()
+    assert np.abs(got - want).max() < 2e-6 * big
+
+
+@pytest.mark.gpu
 def test_omni_split_groups_agree_bitwise():
     """A small pass runs a group of 8 heads as two workgroups of 4: a record's bytes are those it
     has in a pass large enough for one workgroup per group, at both sides of the rule (2 x 16-row
