@@ -140,14 +140,15 @@ __device__ __forceinline__ float xrow_max(float x) {
     return fmaxf(__uint_as_float(q[0]), __uint_as_float(q[1]));
 }
 
-// The rows of a wave in plain FP32, for items whose Q, K or V hold values that have no bf16 parts
-// (infinities, magnitudes above bf16's overflow threshold): one row after the other, a lane per key
+// The rows of `rows` (a bit each) of a wave in plain FP32, for rows whose Q or a key that they see holds an
+// infinity, a NaN or a magnitude next to FP32's limit (split_bad): one row after the other, a lane per key
 // for the scores and four dims per lane for q and the output.
-__device__ __noinline__ void text_rows_plain(const Params p, int q_row0, int nq, int q_pos0, int k_row0, int k_len, int h, int kh, int32_t *flag) {
+__device__ __noinline__ void text_rows_plain(const Params p, unsigned rows, int q_row0, int q_pos0, int k_row0, int k_len, int h, int kh, int32_t *flag) {
     const int lane = threadIdx.x & 63;
     const float *kbase = p.k_plane + ((size_t)kh * p.kvT + k_row0) * HD;
     const float *vbase = p.v_plane + ((size_t)kh * p.kvT + k_row0) * HD;
-    for (int r = 0; r < nq; r++) {
+    for (int r = 0; r < 16; r++) {
+        if (!((rows >> r) & 1)) continue;
         const int t = q_row0 + r;
         const float *src = p.qkv + (size_t)t * p.row + (size_t)h * 2 * HD + 4 * lane;
         f32x4 q = *(const f32x4 *)src;
@@ -249,6 +250,7 @@ __global__ __launch_bounds__(64 * NW) void attn_text_f32_kernel(Params p) {
         const int q_row0 = blk[0] + r0 + (live ? 16 * (wave - slot * wph) : 0), q_pos0 = blk[2] + q_row0 - blk[0];
         const int nq = live ? min(16, blk[0] + r0 + rows - q_row0) : 0;
         const int k_row0 = blk[3], k_len = p.causal ? min(blk[4], blk[2] + r0 + rows) : blk[4];
+        const int whole = p.causal ? min(k_len, blk[2] + r0 + 1) : k_len;   // keys that every row of the item sees
         int32_t *const flag = p.ovf ? p.ovf + blk[5] : nullptr;
         const int n_tiles = (k_len + BK - 1) / BK;
         // keys this wave's rows see, and the tiles it runs
@@ -261,7 +263,8 @@ __global__ __launch_bounds__(64 * NW) void attn_text_f32_kernel(Params p) {
         // ---- tile staging, two pieces a thread. Piece e: K dims 8 c .. 8 c + 7
         // of one key, V keys 8 kg .. 8 kg + 7 of one dim; each load is a uniform base plus a
         // 32-bit lane offset. Keys past the item's range become zeros: their zero probabilities
-        // then give zero products, and what lies there cannot flag the item.
+        // then give zero products, and what lies there cannot flag the item. So do values of V that
+        // are left to plain arithmetic, in tiles that some row sees in part.
         float raw[2][8];
         const unsigned ko = 32u * tid, vo = (tid >> 8) * (8u * HD * 4u) + (tid & 255) * 4u;
         auto load_k = [&](int kb) {
@@ -311,11 +314,15 @@ __global__ __launch_bounds__(64 * NW) void attn_text_f32_kernel(Params p) {
             put(dst_k);
         };
         auto put_v = [&](int kb) {
-            if (kb + BK > k_len) {
+            if (kb + BK > whole) {
 #pragma unroll
-                for (int e = 0; e < 2; e++)
+                for (int e = 0; e < 2; e++) {
 #pragma unroll
                     for (int j = 0; j < 8; j++) raw[e][j] = kb + 8 * (tid >> 8) + 2 * NW * e + j < k_len ? raw[e][j] : 0.f;
+                    amax = split32::split_amax(amax, raw[e]);
+#pragma unroll
+                    for (int j = 0; j < 8; j++) raw[e][j] = split32::split_bad(raw[e][j]) ? 0.f : raw[e][j];
+                }
             }
             put(dst_v);
         };
@@ -478,9 +485,17 @@ __global__ __launch_bounds__(64 * NW) void attn_text_f32_kernel(Params p) {
         float l_row = l_run;
         l_row += __shfl_xor(l_row, 16);
         l_row += __shfl_xor(l_row, 32);
-        if (__syncthreads_or(split32::split_bad(amax))) {   // also: the tiles' last reads are done
-            if (live) text_rows_plain(p, q_row0, nq, q_pos0, k_row0, k_len, h, kh, flag);
-        } else if (q_valid) {
+        bool plain = false;
+        if (__syncthreads_or(!split32::split_fine(amax))) {   // also: the tiles' last reads are done
+            const int first = split32::first_bad_key<HD>(kbase, vbase, k_len, (int *)smem);
+            int own = 0;
+#pragma unroll
+            for (int c = 0; c < 8; c++) own |= split32::query_bad(qh[c]);
+            own |= __shfl_xor(own, 16);
+            own |= __shfl_xor(own, 32);
+            plain = q_valid && (own || first < (p.causal ? q_pos0 + r16 + 1 : k_len));
+        }
+        if (q_valid && !plain) {
             const float il = l_row > 0.f ? 1.0f / l_row : 0.f;
             const size_t t = (size_t)(q_row0 + r16);
             const size_t obase = t * p.nh * HD + (size_t)h * HD + 8 * g;
@@ -510,6 +525,8 @@ __global__ __launch_bounds__(64 * NW) void attn_text_f32_kernel(Params p) {
             else if (p.out_type == CLEF_HIP_OUT_BF16) store(CLEF_HIP_OUT_BF16);
             else store(CLEF_HIP_OUT_F16);
         }
+        const unsigned plain_rows = (unsigned)__ballot(plain) & 0xffffu;
+        if (plain_rows) text_rows_plain(p, plain_rows, q_row0, q_pos0, k_row0, k_len, h, kh, flag);
     }
 }
 

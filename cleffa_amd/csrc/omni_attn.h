@@ -147,15 +147,16 @@ __device__ __forceinline__ float xrow_max(float x) {
     return fmaxf(__uint_as_float(q[0]), __uint_as_float(q[1]));
 }
 
-// The rows of a work item in plain FP32 (FP64 sums), for items whose K, V or Q hold infinities or magnitudes whose
-// FP32 sum over a tile could overflow (split_bad: from 2^121): each wave runs its head's rows one by
-// one, a lane per key for the scores and two dims per lane for the output. Slow, and only a
+// The rows of `rows` (a bit each) of a wave in plain FP32 (FP64 sums), for rows whose Q or a key that they see holds
+// an infinity, a NaN or a magnitude whose FP32 sum over a tile could overflow (split_bad: from 2^121): one
+// by one, a lane per key for the scores and two dims per lane for the output. Slow, and only a
 // pass that is not finite (status 2) or next to FP32's limit gets here.
-__device__ __noinline__ void omni_rows_plain(const AttnParams p, int q_row0, int nq, int q_pos0, int k_row0, int k_len, int h, int kh) {
+__device__ __noinline__ void omni_rows_plain(const AttnParams p, unsigned rows, int q_row0, int q_pos0, int k_row0, int k_len, int h, int kh) {
     const int lane = threadIdx.x & 63;
     const float *kbase = p.k_plane + ((size_t)kh * p.kvT + k_row0) * HD;
     const float *vbase = p.v_plane + ((size_t)kh * p.kvT + k_row0) * HD;
-    for (int r = 0; r < nq; r++) {
+    for (int r = 0; r < BQ; r++) {
+        if (!((rows >> r) & 1)) continue;
         const float *q = p.q_plane + ((size_t)h * p.T + q_row0 + r) * HD;
         const int keys = min(k_len, q_pos0 + r + 1);
         float m = -INFINITY;
@@ -220,7 +221,7 @@ __global__ __launch_bounds__(64 * W, W == 4 ? 2 : 1) void omni_attn_kernel(AttnP
     const int q_row0 = blk[0], nq = blk[1], q_pos0 = blk[2], k_row0 = blk[3], k_len = blk[4];
     const int n_tiles = (k_len + BK - 1) / BK;
     const bool q_valid = r16 < nq;
-    const int qpos = q_pos0 + r16;
+    const int qpos = q_pos0 + r16, whole = min(k_len, q_pos0 + 1);   // whole: keys that every row sees
     const float *kbase = p.k_plane + ((size_t)kh * p.kvT + k_row0) * HD;
     const float *vbase = p.v_plane + ((size_t)kh * p.kvT + k_row0) * HD;
     float amax = 0.f;
@@ -248,14 +249,14 @@ __global__ __launch_bounds__(64 * W, W == 4 ? 2 : 1) void omni_attn_kernel(AttnP
             for (int j = 0; j < 8; j++) vr[e][j] = s[j * HD];
         }
     };
-    auto put = [&](uint8_t *dst, const split32::Parts &s) {
+    auto put = [&](uint8_t *dst, const split32::Parts &s) __attribute__((always_inline)) {
         *(bf16x8 *)dst = s.h;
         *(bf16x8 *)(dst + PL) = s.m;
         *(bf16x8 *)(dst + 2 * PL) = s.l;
     };
     // K chunk c of key 8a + 4t + b sits at position c ^ (4a + b): the 16 rows one operand read
     // touches then hit 16 distinct 16-byte slots.
-    auto put_k = [&](uint8_t *buf) {
+    auto put_k = [&](uint8_t *buf) __attribute__((always_inline)) {
 #pragma unroll
         for (int e = 0; e < NP; e++) {
             const int i = tid + 64 * W * e, key = i >> 4, c = i & 15;
@@ -266,7 +267,7 @@ __global__ __launch_bounds__(64 * W, W == 4 ? 2 : 1) void omni_attn_kernel(AttnP
     // V^T row d: its four 8-key chunks at position kg ^ (-(d / 8) % 4) ^ ((d / 4) % 2): the 16
     // lanes one step of a ds_read_b128 or ds_write_b128 serves, consecutive or {0-3, 12-15, 20-27}
     // and its like, hit 16 distinct 16-byte slots.
-    auto put_v = [&](uint8_t *buf) {
+    auto put_v = [&](uint8_t *buf) __attribute__((always_inline)) {
 #pragma unroll
         for (int e = 0; e < NP; e++) {
             const int i = tid + 64 * W * e, d = i & 127, kg = i >> 7;
@@ -275,19 +276,23 @@ __global__ __launch_bounds__(64 * W, W == 4 ? 2 : 1) void omni_attn_kernel(AttnP
         }
     };
     // Keys past the item's range (slack, or another record's) become zeros: their zero probabilities
-    // then give zero products, and what lies there cannot send the item down the plain path.
-    auto clear_k = [&](int kb) {
+    // then give zero products, and what lies there cannot send a row down the plain path. So do values of V
+    // that are left to it, in tiles that some row sees in part.
+    auto clear_k = [&](int kb) __attribute__((always_inline)) {
 #pragma unroll
         for (int e = 0; e < NP; e++)
 #pragma unroll
             for (int j = 0; j < 8; j++) kr[e][j] = kb + ((tid + 64 * W * e) >> 4) < k_len ? kr[e][j] : 0.f;
     };
-    auto clear_v = [&](int kb) {
+    auto clear_v = [&](int kb) __attribute__((always_inline)) {
 #pragma unroll
         for (int e = 0; e < NP; e++) {
             const int kg = (tid + 64 * W * e) >> 7;
 #pragma unroll
             for (int j = 0; j < 8; j++) vr[e][j] = kb + 8 * kg + j < k_len ? vr[e][j] : 0.f;
+            amax = split32::split_amax(amax, vr[e]);
+#pragma unroll
+            for (int j = 0; j < 8; j++) vr[e][j] = split32::split_bad(vr[e][j]) ? 0.f : vr[e][j];
         }
     };
 
@@ -328,7 +333,7 @@ __global__ __launch_bounds__(64 * W, W == 4 ? 2 : 1) void omni_attn_kernel(AttnP
         put_k(smem);
         if (n_tiles > 1) load_k(BK);
         if constexpr (PP) {
-            if (BK > k_len) clear_v(0);
+            if (BK > whole) clear_v(0);
             put_v(smem);
             if (n_tiles > 1) {
                 load_v(BK);
@@ -359,7 +364,7 @@ __global__ __launch_bounds__(64 * W, W == 4 ? 2 : 1) void omni_attn_kernel(AttnP
     // terms in one accumulator, the smaller ones in another), and O^T += V^T . P^T of the tile at
     // vbuf (pairs of 16-dim tiles, FP32 over the tile's 32 keys, then into the FP64
     // accumulators). Every step is six operand reads and twelve products.
-    auto products = [&](unsigned kbuf, unsigned vbuf, auto S, auto PV, float (&x)[8]) {
+    auto products = [&](unsigned kbuf, unsigned vbuf, auto S, auto PV, float (&x)[8]) __attribute__((always_inline)) {
         constexpr int n_s = decltype(S)::value ? 4 : 0, n = n_s + (decltype(PV)::value ? 4 : 0);
         constexpr int LOOK = W == 4 ? 1 : 2;   // steps the reads run ahead (two waves of W = 4 share a SIMD's registers with 16 staged values more)
         split32::Six ring[LOOK];
@@ -419,7 +424,7 @@ __global__ __launch_bounds__(64 * W, W == 4 ? 2 : 1) void omni_attn_kernel(AttnP
     // One trip (FIRST: no P.V yet). EDGE: some key of the tile lies past a row's position, or the
     // tiles it stages may reach past the record's end.
     int bt = 0;   // t % NB
-    auto trip = [&](const int t, auto FIRST, auto EDGE) {
+    auto trip = [&](const int t, auto FIRST, auto EDGE) __attribute__((always_inline)) {
         constexpr bool first = decltype(FIRST)::value, edge = decltype(EDGE)::value;
         const int kb = t * BK;
         const int b_next = bt + 1 < NB ? bt + 1 : 0, b_prev = bt > 0 ? bt - 1 : NB - 1;
@@ -437,7 +442,7 @@ __global__ __launch_bounds__(64 * W, W == 4 ? 2 : 1) void omni_attn_kernel(AttnP
         }
         if (!edge || t + 2 + AH < n_tiles) load_k(min(t + 2 + AH, n_tiles - 1) * BK);
         if (!edge || t + AH < n_tiles) {
-            if (edge && kb + (1 + AH) * BK > k_len) clear_v(kb + AH * BK);
+            if (edge && kb + (1 + AH) * BK > whole) clear_v(kb + AH * BK);
             put_v(smem + (PP ? b_next : 0) * BUF);
         }
         if (!edge || t + 1 + AH < n_tiles) load_v(min(t + 1 + AH, n_tiles - 1) * BK);
@@ -481,8 +486,8 @@ __global__ __launch_bounds__(64 * W, W == 4 ? 2 : 1) void omni_attn_kernel(AttnP
     };
     using T = std::true_type;
     using F = std::false_type;
-    // trips whose tile every row sees whole, with the tiles they stage inside the record
-    const int n_inner = min((q_pos0 + 1) / BK, k_len / BK - AH - 1);
+    // trips whose tile every row sees whole, as the V that they stage, with the K they stage inside the record
+    const int n_inner = min((q_pos0 + 1) / BK - AH, k_len / BK - AH - 1);
     if (n_tiles > 0) {
         const bool late = PP && wave >= W / 2;
         if (late) half_barrier();
@@ -500,11 +505,17 @@ __global__ __launch_bounds__(64 * W, W == 4 ? 2 : 1) void omni_attn_kernel(AttnP
     double l_row = l_run;
     l_row += __shfl_xor(l_row, 16);
     l_row += __shfl_xor(l_row, 32);
-    if (__syncthreads_or(split32::split_bad(amax))) {
-        omni_rows_plain(p, q_row0, nq, q_pos0, k_row0, k_len, h, kh);
-        return;
+    bool plain = false;
+    if (__syncthreads_or(!split32::split_fine(amax))) {
+        const int first = split32::first_bad_key<HD>(kbase, vbase, k_len, (int *)smem);
+        int own = 0;
+#pragma unroll
+        for (int c = 0; c < 4; c++) own |= split32::query_bad(qh[c]);
+        own |= __shfl_xor(own, 16);
+        own |= __shfl_xor(own, 32);
+        plain = q_valid && (own || first <= qpos);
     }
-    if (q_valid) {
+    if (q_valid && !plain) {
         const double il = l_row > 0.0 ? 1.0 / l_row : 0.0;
         float *dst = p.out + (size_t)(q_row0 + r16) * p.nh * HD + (size_t)h * HD + 8 * g;
 #pragma unroll
@@ -515,6 +526,8 @@ __global__ __launch_bounds__(64 * W, W == 4 ? 2 : 1) void omni_attn_kernel(AttnP
             *(f32x4 *)(dst + 32 * (n >> 1) + 4 * (n & 1)) = w;
         }
     }
+    const unsigned rows = (unsigned)__ballot(plain) & 0xffffu;
+    if (rows) omni_rows_plain(p, rows, q_row0, q_pos0, k_row0, k_len, h, kh);
 }
 
 }  // namespace omni

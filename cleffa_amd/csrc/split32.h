@@ -10,11 +10,11 @@
 //
 // The split is exact for finite |x| below bf16's overflow threshold (0x7f7f8000) whose parts stay
 // clear of the subnormals (|x| above about 2^-108; below, an absolute 2^-133 is lost). Larger and infinite
-// values give infinite or NaN parts, and sums of values next to that threshold are infinite: kernels note
-// the largest magnitude they split (split_amax / split_bad) and recompute such work items with
-// plain FP32 arithmetic. A NaN gives NaN.
+// values and NaN give infinite or NaN parts, and sums of values next to that threshold are infinite: rows that
+// meet one are left to plain arithmetic (split_bad).
 #pragma once
 #include <hip/hip_runtime.h>
+#include <limits.h>
 #include <stdint.h>
 
 #include <utility>
@@ -64,16 +64,50 @@ __device__ __forceinline__ Parts split8(const float (&x)[8], const Weights &w) {
     return {__builtin_bit_cast(bf16x8, h), __builtin_bit_cast(bf16x8, m), __builtin_bit_cast(bf16x8, l)};
 }
 
-// Largest magnitude of a running maximum and eight values (a NaN does not count: its parts are NaN).
-__device__ __forceinline__ void split_amax2(float &amax, float a, float b) { asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(amax) : "v"(a), "v"(b)); }
+// Values that are left to plain arithmetic: infinities, NaN and magnitudes from 2^121 on. Parts are finite up to
+// 0x7f7f8000 (3.39e38), but the sum over a tile's 32 keys, with probabilities up to 1, has to be as well.
+// A row is computed with plain arithmetic if its own Q or a key that it sees holds such a value, which does
+// not depend on how the pass is cut into items. A kernel therefore
+//   keeps the largest magnitude it splits (split_amax); an item without such values (split_fine) is done;
+//   stages such values of V as zeros in tiles that some row sees in part, so that the rows which do not see
+//     them keep their sums, with that key's zero probability, clear of infinities and NaN;
+//   finds the first key with such a value (first_bad_key) and the rows concerned at an item's end.
+constexpr float LIMIT = 0x1p121f;
+__device__ __forceinline__ bool split_bad(float x) { return !(fabsf(x) < LIMIT); }
+// Largest magnitude of a running maximum and eight values; a NaN stays. (In asm: with the builtin the
+// compiler kept the values longer and spilled 13 registers of the text kernel.)
 __device__ __forceinline__ float split_amax(float amax, const float (&x)[8]) {
-#pragma unroll
-    for (int i = 0; i < 8; i += 2) split_amax2(amax, x[i], x[i + 1]);
+    asm("v_maximum3_f32 %0, |%1|, |%2|, %0\n\tv_maximum3_f32 %0, |%3|, |%4|, %0\n\t"
+        "v_maximum3_f32 %0, |%5|, |%6|, %0\n\tv_maximum3_f32 %0, |%7|, |%8|, %0"
+        : "+v"(amax) : "v"(x[0]), "v"(x[1]), "v"(x[2]), "v"(x[3]), "v"(x[4]), "v"(x[5]), "v"(x[6]), "v"(x[7]));
     return amax;
 }
-// Whether a value of that magnitude is left to plain arithmetic: from 2^121 on. Its parts are finite up to
-// 0x7f7f8000 (3.39e38), but the sum over a tile's 32 keys, with probabilities up to 1, has to be as well.
-__device__ __forceinline__ bool split_bad(float amax) { return amax >= 0x1p121f; }
+// (the margin: a bad query is told by its high parts, rounded)
+__device__ __forceinline__ bool split_fine(float amax) { return amax < 0.99f * LIMIT; }
+__device__ __forceinline__ bool query_bad(bf16x8 h) {
+    const u32x4 w = __builtin_bit_cast(u32x4, h);
+    bool bad = false;
+#pragma unroll
+    for (int i = 0; i < 4; i++) bad |= split_bad(bf_lo(w[i])) || split_bad(bf_hi(w[i]));
+    return bad;
+}
+// The first of k_len keys with such a value in its K or V row (HD dims, rows HD apart), INT_MAX: none. Every thread
+// of the workgroup calls it; `shared` is an LDS word that nobody uses any more.
+template <int HD>
+__device__ __forceinline__ int first_bad_key(const float *k, const float *v, int k_len, int *shared) {
+    const int per_row = HD / 4, c = threadIdx.x % per_row * 4;
+    __syncthreads();
+    if (threadIdx.x == 0) *shared = INT_MAX;
+    __syncthreads();
+    for (int key = threadIdx.x / per_row; key < k_len && key < *(volatile int *)shared; key += blockDim.x / per_row) {
+        const f32x4 a = *(const f32x4 *)(k + (size_t)key * HD + c), b = *(const f32x4 *)(v + (size_t)key * HD + c);
+        bool bad = false;
+        for (int e = 0; e < 4; e++) bad |= split_bad(a[e]) || split_bad(b[e]);
+        if (bad) atomicMin(shared, key);
+    }
+    __syncthreads();
+    return *shared;
+}
 
 template <typename F, int... I>
 __device__ __forceinline__ void sfor_impl(F &&f, std::integer_sequence<int, I...>) {

@@ -233,6 +233,56 @@ def test_fp32_values_without_bf16_parts(which):
         assert np.array_equal(alone.cpu().numpy().view(np.uint32), got[a:b].view(np.uint32))
 
 
+BAD_VALUES = ["v_inf", "v_nan", "v_big", "k_inf", "k_nan", "q_inf", "q_nan"]
+
+
+def _with_bad_value(w, which, row):
+    """The workload with one infinite, NaN or huge element in pass row `row`: in kv head 1's V or K, or in
+    head 1's Q. Returns it and the heads that meet it."""
+    nh, nkv, hd = w["nh"], w["nkv"], w["hd"]
+    q = w["qkv"].clone()
+    value = {"inf": float("inf"), "nan": float("nan"), "big": 3e38}[which[2:]]
+    col = {"v": (2 * nh + nkv + 1) * hd + 5, "k": (2 * nh + 1) * hd + 99, "q": 2 * hd + 77}[which[0]]
+    q[row, col] = value
+    group = nh // nkv
+    return dict(w, qkv=q), range(1, 2) if which[0] == "q" else range(group, 2 * group)
+
+
+@pytest.mark.parametrize("which", BAD_VALUES)
+@pytest.mark.parametrize("nh,nkv", [(24, 4), (10, 2)])
+def test_fp32_rows_that_do_not_see_a_value_keep_their_bits(nh, nkv, which):
+    """A value that takes the plain path changes only the rows and heads that see it: every other output
+    has the bits of the same pass without it, also in the rows just before it."""
+    _say(f"[fp32] rows beside {which}, heads {nh}/{nkv}")
+    w = _fp32(dict(workloads.text_inputs([300, 70], nh, nkv, seed=2), gate=True, theta=1e7))
+    row = 150
+    bad, heads = _with_bad_value(w, which, row)
+    clean, got = (_run(x)[0].view(torch.int32).view(370, nh, 256).clone() for x in (w, bad))
+    sees = torch.zeros(370, nh, dtype=torch.bool, device="cuda")
+    sees[row:(row + 1 if which[0] == "q" else 300), list(heads)] = True
+    assert torch.equal(got[~sees], clean[~sees])
+
+
+@pytest.mark.parametrize("which", BAD_VALUES)
+def test_fp32_bad_values_agree_bitwise_over_item_sizes(which):
+    """A record that holds such a value has the same bits alone (four-wave items), in a pass of eight-wave items,
+    and as the continuation of a cached prefix, whose 16-row groups start elsewhere."""
+    _say(f"[fp32] {which} over item sizes")
+    nh, nkv, n, new = 24, 4, 304, 84
+    w = _fp32(dict(workloads.text_inputs([n] + [257] * 30, nh, nkv, seed=5), gate=True, theta=1e7))
+    w, _ = _with_bad_value(w, which, 250)
+    packed, _ = _run(w)
+    att = TextAttention(nh, nkv, 256, 64, rope_theta=1e7)
+    plan = AttnPlan(np.array([0, n], np.int32))
+    kp, vp = att.planes(plan.kvT, fp32=True)
+    alone, _ = _run(dict(w, qkv=w["qkv"][:n].clone(), pos3=w["pos3"][:n].clone()), plan=plan, k_plane=kp, vt_plane=vp, kvT=plan.kvT)
+    assert torch.equal(alone.view(torch.int32), packed[:n].view(torch.int32))
+    a = n - new
+    part, _ = _run(dict(w, qkv=w["qkv"][a:n].clone(), pos3=w["pos3"][a:n].clone()),
+                   plan=AttnPlan(np.array([0, new], np.int32), np.array([0, n], np.int32)), k_plane=kp, vt_plane=vp, kvT=plan.kvT)
+    assert torch.equal(part.view(torch.int32), packed[a:n].view(torch.int32))
+
+
 @pytest.mark.parametrize("nh,nkv", [(24, 4), (15, 3), (16, 2)])
 def test_fp32_item_sizes_agree_bitwise(nh, nkv):
     """A record gives the same bits in a pass large enough for eight-wave items as in a small pass, whose

@@ -288,11 +288,36 @@ def test_omni_values_without_bf16_parts(nh, nkv, which):
     scale = np.abs(V[np.isfinite(V) & (np.abs(V) < 1e30)]).max() if which != "v_big" else 1.0
     big = np.maximum(np.abs(want[fine]), scale)
     assert (np.abs(got[fine] - want[fine]) / big).max() < 3e-6
-    for r in (0, 2):             # the clean records
+    for r in range(3):
         a, b = cu[r], cu[r + 1]
-        if which in ("v_inf", "v_big"):
-            alone = _attend(Q[:, a:b], K[:, a:b], V[:, a:b], [0, b - a])
-            assert np.array_equal(alone.view(np.uint32), got[a:b].view(np.uint32))
+        alone = _attend(Q[:, a:b], K[:, a:b], V[:, a:b], [0, b - a])
+        assert np.array_equal(alone.view(np.uint32), got[a:b].view(np.uint32))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("which", ["v_inf", "v_nan", "v_big", "k_inf", "k_nan", "q_inf", "q_nan"])
+def test_omni_rows_that_do_not_see_a_value_keep_their_bits(which):
+    """A value that takes the plain path changes only the rows and heads that see it, at every group width and
+    where a small pass splits a group of 8 heads; and its record has the same bits in a large pass."""
+    value = np.float32({"inf": np.inf, "nan": np.nan, "big": 3e38}[which[2:]])
+    for nh, nkv in ((16, 2), (8, 2), (4, 2), (2, 2)):
+        print(f"[omni] rows beside {which}, heads {nh}/{nkv}", flush=True)
+        T, row, group = 180, 101, nh // nkv
+        Q, K, V = _planes(T, nh, nkv, seed=nh)
+        clean = _attend(Q, K, V, [0, T])
+        sees = np.zeros((T, nh, 128), bool)
+        if which[0] == "q":
+            Q[1, row, 77] = value
+            sees[row, 1] = True
+        else:
+            (V if which[0] == "v" else K)[1, row, 99] = value
+            sees[row:, group:] = True
+        got = _attend(Q, K, V, [0, T])
+        sees = sees.reshape(T, -1)
+        assert np.array_equal(got.view(np.uint32)[~sees], clean.view(np.uint32)[~sees])
+        more = [np.concatenate(x, axis=1) for x in zip((Q, K, V), _planes(2400, nh, nkv, seed=9))]
+        packed = _attend(*more, np.concatenate([[0], T + np.arange(0, 2401, 100)]))
+        assert np.array_equal(packed[:T].view(np.uint32), got.view(np.uint32))
 
 
 @pytest.mark.gpu
