@@ -140,72 +140,161 @@ __device__ __forceinline__ float xrow_max(float x) {
     return fmaxf(__uint_as_float(q[0]), __uint_as_float(q[1]));
 }
 
-// The rows of `rows` (a bit each) of a wave in plain FP32, for rows whose Q or a key that they see holds an
-// infinity, a NaN or a magnitude next to FP32's limit (split_bad): one row after the other, a lane per key
-// for the scores and four dims per lane for q and the output.
-__device__ __noinline__ void text_rows_plain(const Params p, unsigned rows, int q_row0, int q_pos0, int k_row0, int k_len, int h, int kh, int32_t *flag) {
-    const int lane = threadIdx.x & 63;
+// The rows of `rows` (a bit each) of a wave's 16 in plain FP32, for rows whose Q or a key that they see holds an
+// infinity, a NaN or a magnitude next to FP32's limit (split_bad): FP32 matrix products of operands
+// straight from the planes, 16 keys at a time from the record's first, so that a row's bits do not depend on
+// the rows beside it. One infinity that all tokens see, 24 / 4 heads: 425 tokens 165 us with the item's first
+// run (57 without it; row by row in vector code 2,170), 2,000 tokens 1.0 ms (13.9).
+//   S^T = K . Q^T      A = 16 keys x 4 dims, B = Q: lane (g, r16) holds dims 16 c + 4 g + e of row r16.
+//   O^T += V^T . P^T   A = dims 64 m + 4 i + e x keys 4 g + v, B = P: O is dims 64 m + 16 g + 4 v + e of row r16.
+__device__ __forceinline__ void text_rows_plain(const Params &p, unsigned rows, int q_row0, int q_pos0, int k_row0, int k_len, int h, int kh, int32_t *flag) {
+    const int lane = threadIdx.x & 63, r16 = lane & 15, g = lane >> 4;
+    const bool mine = (rows >> r16) & 1;
+    const int r = mine ? r16 : __builtin_ctz(rows), t = q_row0 + r;
     const float *kbase = p.k_plane + ((size_t)kh * p.kvT + k_row0) * HD;
     const float *vbase = p.v_plane + ((size_t)kh * p.kvT + k_row0) * HD;
-    for (int r = 0; r < 16; r++) {
-        if (!((rows >> r) & 1)) continue;
-        const int t = q_row0 + r;
-        const float *src = p.qkv + (size_t)t * p.row + (size_t)h * 2 * HD + 4 * lane;
-        f32x4 q = *(const f32x4 *)src;
-        if (p.q_norm) {
-            float ss = q.x * q.x + q.y * q.y + q.z * q.z + q.w * q.w;
-            for (int o = 32; o > 0; o >>= 1) ss += __shfl_xor(ss, o);
-            const float inv = 1.0f / sqrtf(ss / (float)HD + p.eps);
-            const f32x4 w = *(const f32x4 *)(p.q_norm + 4 * lane);
-            for (int e = 0; e < 4; e++) q[e] = q[e] * inv * w[e];
+    const float *src = p.qkv + (size_t)t * p.row + (size_t)h * 2 * HD;
+    f32x4 q[16];
+#pragma unroll
+    for (int c = 0; c < 16; c++) q[c] = *(const f32x4 *)(src + 16 * c + 4 * g);
+    if (p.q_norm) {
+        float ss = 0.f;
+#pragma unroll
+        for (int c = 0; c < 16; c++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) ss += q[c][e] * q[c][e];
+        ss += __shfl_xor(ss, 16);
+        ss += __shfl_xor(ss, 32);
+        const float inv = 1.0f / sqrtf(ss / (float)HD + p.eps);
+#pragma unroll
+        for (int c = 0; c < 16; c++) {
+            const f32x4 w = *(const f32x4 *)(p.q_norm + 16 * c + 4 * g);
+#pragma unroll
+            for (int e = 0; e < 4; e++) q[c][e] = q[c][e] * inv * w[e];
         }
-        if (p.n_rot) {   // dims i (lanes 0-7) and i + 32 (lanes 8-15)
-            for (int e = 0; e < 4; e++) {
-                const float other = __shfl_xor(q[e], 8);
-                if (lane < 16) {
-                    float c, s;
-                    rope_cs_f32(p.pos3, p.inv_freq, t, (4 * lane + e) & 31, &c, &s);
-                    q[e] = lane < 8 ? q[e] * c - other * s : q[e] * c + other * s;
-                }
-            }
-        }
-        const int keys = p.causal ? min(k_len, q_pos0 + r + 1) : k_len;
-        float m = -INFINITY, l = 0.f;
-        f32x4 o = {0.f, 0.f, 0.f, 0.f};
-        for (int kb = 0; kb < keys; kb += 64) {
-            const int key = kb + lane;
-            const float *k = kbase + (size_t)min(key, keys - 1) * HD;
-            float s = 0.f;
-            for (int c = 0; c < 64; c++) {
-                const f32x4 kv = *(const f32x4 *)(k + 4 * c);
-                for (int e = 0; e < 4; e++) s = fmaf(__shfl(q[e], c), kv[e], s);
-            }
-            const float x = key < keys ? s * p.scale : -INFINITY;
-            float mx = x;
-            for (int i = 32; i > 0; i >>= 1) mx = fmaxf(mx, __shfl_xor(mx, i));
-            const float mn = fmaxf(m, mx);
-            const float alpha = m == mn ? 1.f : expf(m - mn);
-            const float pr = x == -INFINITY ? 0.f : expf(x - mn);
-            float rs = pr;
-            for (int i = 32; i > 0; i >>= 1) rs += __shfl_xor(rs, i);
-            m = mn;
-            l = l * alpha + rs;
-            o *= alpha;
-            for (int j = 0; j < 64 && kb + j < keys; j++) {
-                const float pj = __shfl(pr, j);
-                const f32x4 v = *(const f32x4 *)(vbase + (size_t)(kb + j) * HD + 4 * lane);
-                for (int e = 0; e < 4; e++) o[e] = fmaf(pj, v[e], o[e]);
-            }
-        }
-        const float il = l > 0.f ? 1.0f / l : 0.f;
-        f32x4 w;
-        for (int e = 0; e < 4; e++) w[e] = o[e] * il;
-        if (p.gate) {
-            const f32x4 gv = *(const f32x4 *)(src + HD);
-            for (int e = 0; e < 4; e++) w[e] = w[e] * sigmoidf(gv[e]);
-        }
-        store_out4(p.out, (size_t)t * p.nh * HD + (size_t)h * HD + 4 * lane, w, p.out_type, p.f16_lim, flag);
     }
+    if (p.n_rot) {
+#pragma unroll
+        for (int c = 0; c < 2; c++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                float cs, sn;
+                rope_cs_f32(p.pos3, p.inv_freq, t, 16 * c + 4 * g + e, &cs, &sn);
+                const float x0 = q[c][e], x1 = q[c + 2][e];
+                q[c][e] = x0 * cs - x1 * sn;
+                q[c + 2][e] = x1 * cs + x0 * sn;
+            }
+    }
+    const float sl2 = p.scale * 1.4426950408889634f;
+#pragma unroll
+    for (int c = 0; c < 16; c++) q[c] *= sl2;
+    // keys that the lane's row sees, and the most that one of `rows` does
+    const int keys = p.causal ? min(k_len, q_pos0 + r + 1) : k_len;
+    const int last = p.causal ? min(k_len, q_pos0 + 32 - __builtin_clz(rows)) : k_len;
+    f32x4 o[4][4];
+#pragma unroll
+    for (int m = 0; m < 4; m++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) o[m][e] = f32x4{0.f, 0.f, 0.f, 0.f};
+    float m_run = -INFINITY, l_run = 0.f;
+    for (int kb = 0; kb < last; kb += 16) {
+        f32x4 s = {0.f, 0.f, 0.f, 0.f};
+        // every load goes out before the products (the compiler would wait for each)
+        const float *kr = kbase + (size_t)min(kb + r16, k_len - 1) * HD + 4 * g;
+        f32x4 k[16], w[2][4];
+#pragma unroll
+        for (int c = 0; c < 16; c++) k[c] = *(const f32x4 *)(kr + 16 * c);
+        auto load_v = [&](int v) {
+            const float *vr = vbase + (size_t)min(kb + 4 * g + v, k_len - 1) * HD + 4 * r16;
+#pragma unroll
+            for (int m = 0; m < 4; m++) w[v & 1][m] = *(const f32x4 *)(vr + 64 * m);
+        };
+        load_v(0);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int c = 0; c < 16; c++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) s = __builtin_amdgcn_mfma_f32_16x16x4f32(k[c][e], q[c][e], s, 0, 0, 0);
+        // s[v] is the score (exponent of 2) of key kb + 4g + v for row r16
+        float x[4], mx = -INFINITY, rs = 0.f;
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            x[v] = kb + 4 * g + v < keys ? s[v] : -INFINITY;
+            mx = fmaxf(mx, x[v]);
+        }
+        const float mn = fmaxf(m_run, xrow_max(mx));
+        const float alpha = m_run == -INFINITY ? (mn == -INFINITY ? 1.f : 0.f) : __builtin_amdgcn_exp2f(m_run - mn);
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            x[v] = x[v] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(x[v] - mn);
+            rs += x[v];
+        }
+        m_run = mn;
+        l_run = l_run * alpha + rs;
+#pragma unroll
+        for (int m = 0; m < 4; m++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) o[m][e] *= alpha;
+        // infinities and NaN of V stay out of the matrix products, whose other rows may not see their keys
+        bool special = false;
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            if (v < 3) load_v(v + 1);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int m = 0; m < 4; m++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    const float a = w[v & 1][m][e];
+                    const bool fin = isfinite(a);
+                    special |= !fin;
+                    o[m][e] = __builtin_amdgcn_mfma_f32_16x16x4f32(fin ? a : 0.f, x[v], o[m][e], 0, 0, 0);
+                }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if (__any(special)) {
+#pragma unroll 1
+            for (int j = 0; j < 16; j++) {
+                const int from = (j >> 2) * 16 + r16;   // the lane that holds key kb + j of row r16
+                float pj = 0.f;
+#pragma unroll
+                for (int v = 0; v < 4; v++) {
+                    const float y = __shfl(x[v], from);
+                    pj = (j & 3) == v ? y : pj;
+                }
+                const float *vr = vbase + (size_t)min(kb + j, k_len - 1) * HD + 16 * g;
+#pragma unroll
+                for (int m = 0; m < 4; m++)
+#pragma unroll
+                    for (int v = 0; v < 4; v++) {
+                        const f32x4 a = *(const f32x4 *)(vr + 64 * m + 4 * v);
+#pragma unroll
+                        for (int e = 0; e < 4; e++)
+                            if (!isfinite(a[e]) && kb + j < keys) o[m][e][v] = fmaf(pj, a[e], o[m][e][v]);
+                    }
+            }
+        }
+    }
+    float l_row = l_run;
+    l_row += __shfl_xor(l_row, 16);
+    l_row += __shfl_xor(l_row, 32);
+    if (!mine) return;
+    const float il = l_row > 0.f ? 1.0f / l_row : 0.f;
+#pragma unroll
+    for (int m = 0; m < 4; m++)
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            const int d = 64 * m + 16 * g + 4 * v;
+            f32x4 w;
+#pragma unroll
+            for (int e = 0; e < 4; e++) w[e] = o[m][e][v] * il;
+            if (p.gate) {
+                const f32x4 gv = *(const f32x4 *)(src + HD + d);
+#pragma unroll
+                for (int e = 0; e < 4; e++) w[e] = w[e] * sigmoidf(gv[e]);
+            }
+            store_out4(p.out, (size_t)t * p.nh * HD + (size_t)h * HD + d, w, p.out_type, p.f16_lim, flag);
+        }
 }
 
 // Work items are (block, R x 16 rows of it, k heads of a kv group, kv head), the plan's longest-first

@@ -147,47 +147,119 @@ __device__ __forceinline__ float xrow_max(float x) {
     return fmaxf(__uint_as_float(q[0]), __uint_as_float(q[1]));
 }
 
-// The rows of `rows` (a bit each) of a wave in plain FP32 (FP64 sums), for rows whose Q or a key that they see holds
-// an infinity, a NaN or a magnitude whose FP32 sum over a tile could overflow (split_bad: from 2^121): one
-// by one, a lane per key for the scores and two dims per lane for the output. Slow, and only a
-// pass that is not finite (status 2) or next to FP32's limit gets here.
-__device__ __noinline__ void omni_rows_plain(const AttnParams p, unsigned rows, int q_row0, int q_pos0, int k_row0, int k_len, int h, int kh) {
-    const int lane = threadIdx.x & 63;
+// The rows of `rows` (a bit each) of a wave's 16 in plain FP32 with FP64 sums, for rows whose Q or a key that they see
+// holds an infinity, a NaN or a magnitude whose FP32 sum over a tile could overflow (split_bad): FP32 and FP64
+// matrix products of operands straight from the planes, 16 keys at a time from the record's first, so that a
+// row's bits do not depend on the rows beside it. One infinity that all tokens see, 32 / 4 heads: 425 tokens
+// 115 us (row by row in vector code 1,300), 2,000 tokens 0.74 ms (8.7).
+//   S^T = K . Q^T      A = 16 keys x 4 dims, B = Q: lane (g, r16) holds dims 16 c + 4 g + e of row r16.
+//   O^T += V^T . P^T   A = dims 64 m + 4 i + e x keys 4 g + v, B = P: O is dims 64 m + 16 v + 4 g + e of row r16.
+__device__ __forceinline__ void omni_rows_plain(const AttnParams &p, unsigned rows, int q_row0, int q_pos0, int k_row0, int k_len, int h, int kh) {
+    const int lane = threadIdx.x & 63, r16 = lane & 15, g = lane >> 4;
+    const bool mine = (rows >> r16) & 1;
+    const int r = mine ? r16 : __builtin_ctz(rows);
     const float *kbase = p.k_plane + ((size_t)kh * p.kvT + k_row0) * HD;
     const float *vbase = p.v_plane + ((size_t)kh * p.kvT + k_row0) * HD;
-    for (int r = 0; r < BQ; r++) {
-        if (!((rows >> r) & 1)) continue;
-        const float *q = p.q_plane + ((size_t)h * p.T + q_row0 + r) * HD;
-        const int keys = min(k_len, q_pos0 + r + 1);
-        float m = -INFINITY;
-        double l = 0.0, o0 = 0.0, o1 = 0.0;
-        for (int kb = 0; kb < keys; kb += 64) {
-            const int key = kb + lane;
-            const float *k = kbase + (size_t)min(key, keys - 1) * HD;
-            float s = 0.f;
-            for (int d = 0; d < HD; d++) s = fmaf(q[d], k[d], s);
-            const float x = key < keys ? s * p.scale : -INFINITY;
-            float mx = x;
-            for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
-            const float mn = fmaxf(m, mx);
-            const float alpha = m == mn ? 1.f : expf(m - mn);
-            const float pr = x == -INFINITY ? 0.f : expf(x - mn);
-            double rs = (double)pr;
-            for (int o = 32; o > 0; o >>= 1) rs += __shfl_xor(rs, o);
-            m = mn;
-            l = l * (double)alpha + rs;
-            o0 *= (double)alpha;
-            o1 *= (double)alpha;
-            for (int j = 0; j < 64 && kb + j < keys; j++) {
-                const double pj = (double)__shfl(pr, j);
-                const float2 v = *(const float2 *)(vbase + (size_t)(kb + j) * HD + 2 * lane);
-                o0 = fma(pj, (double)v.x, o0);
-                o1 = fma(pj, (double)v.y, o1);
+    const float *qs = p.q_plane + ((size_t)h * p.T + q_row0 + r) * HD + 4 * g;
+    f32x4 q[8];
+#pragma unroll
+    for (int c = 0; c < 8; c++) q[c] = *(const f32x4 *)(qs + 16 * c);
+    // keys that the lane's row sees, and the most that one of `rows` does
+    const int keys = min(k_len, q_pos0 + r + 1), last = min(k_len, q_pos0 + 32 - __builtin_clz(rows));
+    f64x4 o[2][4];
+#pragma unroll
+    for (int m = 0; m < 2; m++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) o[m][e] = f64x4{0.0, 0.0, 0.0, 0.0};
+    float m_run = -INFINITY;
+    double l_run = 0.0;
+    for (int kb = 0; kb < last; kb += 16) {
+        f32x4 s = {0.f, 0.f, 0.f, 0.f};
+        // every load goes out before the products (the compiler would wait for each)
+        const float *kr = kbase + (size_t)min(kb + r16, k_len - 1) * HD + 4 * g;
+        f32x4 k[8], w[4][2];
+#pragma unroll
+        for (int c = 0; c < 8; c++) k[c] = *(const f32x4 *)(kr + 16 * c);
+#pragma unroll
+        for (int v = 0; v < 4; v++)
+#pragma unroll
+            for (int m = 0; m < 2; m++) w[v][m] = *(const f32x4 *)(vbase + (size_t)min(kb + 4 * g + v, k_len - 1) * HD + 4 * r16 + 64 * m);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int c = 0; c < 8; c++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) s = __builtin_amdgcn_mfma_f32_16x16x4f32(k[c][e], q[c][e], s, 0, 0, 0);
+        // s[v] is the score of key kb + 4g + v for row r16
+        float x[4], mx = -INFINITY, rs = 0.f;
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            x[v] = kb + 4 * g + v < keys ? s[v] * p.scale : -INFINITY;
+            mx = fmaxf(mx, x[v]);
+        }
+        const float mn = fmaxf(m_run, xrow_max(mx));
+        const float alpha = m_run == -INFINITY ? (mn == -INFINITY ? 1.f : 0.f) : expf(m_run - mn);
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            x[v] = x[v] == -INFINITY ? 0.f : expf(x[v] - mn);
+            rs += x[v];
+        }
+        m_run = mn;
+        l_run = l_run * (double)alpha + (double)rs;
+#pragma unroll
+        for (int m = 0; m < 2; m++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) o[m][e] *= (double)alpha;
+        // infinities and NaN of V stay out of the matrix products, whose other rows may not see their keys
+        bool special = false;
+#pragma unroll
+        for (int v = 0; v < 4; v++)
+#pragma unroll
+            for (int m = 0; m < 2; m++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    const float a = w[v][m][e];
+                    const bool fin = isfinite(a);
+                    special |= !fin;
+                    o[m][e] = __builtin_amdgcn_mfma_f64_16x16x4f64((double)(fin ? a : 0.f), (double)x[v], o[m][e], 0, 0, 0);
+                }
+        if (__any(special)) {
+#pragma unroll 1
+            for (int j = 0; j < 16; j++) {
+                const int from = (j >> 2) * 16 + r16;   // the lane that holds key kb + j of row r16
+                float pj = 0.f;
+#pragma unroll
+                for (int v = 0; v < 4; v++) {
+                    const float y = __shfl(x[v], from);
+                    pj = (j & 3) == v ? y : pj;
+                }
+                const float *vr = vbase + (size_t)min(kb + j, k_len - 1) * HD + 4 * g;
+#pragma unroll
+                for (int m = 0; m < 2; m++)
+#pragma unroll
+                    for (int v = 0; v < 4; v++) {
+                        const f32x4 a = *(const f32x4 *)(vr + 64 * m + 16 * v);
+#pragma unroll
+                        for (int e = 0; e < 4; e++)
+                            if (!isfinite(a[e]) && kb + j < keys) o[m][e][v] = fma((double)pj, (double)a[e], o[m][e][v]);
+                    }
             }
         }
-        const double il = l > 0.0 ? 1.0 / l : 0.0;
-        *(float2 *)(p.out + (size_t)(q_row0 + r) * p.nh * HD + (size_t)h * HD + 2 * lane) = make_float2((float)(o0 * il), (float)(o1 * il));
     }
+    double l_row = l_run;
+    l_row += __shfl_xor(l_row, 16);
+    l_row += __shfl_xor(l_row, 32);
+    if (!mine) return;
+    const double il = l_row > 0.0 ? 1.0 / l_row : 0.0;
+    float *dst = p.out + (size_t)(q_row0 + r) * p.nh * HD + (size_t)h * HD + 4 * g;
+#pragma unroll
+    for (int m = 0; m < 2; m++)
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            f32x4 w;
+#pragma unroll
+            for (int e = 0; e < 4; e++) w[e] = (float)(o[m][e][v] * il);
+            *(f32x4 *)(dst + 64 * m + 16 * v) = w;
+        }
 }
 
 // Grid: one workgroup per (block, kv head, W heads of its group); wave w is head w of those.
