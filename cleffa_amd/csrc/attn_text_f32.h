@@ -141,7 +141,7 @@ __device__ __forceinline__ float xrow_max(float x) {
 }
 
 // The rows of `rows` (a bit each) of a wave's 16 in plain FP32, for rows whose Q or a key that they see holds an
-// infinity, a NaN or a magnitude next to FP32's limit (split_bad): FP32 matrix products of operands
+// infinity, a NaN or a magnitude from 2^55 on (split_bad): FP32 matrix products of operands
 // straight from the planes, 16 keys at a time from the record's first, so that a row's bits do not depend on
 // the rows beside it. One infinity that all tokens see, 24 / 4 heads: 425 tokens 165 us with the item's first
 // run (57 without it; row by row in vector code 2,170), 2,000 tokens 1.0 ms (13.9).
@@ -382,10 +382,11 @@ __global__ __launch_bounds__(64 * NW) void attn_text_f32_kernel(Params p) {
         // piece e lies 2 NW e keys on, or NW e / 4 chunks: no carry into the bits of the thread's own
         auto dst_k = [&](int e) { return smem + (dk ^ (unsigned)(((2 * NW * e) >> 3 << 2) * 16)) + 2 * NW * e * (2 * HD); };
         auto dst_v = [&](int e) { return smem + (dv ^ (unsigned)((NW / 4 * e) * 16)); };
-        auto put = [&](auto DST) {
+        auto put = [&](auto DST, auto V) {
 #pragma unroll
             for (int e = 0; e < 2; e++) {
                 amax = split32::split_amax(amax, raw[e]);
+                if constexpr (decltype(V)::value) split32::scale_v(raw[e]);
                 const split32::Parts x = split32::split8(raw[e], wt);
                 uint8_t *const dst = DST(e);
                 *(bf16x8 *)dst = x.h;
@@ -400,7 +401,7 @@ __global__ __launch_bounds__(64 * NW) void attn_text_f32_kernel(Params p) {
 #pragma unroll
                     for (int j = 0; j < 8; j++) raw[e][j] = kb + (tid >> 5) + 2 * NW * e < k_len ? raw[e][j] : 0.f;
             }
-            put(dst_k);
+            put(dst_k, std::false_type{});
         };
         auto put_v = [&](int kb) {
             if (kb + BK > whole) {
@@ -413,7 +414,7 @@ __global__ __launch_bounds__(64 * NW) void attn_text_f32_kernel(Params p) {
                     for (int j = 0; j < 8; j++) raw[e][j] = split32::split_bad(raw[e][j]) ? 0.f : raw[e][j];
                 }
             }
-            put(dst_v);
+            put(dst_v, std::true_type{});
         };
 
         load_k(0);
@@ -545,7 +546,7 @@ __global__ __launch_bounds__(64 * NW) void attn_text_f32_kernel(Params p) {
                 const float alpha = __builtin_amdgcn_exp2f(m_run - mn);
 #pragma unroll
                 for (int j = 0; j < 8; j++) {
-                    x[j] = __builtin_amdgcn_exp2f(x[j] - mn);   // a masked key's -inf gives 0
+                    x[j] = split32::P_SCALE * __builtin_amdgcn_exp2f(x[j] - mn);   // a masked key's -inf gives 0
                     rs += x[j];
                 }
                 m_run = mn;
@@ -585,7 +586,7 @@ __global__ __launch_bounds__(64 * NW) void attn_text_f32_kernel(Params p) {
             plain = q_valid && (own || first < (p.causal ? q_pos0 + r16 + 1 : k_len));
         }
         if (q_valid && !plain) {
-            const float il = l_row > 0.f ? 1.0f / l_row : 0.f;
+            const float il = l_row > 0.f ? (1.0f / split32::V_SCALE) / l_row : 0.f;
             const size_t t = (size_t)(q_row0 + r16);
             const size_t obase = t * p.nh * HD + (size_t)h * HD + 8 * g;
             if (p.gate) {   // every gate load goes out before the first store

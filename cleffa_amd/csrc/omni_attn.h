@@ -148,7 +148,7 @@ __device__ __forceinline__ float xrow_max(float x) {
 }
 
 // The rows of `rows` (a bit each) of a wave's 16 in plain FP32 with FP64 sums, for rows whose Q or a key that they see
-// holds an infinity, a NaN or a magnitude whose FP32 sum over a tile could overflow (split_bad): FP32 and FP64
+// holds an infinity, a NaN or a magnitude from 2^55 on (split_bad): FP32 and FP64
 // matrix products of operands straight from the planes, 16 keys at a time from the record's first, so that a
 // row's bits do not depend on the rows beside it. One infinity that all tokens see, 32 / 4 heads: 425 tokens
 // 115 us (row by row in vector code 1,300), 2,000 tokens 0.74 ms (8.7).
@@ -344,6 +344,7 @@ __global__ __launch_bounds__(64 * W, W == 4 ? 2 : 1) void omni_attn_kernel(AttnP
         for (int e = 0; e < NP; e++) {
             const int i = tid + 64 * W * e, d = i & 127, kg = i >> 7;
             amax = split32::split_amax(amax, vr[e]);
+            split32::scale_v(vr[e]);
             put(buf + KV + d * (2 * BK) + ((kg ^ (-(d >> 3) & 3) ^ ((d >> 2) & 1)) * 16), split32::split8(vr[e], wt));
         }
     };
@@ -532,7 +533,7 @@ __global__ __launch_bounds__(64 * W, W == 4 ? 2 : 1) void omni_attn_kernel(AttnP
         float rs = 0.f;
 #pragma unroll
         for (int j = 0; j < 8; j++) {
-            x[j] = __builtin_amdgcn_exp2f(x[j] - mn);   // a masked key's -inf gives 0
+            x[j] = split32::P_SCALE * __builtin_amdgcn_exp2f(x[j] - mn);   // a masked key's -inf gives 0
             rs += x[j];
         }
         m_run = mn;
@@ -588,7 +589,7 @@ __global__ __launch_bounds__(64 * W, W == 4 ? 2 : 1) void omni_attn_kernel(AttnP
         plain = q_valid && (own || first <= qpos);
     }
     if (q_valid && !plain) {
-        const double il = l_row > 0.0 ? 1.0 / l_row : 0.0;
+        const double il = l_row > 0.0 ? (1.0 / split32::V_SCALE) / l_row : 0.0;
         float *dst = p.out + (size_t)(q_row0 + r16) * p.nh * HD + (size_t)h * HD + 8 * g;
 #pragma unroll
         for (int n = 0; n < 8; n++) {

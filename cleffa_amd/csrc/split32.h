@@ -8,10 +8,12 @@
 // is rounded once per 32-deep step, where v_mfma_f32_16x16x4f32 rounds it once per 4. Six bf16
 // products cost 6 / 16 of the FP32 matrix instructions' time (2.5 PFLOP/s against 157 TFLOP/s).
 //
-// The split is exact for finite |x| below bf16's overflow threshold (0x7f7f8000) whose parts stay
-// clear of the subnormals (|x| above about 2^-108; below, an absolute 2^-133 is lost). Larger and infinite
-// values and NaN give infinite or NaN parts, and sums of values next to that threshold are infinite: rows that
-// meet one are left to plain arithmetic (split_bad).
+// The split is exact for finite |x| below bf16's overflow threshold (0x7f7f8000) down to 2^-110; smaller values lose
+// what lies below 2^-133, bf16's smallest subnormal. V and P are split as 2^24 times their value, which every FP32
+// value survives whole (their products go into a sum that may be as small as they are; unscaled, values of
+// 1e-35 came back with an error of 2^-19, and below 2^-134 as zeros; the multiplications cost 1% of C1 in FP32, 3%
+// of a 425-token pass, 2% of Omni's 16,344). Q and K need no scale: what a product of theirs loses is below 2^-133 x
+// 2^55 (LIMIT) = 2^-78 of a score.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <limits.h>
@@ -64,15 +66,15 @@ __device__ __forceinline__ Parts split8(const float (&x)[8], const Weights &w) {
     return {__builtin_bit_cast(bf16x8, h), __builtin_bit_cast(bf16x8, m), __builtin_bit_cast(bf16x8, l)};
 }
 
-// Values that are left to plain arithmetic: infinities, NaN and magnitudes from 2^121 on. Parts are finite up to
-// 0x7f7f8000 (3.39e38), but the sum over a tile's 32 keys, with probabilities up to 1, has to be as well.
+// Values that are left to plain arithmetic: infinities, NaN and magnitudes from 2^55 on. Below, no score overflows
+// (256 products of 2^110), nor does a sum of V: 2^55 x 2^24 x 2^24 (the scales) in each of up to 2^24 keys.
 // A row is computed with plain arithmetic if its own Q or a key that it sees holds such a value, which does
 // not depend on how the pass is cut into items. A kernel therefore
 //   keeps the largest magnitude it splits (split_amax); an item without such values (split_fine) is done;
 //   stages such values of V as zeros in tiles that some row sees in part, so that the rows which do not see
 //     them keep their sums, with that key's zero probability, clear of infinities and NaN;
 //   finds the first key with such a value (first_bad_key) and the rows concerned at an item's end.
-constexpr float LIMIT = 0x1p121f;
+constexpr float LIMIT = 0x1p55f, V_SCALE = 0x1p24f, P_SCALE = 0x1p24f;   // the output's 1 / l divides by V_SCALE, P's is in l
 __device__ __forceinline__ bool split_bad(float x) { return !(fabsf(x) < LIMIT); }
 // Largest magnitude of a running maximum and eight values; a NaN stays. (In asm: with the builtin the
 // compiler kept the values longer and spilled 13 registers of the text kernel.)
@@ -107,6 +109,11 @@ __device__ __forceinline__ int first_bad_key(const float *k, const float *v, int
     }
     __syncthreads();
     return *shared;
+}
+
+__device__ __forceinline__ void scale_v(float (&x)[8]) {
+#pragma unroll
+    for (int j = 0; j < 8; j++) x[j] *= V_SCALE;
 }
 
 template <typename F, int... I>

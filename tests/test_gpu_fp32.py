@@ -233,6 +233,43 @@ def test_fp32_values_without_bf16_parts(which):
         assert np.array_equal(alone.cpu().numpy().view(np.uint32), got[a:b].view(np.uint32))
 
 
+def _every_magnitude(n, seed):
+    """[n][256] f32 of both signs over FP32's whole range, subnormals included: 24-bit values times 2^e."""
+    rng = np.random.default_rng(seed)
+    e = rng.integers(-149, 105, (n, 256))
+    return np.ldexp(rng.integers(1 << 22, 1 << 24, (n, 256)) * rng.choice([-1.0, 1.0], (n, 256)), e).astype(np.float32)
+
+
+def test_fp32_one_key_gives_its_value_back():
+    """A row that sees one key gives that key's V: probability 1, the sum of V's three parts (or, from 2^55
+    on, the plain path). Exact for every magnitude, so the parts lose no bit of any of them."""
+    _say("[fp32] one key")
+    n = 4096
+    V = _every_magnitude(n, 1)
+    qkv = torch.zeros(n, 4 * 256)
+    qkv[:, 3 * 256:] = torch.from_numpy(V)
+    w = dict(qkv=qkv, q_norm=None, k_norm=None, pos3=torch.zeros(n, 3, dtype=torch.int32), nh=1, nkv=1, hd=256, n_rot=0, gate=False,
+             cu_seqlens=np.arange(n + 1, dtype=np.int32))
+    got = _run(w)[0].cpu().numpy()
+    assert np.array_equal(got.view(np.uint32), V.view(np.uint32))
+
+
+def test_fp32_small_probabilities_keep_their_precision():
+    """Probabilities near 2^-124 of a large V beside a likely key whose V is nothing: the output is
+    theirs. Bound: the exponent's FP32 rounding, 2^-24 x 124, three times over, is 2.2e-5."""
+    _say("[fp32] small probabilities")
+    qkv = torch.zeros(64, 4 * 256)
+    rng = np.random.default_rng(2)
+    qkv[:, 0] = 32.0                                                      # Q
+    qkv[1:, 2 * 256] = torch.from_numpy(rng.uniform(-43.2, -42.8, 63))    # K: scores of -86, 2^-124
+    qkv[0, 3 * 256:] = 1e-38
+    qkv[1:, 3 * 256:] = torch.from_numpy(rng.uniform(0.5e10, 1e10, (63, 256)))
+    w = dict(qkv=qkv, q_norm=None, k_norm=None, pos3=torch.zeros(64, 3, dtype=torch.int32), nh=1, nkv=1, hd=256, n_rot=0, gate=False,
+             cu_seqlens=np.array([0, 64], np.int32))
+    got, want = _run(w)[0].cpu().numpy(), oracle_text(w)
+    assert (np.abs(got - want) / np.abs(want)).max() < 2.2e-5
+
+
 BAD_VALUES = ["v_inf", "v_nan", "v_big", "k_inf", "k_nan", "q_inf", "q_nan"]
 
 

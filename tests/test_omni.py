@@ -321,6 +321,35 @@ def test_omni_rows_that_do_not_see_a_value_keep_their_bits(which):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("nh,nkv", [(8, 1), (8, 2), (2, 2)])
+def test_omni_one_key_gives_its_value_back(nh, nkv):
+    """A row that sees one key gives that key's V, exactly, for every magnitude of FP32 (24-bit values times
+    2^e, subnormals included): the three parts of V lose no bit, and the plain path none of the largest."""
+    print(f"[omni] one key {nh}/{nkv}", flush=True)
+    n, rng = 2048, np.random.default_rng(1)
+    V = np.ldexp(rng.integers(1 << 22, 1 << 24, (nkv, n, 128)) * rng.choice([-1.0, 1.0], (nkv, n, 128)),
+                 rng.integers(-149, 105, (nkv, n, 128))).astype(np.float32)
+    Q, K, _ = _planes(n, nh, nkv, seed=4)
+    got = _attend(Q, K, V, np.arange(n + 1)).reshape(n, nh, 128)
+    want = V.transpose(1, 0, 2).repeat(nh // nkv, axis=1)
+    assert np.array_equal(got.view(np.uint32), np.ascontiguousarray(want).view(np.uint32))
+
+
+@pytest.mark.gpu
+def test_omni_small_probabilities_keep_their_precision():
+    """Probabilities near 2^-124 of a large V beside a likely key whose V is nothing: the output is
+    theirs. Bound: the exponent's FP32 rounding, 2^-24 x 124, three times over, is 2.2e-5."""
+    Q, K, V = (np.zeros((1, 64, 128), np.float32) for _ in range(3))
+    rng = np.random.default_rng(2)
+    Q[0, :, 0] = 32.0
+    K[0, 1:, 0] = rng.uniform(-30.5, -30.3, 63)      # scores of -86
+    V[0, 0] = 1e-38
+    V[0, 1:] = rng.uniform(0.5e10, 1e10, (63, 128))
+    got, want = _attend(Q, K, V, [0, 64]), _reference(Q, K, V, [0, 64])
+    assert (np.abs(got - want) / np.abs(want)).max() < 2.2e-5
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("nh,nkv", [(8, 1), (4, 1)])
 @pytest.mark.parametrize("big", [1e36, 1.1e37, 2e37, 1e38, 3.3e38])
 def test_omni_sums_of_large_values_stay_finite(nh, nkv, big):
