@@ -279,7 +279,7 @@ def bench_omni(a):
     peak = PEAK_SPLIT32
     achieved = flops / (core_ms * 1e-3) / 1e12
     print(json.dumps({
-        "metric": "Omni attention TFLOP/s (16,344-token causal record, 32/4 heads, hd 128, FP32 in, FP64 accumulate)",
+        "metric": "Omni attention TFLOP/s (16,344-token causal record, 32/4 heads, hd 128, FP32 in, FP64 sums across 32-key tiles)",
         "value": round(flops / (ms * 1e-3) / 1e12, 2), "unit": "TFLOP/s",
         "tokens_per_s": round(T / (ms * 1e-3), 1), "n_gpus": 1, "steps": a.steps, "warmup": a.warmup,
         "ms_per_step": round(ms, 5), "host_ms_per_step": round(wall_ms, 5), "higher_is_better": True,

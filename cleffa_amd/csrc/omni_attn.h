@@ -1,16 +1,16 @@
 // Omni decoder attention for head dim 128 on CDNA4: FP32 operands, causal within each packed
-// record, ungated, with the output accumulated in FP64 (metal/clef.metal:2055-2319:
-// omni_attn_prep, omni_attention).
+// record, ungated (metal/clef.metal:2055-2319: omni_attn_prep, omni_attention).
 //
 // The reference keeps the P.V accumulator as an FP32 hi/lo pair so that thousands of updates
-// do not round into one component. Here the P.V accumulators are FP64.
+// do not round into one component. Here the P.V sums are FP32 within a tile of 32 keys and FP64 across tiles.
 //
 // Both products run on the bf16 matrix cores with every FP32 operand split into three bf16 parts
 // and six products per pair (split32.h). Bounds of the item loop, per 32-key tile and SIMD: 192
 // matrix instructions of 16 cycles against 128 FP32 ones of 32 cycles and 128 FP64 ones of 64 for
 // the same work before. At 16,344 tokens, 32 / 4 heads: 27.9 -> 10.7 ms, 53% of the cycles on the matrix cores at
 // 2.1 GHz; relative error against float64 3.2e-7 -> 1.8e-7 (most of it the FP32 output's
-// rounding: the scores take 8 full-size roundings instead of 32).
+// rounding: the scores take 5 full-size roundings instead of 32). Where the scores do not matter, the FP32 sums
+// within a tile show: constant V over 200 random scores comes back within 0.5 x 2^-24 rms, with FP64 products 0.2.
 //
 // Workgroup: one wave per q head of a GQA group (nh / nkv waves), all on the same 16 query
 // rows of one record, so one 32-key K/V tile in LDS serves the whole group.

@@ -1,11 +1,12 @@
 // FP32 products on the bf16 matrix cores of CDNA4 (gfx950).
 //
 // An FP32 value is the exact sum of three bf16 values: h = bf16(x), m = bf16(x - h),
-// l = bf16(x - h - m), each rounded to nearest even, so |m| <= 2^-9 |x| and |l| <= 2^-18 |x|. A product a . b then
-// takes the six terms hh, hm, mh, hl, lh, mm; the three left out (ml, lm, ll) are at most 2^-26 |a b| together, below the
-// rounding of one FP32 product (2^-24 |a b|). The terms run on v_mfma_f32_16x16x32_bf16 with FP32
+// l = bf16(x - h - m), each rounded to nearest even, so |m| <= 2^-8 |x| and |l| <= 2^-17 |x|. A product a . b then
+// takes the six terms hh, hm, mh, hl, lh, mm; the three left out (ml, lm, ll) are at most 2^-24 |a b| together, the
+// rounding of one FP32 product (2^-27 |a b| root mean square over random operands). The terms run on v_mfma_f32_16x16x32_bf16 with FP32
 // accumulation, the small ones first or into accumulators of their own, so that the full-size sum
-// is rounded once per 32-deep step, where v_mfma_f32_16x16x4f32 rounds it once per 4. Six bf16
+// is rounded once per 32-deep step, where v_mfma_f32_16x16x4f32 rounds it once per 4: the score of 256 equal operands
+// 0x1.00ff8p+0, whose left-out terms all have one sign, is off by 0.1 x 2^-24, with the FP32 instruction by 16. Six bf16
 // products cost 6 / 16 of the FP32 matrix instructions' time (2.5 PFLOP/s against 157 TFLOP/s).
 //
 // The split is exact for finite |x| below bf16's overflow threshold (0x7f7f8000) down to 2^-110; smaller values lose
@@ -35,7 +36,8 @@ struct Parts {
 
 // x - h of one element of a packed pair: v_dot2_f32_bf16 with weights (-1, 0) or (0, -1), one instruction
 // for the widening and the subtraction. The difference is exact, so the instruction's own rounding does not
-// enter (checked over the exponent range against the two-instruction form). The weights sit in
+// enter (a value that passes through the attention kernels alone comes back bit for bit, over all exponents:
+// tests/test_gpu_fp32.py). The weights sit in
 // registers the compiler cannot see through: as constants it encoded (-1, 0) wrongly.
 struct Weights {
     unsigned lo, hi;

@@ -1,4 +1,4 @@
-"""Omni decoder attention (hd 128, FP32 operands, FP64-accumulated output) through the C ABI:
+"""Omni decoder attention (hd 128, FP32 operands; sums in FP32 within 32 keys, FP64 across) through the C ABI:
 the host side of clef_omni_encode_attention (clef_metal_omni.m:200-245) between the QKV GEMM
 and o_proj. torch provides device memory and the stream; the compute is libclef_hip_attn.so."""
 import ctypes

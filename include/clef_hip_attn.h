@@ -145,11 +145,15 @@ typedef struct {
                                  CLEF_HIP_QKV_F32 (1): the FP32 path (clef_metal.m:1330-1413,
                                  attn_prep + attention_prefetch_64 and kin): f32 rows, f32 K and V
                                  planes, FP32 products and softmax, for the per-record rerun after
-                                 an overflow (clef.c:526-550) and CLEF_ATTN_TU=0 (the products run
-                                 as six bf16 products of operands split exactly in three, at the
-                                 error of FP32 ones or below). In FP32 mode any nh / nkv works,
-                                 sched and trace are ignored, and only the output (f16
-                                 out_type) can flag. Other values are rejected */
+                                 an overflow (clef.c:526-550) and CLEF_ATTN_TU=0. The products run
+                                 as six bf16 products of operands split exactly in three; what
+                                 they leave out is at most 2^-24 of a product, one FP32 rounding,
+                                 and the sums take fewer roundings: measured against float64,
+                                 errors are below those of the FP32 matrix instructions on random
+                                 data and on equal operands. Rows that see an infinity, a NaN or
+                                 a magnitude from 2^55 on run on those instructions. In FP32 mode
+                                 any nh / nkv works, sched and trace are ignored, and only the
+                                 output (f16 out_type) can flag. Other values are rejected */
     const int32_t *tok_kv;    /* [T] device int32: the plan's pass row -> plane row map (the inverse
                                  of kv_tok); the bf16 K/V prologue runs over pass rows with it */
 } clef_hip_attn_args;
@@ -313,7 +317,8 @@ bool clef_hip_gguf_vis_layer(const clef_hip_gguf *g, int layer, int heads, uint1
 
 /* ---- Omni decoder attention (metal/clef.metal:2055-2319 omni_attn_prep / omni_attention, host
  * clef_metal_omni.m:200-245 clef_omni_encode_attention). FP32 operands, hd 128, causal within
- * each record, no gate; the output is accumulated in FP64 (the reference: FP32 hi/lo pairs).
+ * each record, no gate; the output is accumulated in FP32 within a tile of 32 keys and in FP64
+ * across tiles (the reference: FP32 hi/lo pairs), so that long records round no more than short ones.
  *
  * clef_hip_omni_rope_table: the 192-float rotary table of the reference (clef_metal.m:172-180):
  * [0, 64) 1 / theta^(2j/128) in FP32, [64, 128) and [128, 192) the FP64 theta^(-2j/128) as an

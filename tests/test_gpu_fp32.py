@@ -233,6 +233,36 @@ def test_fp32_values_without_bf16_parts(which):
         assert np.array_equal(alone.cpu().numpy().view(np.uint32), got[a:b].view(np.uint32))
 
 
+# Equal operands whose parts the products leave out (m l) all have one sign: 2^-24 of each product at 0x1.00ff8p+0.
+# Below 1.16, so that e^(-64 x^2), which the test reads the scores from, is a normal FP32 number.
+REPEATED = np.array([float.fromhex("0x1.00ff8p+0"), float.fromhex("0x1.00ff7ep+0"), float.fromhex("0x1.01017ep+0"), 1.1, 1.15], np.float32)
+
+
+def test_fp32_repeated_operands():
+    """Products whose rounding errors add up. Scores: key 0's, 4 x^2 256 / 16, against a key of score 0,
+    whose V alone is not zero: the output's relative error is the score's. Bound on that of the score: 8 steps
+    and their sum's roundings, the left-out terms, Q's scale and its product, 12 x 2^-24 of it (the
+    FP32 matrix instructions' 64 steps gave 16). P . V: constant V over 32 keys, one tile: 6 roundings at full size,
+    the left-out terms, 12 of the sum of P and the output's, 20 x 2^-24."""
+    _say("[fp32] repeated operands")
+    n = len(REPEATED)
+    x = torch.from_numpy(REPEATED).repeat_interleave(2)[:, None]
+    qkv = torch.zeros(2 * n, 4 * 256)
+    qkv[:, :256] = 4 * x
+    qkv[0::2, 512:768] = x[0::2]
+    qkv[1::2, 768:] = 1
+    w = dict(qkv=qkv, q_norm=None, k_norm=None, pos3=torch.zeros(2 * n, 3, dtype=torch.int32), nh=1, nkv=1, hd=256, n_rot=0, gate=False,
+             cu_seqlens=np.arange(0, 2 * n + 1, 2, dtype=np.int32))
+    o = _run(w)[0].cpu().numpy()[1::2].astype(np.float64)
+    s = 4 * REPEATED.astype(np.float64)[:, None] ** 2 * 16
+    assert (np.abs(np.log(1 / o - 1) - s) / s).max() < 12 * 2.0 ** -24
+    qkv = torch.randn(32 * n, 4 * 256, generator=torch.Generator().manual_seed(3))
+    qkv[:, 768:] = torch.from_numpy(REPEATED).repeat_interleave(32)[:, None]
+    w = dict(w, qkv=qkv, pos3=torch.zeros(32 * n, 3, dtype=torch.int32), cu_seqlens=np.arange(0, 32 * n + 1, 32, dtype=np.int32))
+    v = qkv[:, 768:].numpy().astype(np.float64)
+    assert (np.abs(_run(w)[0].cpu().numpy() - v) / v).max() < 20 * 2.0 ** -24
+
+
 def _every_magnitude(n, seed):
     """[n][256] f32 of both signs over FP32's whole range, subnormals included: 24-bit values times 2^e."""
     rng = np.random.default_rng(seed)

@@ -248,8 +248,8 @@ def _reference(Q, K, V, cu):
 @pytest.mark.parametrize("nh,nkv", [(8, 1), (8, 2), (6, 3), (3, 3)])
 def test_omni_group_widths_and_tile_edges(nh, nkv):
     """Every group width (8, 4, 2, 1 heads) over records that end on, before and after 32-key
-    tiles. Bound: the scores' FP32 rounding (|s| up to ~40 in exponents of 2, 8 roundings of 2^-24
-    each: 2e-5 of P at most, averaged over keys) leaves outputs of size ~1 within 3e-6, as the
+    tiles. Bound: the scores' FP32 rounding (|s| up to ~40 in exponents of 2, 5 roundings of 2^-24
+    each: 1.2e-5 of P at most, averaged over keys) leaves outputs of size ~1 within 3e-6, as the
     reference's tests ask."""
     print(f"[omni] widths {nh}/{nkv}", flush=True)
     lens = [1, 16, 17, 31, 32, 33, 48, 63, 64, 65, 95, 96, 97, 130, 257]
@@ -318,6 +318,28 @@ def test_omni_rows_that_do_not_see_a_value_keep_their_bits(which):
         more = [np.concatenate(x, axis=1) for x in zip((Q, K, V), _planes(2400, nh, nkv, seed=9))]
         packed = _attend(*more, np.concatenate([[0], T + np.arange(0, 2401, 100)]))
         assert np.array_equal(packed[:T].view(np.uint32), got.view(np.uint32))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nh,nkv", [(8, 1), (4, 1), (1, 1)])
+def test_omni_repeated_operands(nh, nkv):
+    """Products whose rounding errors add up: equal operands, whose left-out parts all have one sign (2^-24 of
+    each product at 0x1.00ff8p+0). Scores: key 0's, 4 x^2 128 / sqrt(128), against a key of score 0, whose V
+    alone is not zero: the output's relative error is the score's; 4 steps and their sum's roundings, the
+    left-out terms, Q's scale and its product: 8 x 2^-24. P . V: constant V over 200 keys: 6 FP32 roundings of
+    a tile's sum, its left-out terms, 12 of the sum of P, the output's: 20 x 2^-24."""
+    for x in (float.fromhex("0x1.00ff8p+0"), float.fromhex("0x1.00ff7ep+0"), float.fromhex("0x1.01017ep+0"), 1.1, 1.3):
+        x = np.float32(x)
+        print(f"[omni] repeated {x!r} {nh}/{nkv}", flush=True)
+        Q, K, V = np.full((nh, 2, 128), 4 * x, np.float32), np.full((nkv, 2, 128), x, np.float32), np.ones((nkv, 2, 128), np.float32)
+        K[:, 1] = 0
+        V[:, 0] = 0
+        o = _attend(Q, K, V, [0, 2])[1].astype(np.float64)
+        s = 4 * float(x) ** 2 * 128 ** 0.5
+        assert (np.abs(np.log(1 / o - 1) - s) / s).max() < 8 * 2.0 ** -24
+        Q, K, V = _planes(200, nh, nkv, seed=7)
+        V[:] = x
+        assert (np.abs(_attend(Q, K, V, [0, 200]) - float(x)) / x).max() < 20 * 2.0 ** -24
 
 
 @pytest.mark.gpu
