@@ -593,15 +593,19 @@ bool clef_hip_qkv_gemm(int H, const uint16_t *X, const uint16_t *W, const clef_h
     //             The three narrower than 256 columns hold no whole head, so the prologue follows as a
     //             launch (in these times).
     //   256 x 256, its last round as halves (226 at T = 1300 with the layer's attention, 250 without): where
-    //             that round fills at most half of the CUs (qkv_gemm_halved_kernel).
+    //             that round fills at most half of the CUs (qkv_gemm_halved_kernel). Exactly half full behind
+    //             two rounds or more, its halves' K / V prologues are a full round's, and a shorter K no longer pays for
+    //             them (T = 4096, whole against halves: 10240 x 2560 209 / 217, 18432 x 2560 347 / 362, 14336 x
+    //             5120 518 / 514).
     // Each element's sum runs over k in the same order in all of them: the bits do not depend on the tile.
     auto rounds = [&](int bm, int bn) {
         const long n_per_xcd = (N / bn + 7) / 8, m = (a->T + bm - 1) / bm;
         return (m * n_per_xcd + 31) / 32;
     };
     const int most = (int)((N / 256 + 7) / 8 * ((a->T + 255L) / 256)), whole = gemm::whole_tiles(most);   // 256 x 256 tiles of an XCD
+    const bool even = p.kv && most % gemm::XCD_CUS == gemm::XCD_CUS / 2 && whole > gemm::XCD_CUS && H < 5120;
     const long cost[6] = {100 * rounds(256, 256), 63 * rounds(128, 256), 38 * rounds(128, 64), 33 * rounds(64, 64), 48 * rounds(128, 128),
-                          whole == most ? LONG_MAX : 100L * (whole / gemm::XCD_CUS) + 63};
+                          whole == most || even ? LONG_MAX : 100L * (whole / gemm::XCD_CUS) + 63};
     const int best = (int)(std::min_element(cost, cost + 6) - cost);
     const bool kv = p.kv;
     if (best >= 2 && best != 5) p.kv = 0;
