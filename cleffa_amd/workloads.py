@@ -1,4 +1,4 @@
-"""Seeded synthetic workloads for the prefill attention path (the BASELINE configurations).
+"""Seeded synthetic workloads for the prefill attention path (the benchmark's configurations).
 
 C0  one causal sequence of 1,024 tokens, 16/4 heads, hd 256, plain SDPA operands (no norm,
     no rotary, no gate), Q/K/V ~ N(0,1) rounded to bf16.
@@ -10,7 +10,7 @@ C3  prefix-cache continuation: 4 records x (2,048 cached K/V rows + 512 new quer
     positions 2,048..2,559), 16/4 heads, hd 256.
 C4  vision: 4 images x 1,024 patches (32x32 grid), bidirectional, 16 heads, hd 72, 2-D rotary.
 S   a batch of short records: 256 records x 16 tokens (4,096 tokens), 24/4 heads, hd 256, C1's
-    prologue and gate (not a BASELINE configuration: the serving case of many short prompts).
+    prologue and gate (the serving case of many short prompts).
 
 Record lengths come from a numpy PCG64 stream so they are identical on every machine; the
 tensor values come from a torch generator on the target device.
@@ -98,7 +98,7 @@ def text_inputs(lengths, nh, nkv, hd=256, n_rot=64, seed=0, device="cpu", norm=T
 
 
 def config(name, seed=0, device="cpu"):
-    """Inputs of one BASELINE configuration."""
+    """Inputs of one configuration."""
     if name == "C0":
         w = text_inputs([1024], 16, 4, n_rot=0, seed=seed, device=device, norm=False, outlier_frac=0)
         w.update(gate=False, theta=1e7)

@@ -5,7 +5,7 @@ import torch
 from cleffa_amd import AttnPlan, TextAttention, VisionAttention, rope_inv_freq
 from oracle import oracle
 
-# north_star tolerance on bf16 outputs against the oracle (fp64 here, stricter than fp32)
+# tolerance on bf16 outputs against the oracle (fp64 here, stricter than fp32)
 MAX_ABS = 2e-2
 MEAN_ABS = 2e-3
 

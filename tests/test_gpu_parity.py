@@ -1,4 +1,4 @@
-"""HIP path vs the float64 CPU oracle on the BASELINE configurations (bf16 outputs, north_star
+"""HIP path vs the float64 CPU oracle on the benchmark's configurations (bf16 outputs,
 tolerance max-abs 2e-2 / mean-abs 2e-3), through the C ABI (libclef_hip_attn.so)."""
 import numpy as np
 import pytest

@@ -162,7 +162,7 @@ def test_rows_do_not_depend_on_the_pass_size(nh, nkv, H):
 def test_halved_last_round(nh, nkv, T):
     """Passes whose last round of 256 x 256 tiles is at most half full run it as 128-row tiles (three to
     sixteen tiles of an XCD, XCDs that own a tile less, a last half past the rows): each row's projection and planes
-    have the bits of a pass of 60 rows, which takes 64-column tiles."""
+    have the bits of a pass of 60 rows, which takes 64-column tiles (128 at 60 / 4 heads)."""
     q_norm, k_norm, pos3, cu = _plan_inputs([T], nh, 8)
     X, W = _operands(T, 128, nh, nkv, 9)
     att = TextAttention(nh, nkv, 256, 64)

@@ -1,4 +1,4 @@
-"""Synthetic BASELINE workloads: shapes and the C1 length draw."""
+"""Synthetic workloads: shapes and the C1 length draw."""
 import numpy as np
 
 from cleffa_amd import workloads
