@@ -56,11 +56,17 @@ def _device(device):
     return d
 
 
+# torch's own shortcut to the current stream's handle; not part of its public interface
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _stream_handle(stream):
-    """The stream's handle, of the current device's current stream for None (read directly: building a
-    torch.cuda.Stream around it took 3 us of a 24 us call)."""
+    """The stream's handle, of the current device's current stream for None (read directly where torch has
+    that: building a torch.cuda.Stream around it took 3 us of a 24 us call)."""
     if stream is None:
-        return ctypes.c_void_p(torch._C._cuda_getCurrentRawStream(torch.cuda.current_device()))
+        if _raw_stream is not None:
+            return ctypes.c_void_p(_raw_stream(torch.cuda.current_device()))
+        stream = torch.cuda.current_stream()
     return ctypes.c_void_p(stream.cuda_stream)
 
 

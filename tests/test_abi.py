@@ -79,3 +79,17 @@ def test_null_args_and_small_error_buffer():
     err = ctypes.create_string_buffer(8)
     assert not lib.clef_hip_attn_core(None, None, err, len(err))
     assert err.value.decode() == "hip: nu"
+
+
+def test_current_stream_without_torchs_shortcut(monkeypatch):
+    """Calls go to the current device's current stream also with a torch that lacks the private shortcut."""
+    from types import SimpleNamespace
+
+    from cleffa_amd import attention
+    monkeypatch.setattr(attention.torch.cuda, "current_device", lambda: 3)
+    monkeypatch.setattr(attention, "_raw_stream", lambda device: 0x1000 + device)
+    assert attention._stream_handle(None).value == 0x1003
+    monkeypatch.setattr(attention, "_raw_stream", None)
+    monkeypatch.setattr(attention.torch.cuda, "current_stream", lambda: SimpleNamespace(cuda_stream=0x2003))
+    assert attention._stream_handle(None).value == 0x2003
+    assert attention._stream_handle(SimpleNamespace(cuda_stream=0x3000)).value == 0x3000
