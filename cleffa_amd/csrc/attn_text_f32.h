@@ -325,299 +325,296 @@ __global__ __launch_bounds__(64 * NW) void attn_text_f32_kernel(Params p) {
     for (int w = 0; w < 2; w++)
         va[w] = lds0 + KV + (8 * (r16 >> 2) + 4 * w + (r16 & 3)) * (2 * BK) + ((g ^ (-(r16 >> 2) & 3) ^ w) * 16);
 
-    {
-        const int item = blockIdx.x;
-        const int kh = item % p.nkv, ic = item / p.nkv % n_ch, ib = item / p.nkv / n_ch;
-        const int32_t *blk = p.blocks + 8 * (ib / n_sub);
-        const int r0 = span * (n_sub - 1 - ib % n_sub), rows = min(span, blk[1] - r0);
-        if (rows <= 0) return;
-        const int kk = f32_heads(p.slots, rows, group), wph = (rows + 15) / 16;
-        if (ic * kk >= group) return;
-        const int slot = wave / wph;
-        const bool live = slot < kk;
-        const int h = kh * group + ic * kk + (live ? slot : 0);
-        const int q_row0 = blk[0] + r0 + (live ? 16 * (wave - slot * wph) : 0), q_pos0 = blk[2] + q_row0 - blk[0];
-        const int nq = live ? min(16, blk[0] + r0 + rows - q_row0) : 0;
-        const int k_row0 = blk[3], k_len = p.causal ? min(blk[4], blk[2] + r0 + rows) : blk[4];
-        const int whole = p.causal ? min(k_len, blk[2] + r0 + 1) : k_len;   // keys that every row of the item sees
-        int32_t *const flag = p.ovf ? p.ovf + blk[5] : nullptr;
-        const int n_tiles = (k_len + BK - 1) / BK;
-        // keys this wave's rows see, and the tiles it runs
-        const int my_len = live ? (p.causal ? min(k_len, q_pos0 + nq) : k_len) : 0;
-        const bool q_valid = r16 < nq;
-        const float *const kbase = p.k_plane + ((size_t)kh * p.kvT + k_row0) * HD;
-        const float *const vbase = p.v_plane + ((size_t)kh * p.kvT + k_row0) * HD;
-        float amax = 0.f;
+    const int item = blockIdx.x;
+    const int kh = item % p.nkv, ic = item / p.nkv % n_ch, ib = item / p.nkv / n_ch;
+    const int32_t *blk = p.blocks + 8 * (ib / n_sub);
+    const int r0 = span * (n_sub - 1 - ib % n_sub), rows = min(span, blk[1] - r0);
+    if (rows <= 0) return;
+    const int kk = f32_heads(p.slots, rows, group), wph = (rows + 15) / 16;
+    if (ic * kk >= group) return;
+    const int slot = wave / wph;
+    const bool live = slot < kk;
+    const int h = kh * group + ic * kk + (live ? slot : 0);
+    const int q_row0 = blk[0] + r0 + (live ? 16 * (wave - slot * wph) : 0), q_pos0 = blk[2] + q_row0 - blk[0];
+    const int nq = live ? min(16, blk[0] + r0 + rows - q_row0) : 0;
+    const int k_row0 = blk[3], k_len = p.causal ? min(blk[4], blk[2] + r0 + rows) : blk[4];
+    const int whole = p.causal ? min(k_len, blk[2] + r0 + 1) : k_len;   // keys that every row of the item sees
+    int32_t *const flag = p.ovf ? p.ovf + blk[5] : nullptr;
+    const int n_tiles = (k_len + BK - 1) / BK;
+    // keys this wave's rows see, and the tiles it runs
+    const int my_len = live ? (p.causal ? min(k_len, q_pos0 + nq) : k_len) : 0;
+    const bool q_valid = r16 < nq;
+    const float *const kbase = p.k_plane + ((size_t)kh * p.kvT + k_row0) * HD;
+    const float *const vbase = p.v_plane + ((size_t)kh * p.kvT + k_row0) * HD;
+    float amax = 0.f;
 
-        // ---- tile staging, two pieces a thread. Piece e: K dims 8 c .. 8 c + 7
-        // of one key, V keys 8 kg .. 8 kg + 7 of one dim; each load is a uniform base plus a
-        // 32-bit lane offset. Keys past the item's range become zeros: their zero probabilities
-        // then give zero products, and what lies there cannot flag the item. So do values of V that
-        // are left to plain arithmetic, in tiles that some row sees in part.
-        float raw[2][8];
-        const unsigned ko = 32u * tid, vo = (tid >> 8) * (8u * HD * 4u) + (tid & 255) * 4u;
-        auto load_k = [&](int kb) {
+    // ---- tile staging, two pieces a thread. Piece e: K dims 8 c .. 8 c + 7
+    // of one key, V keys 8 kg .. 8 kg + 7 of one dim; each load is a uniform base plus a
+    // 32-bit lane offset. Keys past the item's range become zeros: their zero probabilities
+    // then give zero products, and what lies there cannot flag the item. So do values of V that
+    // are left to plain arithmetic, in tiles that some row sees in part.
+    float raw[2][8];
+    const unsigned ko = 32u * tid, vo = (tid >> 8) * (8u * HD * 4u) + (tid & 255) * 4u;
+    auto load_k = [&](int kb) {
 #pragma unroll
-            for (int e = 0; e < 2; e++) {
-                const char *s = (const char *)(kbase + (size_t)(kb + 2 * NW * e) * HD);
-                const f32x4 a = *(const f32x4 *)(s + ko), b = *(const f32x4 *)(s + ko + 16);
+        for (int e = 0; e < 2; e++) {
+            const char *s = (const char *)(kbase + (size_t)(kb + 2 * NW * e) * HD);
+            const f32x4 a = *(const f32x4 *)(s + ko), b = *(const f32x4 *)(s + ko + 16);
 #pragma unroll
-                for (int j = 0; j < 4; j++) { raw[e][j] = a[j]; raw[e][4 + j] = b[j]; }
+            for (int j = 0; j < 4; j++) { raw[e][j] = a[j]; raw[e][4 + j] = b[j]; }
+        }
+    };
+    auto load_v = [&](int kb) {
+#pragma unroll
+        for (int e = 0; e < 2; e++)
+#pragma unroll
+            for (int j = 0; j < 8; j++) {
+                const char *s = (const char *)(vbase + (size_t)(kb + 2 * NW * e + j) * HD);
+                raw[e][j] = *(const float *)(s + vo);
             }
-        };
-        auto load_v = [&](int kb) {
+    };
+    // K chunk c of key 8a + 4t + b sits at position c ^ (4a + b), V^T chunk kg of dim d at
+    // kg ^ (-(d / 8) % 4) ^ ((d / 4) % 2): the lanes one step of a read or write serves hit
+    // distinct 16-byte slots.
+    const unsigned dk = (tid >> 5) * (2 * HD) + (((tid & 31) ^ (((tid >> 5) & 3) | (((tid >> 5) >> 3) << 2))) * 16);
+    const unsigned dv = KV + (tid & 255) * (2 * BK) + (((tid >> 8) ^ (-((tid & 255) >> 3) & 3) ^ ((tid >> 2) & 1)) * 16);
+    // piece e lies 2 NW e keys on, or NW e / 4 chunks: no carry into the bits of the thread's own
+    auto dst_k = [&](int e) { return smem + (dk ^ (unsigned)(((2 * NW * e) >> 3 << 2) * 16)) + 2 * NW * e * (2 * HD); };
+    auto dst_v = [&](int e) { return smem + (dv ^ (unsigned)((NW / 4 * e) * 16)); };
+    auto put = [&](auto DST, auto V) {
+#pragma unroll
+        for (int e = 0; e < 2; e++) {
+            amax = split32::split_amax(amax, raw[e]);
+            if constexpr (decltype(V)::value) split32::scale_v(raw[e]);
+            const split32::Parts x = split32::split8(raw[e], wt);
+            uint8_t *const dst = DST(e);
+            *(bf16x8 *)dst = x.h;
+            *(bf16x8 *)(dst + PL) = x.m;
+            *(bf16x8 *)(dst + 2 * PL) = x.l;
+        }
+    };
+    auto put_k = [&](int kb) {
+        if (kb + BK > k_len) {
 #pragma unroll
             for (int e = 0; e < 2; e++)
 #pragma unroll
-                for (int j = 0; j < 8; j++) {
-                    const char *s = (const char *)(vbase + (size_t)(kb + 2 * NW * e + j) * HD);
-                    raw[e][j] = *(const float *)(s + vo);
-                }
-        };
-        // K chunk c of key 8a + 4t + b sits at position c ^ (4a + b), V^T chunk kg of dim d at
-        // kg ^ (-(d / 8) % 4) ^ ((d / 4) % 2): the lanes one step of a read or write serves hit
-        // distinct 16-byte slots.
-        const unsigned dk = (tid >> 5) * (2 * HD) + (((tid & 31) ^ (((tid >> 5) & 3) | (((tid >> 5) >> 3) << 2))) * 16);
-        const unsigned dv = KV + (tid & 255) * (2 * BK) + (((tid >> 8) ^ (-((tid & 255) >> 3) & 3) ^ ((tid >> 2) & 1)) * 16);
-        // piece e lies 2 NW e keys on, or NW e / 4 chunks: no carry into the bits of the thread's own
-        auto dst_k = [&](int e) { return smem + (dk ^ (unsigned)(((2 * NW * e) >> 3 << 2) * 16)) + 2 * NW * e * (2 * HD); };
-        auto dst_v = [&](int e) { return smem + (dv ^ (unsigned)((NW / 4 * e) * 16)); };
-        auto put = [&](auto DST, auto V) {
+                for (int j = 0; j < 8; j++) raw[e][j] = kb + (tid >> 5) + 2 * NW * e < k_len ? raw[e][j] : 0.f;
+        }
+        put(dst_k, std::false_type{});
+    };
+    auto put_v = [&](int kb) {
+        if (kb + BK > whole) {
 #pragma unroll
             for (int e = 0; e < 2; e++) {
+#pragma unroll
+                for (int j = 0; j < 8; j++) raw[e][j] = kb + 8 * (tid >> 8) + 2 * NW * e + j < k_len ? raw[e][j] : 0.f;
                 amax = split32::split_amax(amax, raw[e]);
-                if constexpr (decltype(V)::value) split32::scale_v(raw[e]);
-                const split32::Parts x = split32::split8(raw[e], wt);
-                uint8_t *const dst = DST(e);
-                *(bf16x8 *)dst = x.h;
-                *(bf16x8 *)(dst + PL) = x.m;
-                *(bf16x8 *)(dst + 2 * PL) = x.l;
+#pragma unroll
+                for (int j = 0; j < 8; j++) raw[e][j] = split32::split_bad(raw[e][j]) ? 0.f : raw[e][j];
             }
-        };
-        auto put_k = [&](int kb) {
-            if (kb + BK > k_len) {
-#pragma unroll
-                for (int e = 0; e < 2; e++)
-#pragma unroll
-                    for (int j = 0; j < 8; j++) raw[e][j] = kb + (tid >> 5) + 2 * NW * e < k_len ? raw[e][j] : 0.f;
-            }
-            put(dst_k, std::false_type{});
-        };
-        auto put_v = [&](int kb) {
-            if (kb + BK > whole) {
-#pragma unroll
-                for (int e = 0; e < 2; e++) {
-#pragma unroll
-                    for (int j = 0; j < 8; j++) raw[e][j] = kb + 8 * (tid >> 8) + 2 * NW * e + j < k_len ? raw[e][j] : 0.f;
-                    amax = split32::split_amax(amax, raw[e]);
-#pragma unroll
-                    for (int j = 0; j < 8; j++) raw[e][j] = split32::split_bad(raw[e][j]) ? 0.f : raw[e][j];
-                }
-            }
-            put(dst_v, std::true_type{});
-        };
+        }
+        put(dst_v, std::true_type{});
+    };
 
-        load_k(0);
-        // ---- Q prologue: lane holds Q[row r16][32 c + 8 g + j], the B operand of step c:
-        // normalised, rotated (pair i < 32 is chunks 0 and 1 of the lane) and scaled by
-        // scale * log2 e (the scores then are exponents of 2), in FP32, then split
-        bf16x8 qh[8], qm[8], ql[8];
-        {
-            // every load goes out before the first is used
-            const int t = q_row0 + (q_valid ? r16 : 0);
-            const float *qs = p.qkv + (size_t)t * p.row + (size_t)h * 2 * HD + 8 * g;
-            float x[8][8];
-            f32x4 w[8][2], cs[4];
+    load_k(0);
+    // ---- Q prologue: lane holds Q[row r16][32 c + 8 g + j], the B operand of step c:
+    // normalised, rotated (pair i < 32 is chunks 0 and 1 of the lane) and scaled by
+    // scale * log2 e (the scores then are exponents of 2), in FP32, then split
+    bf16x8 qh[8], qm[8], ql[8];
+    {
+        // every load goes out before the first is used
+        const int t = q_row0 + (q_valid ? r16 : 0);
+        const float *qs = p.qkv + (size_t)t * p.row + (size_t)h * 2 * HD + 8 * g;
+        float x[8][8];
+        f32x4 w[8][2], cs[4];
 #pragma unroll
-            for (int c = 0; c < 8; c++) {
-                const f32x4 a = *(const f32x4 *)(qs + 32 * c), b = *(const f32x4 *)(qs + 32 * c + 4);
+        for (int c = 0; c < 8; c++) {
+            const f32x4 a = *(const f32x4 *)(qs + 32 * c), b = *(const f32x4 *)(qs + 32 * c + 4);
 #pragma unroll
-                for (int j = 0; j < 4; j++) { x[c][j] = a[j]; x[c][4 + j] = b[j]; }
+            for (int j = 0; j < 4; j++) { x[c][j] = a[j]; x[c][4 + j] = b[j]; }
+        }
+        // without norms or a table, the pass's own rows stand in (loaded, not used)
+        const float *ws = p.q_norm ? p.q_norm + 8 * g : qs, *ts = p.rope_cs ? p.rope_cs + (size_t)t * 64 + 16 * g : qs;
+#pragma unroll
+        for (int c = 0; c < 8; c++)
+#pragma unroll
+            for (int i = 0; i < 2; i++) w[c][i] = *(const f32x4 *)(ws + 32 * c + 4 * i);
+#pragma unroll
+        for (int q = 0; q < 4; q++) cs[q] = *(const f32x4 *)(ts + 4 * q);   // cos, sin of pairs 8g + 2q, 8g + 2q + 1
+        if (p.n_rot && !p.rope_cs) {
+            // no table: the wave evaluates its rows' angles into LDS (the V^T region is free)
+            float2 *tab = (float2 *)(smem + KV) + 16 * 32 * wave;
+            for (int i = lane; i < 16 * 32; i += 64) {
+                const int row = i >> 5;
+                float c, s;
+                rope_cs_f32(p.pos3, p.inv_freq, q_row0 + (row < nq ? row : 0), i & 31, &c, &s);
+                tab[i] = make_float2(c, s);
             }
-            // without norms or a table, the pass's own rows stand in (loaded, not used)
-            const float *ws = p.q_norm ? p.q_norm + 8 * g : qs, *ts = p.rope_cs ? p.rope_cs + (size_t)t * 64 + 16 * g : qs;
+#pragma unroll
+            for (int q = 0; q < 4; q++) cs[q] = *(const f32x4 *)(tab + 32 * r16 + 8 * g + 2 * q);
+        }
+        if (p.q_norm) {
+            float ss = 0.f;
 #pragma unroll
             for (int c = 0; c < 8; c++)
 #pragma unroll
-                for (int i = 0; i < 2; i++) w[c][i] = *(const f32x4 *)(ws + 32 * c + 4 * i);
+                for (int j = 0; j < 8; j++) ss += x[c][j] * x[c][j];
+            ss += __shfl_xor(ss, 16);
+            ss += __shfl_xor(ss, 32);
+            const float inv = 1.0f / sqrtf(ss / (float)HD + p.eps);
 #pragma unroll
-            for (int q = 0; q < 4; q++) cs[q] = *(const f32x4 *)(ts + 4 * q);   // cos, sin of pairs 8g + 2q, 8g + 2q + 1
-            if (p.n_rot && !p.rope_cs) {
-                // no table: the wave evaluates its rows' angles into LDS (the V^T region is free)
-                float2 *tab = (float2 *)(smem + KV) + 16 * 32 * wave;
-                for (int i = lane; i < 16 * 32; i += 64) {
-                    const int row = i >> 5;
-                    float c, s;
-                    rope_cs_f32(p.pos3, p.inv_freq, q_row0 + (row < nq ? row : 0), i & 31, &c, &s);
-                    tab[i] = make_float2(c, s);
-                }
+            for (int c = 0; c < 8; c++)
 #pragma unroll
-                for (int q = 0; q < 4; q++) cs[q] = *(const f32x4 *)(tab + 32 * r16 + 8 * g + 2 * q);
-            }
-            if (p.q_norm) {
-                float ss = 0.f;
+                for (int j = 0; j < 8; j++) x[c][j] = x[c][j] * inv * w[c][j >> 2][j & 3];
+        }
+        if (p.n_rot) {
 #pragma unroll
-                for (int c = 0; c < 8; c++)
-#pragma unroll
-                    for (int j = 0; j < 8; j++) ss += x[c][j] * x[c][j];
-                ss += __shfl_xor(ss, 16);
-                ss += __shfl_xor(ss, 32);
-                const float inv = 1.0f / sqrtf(ss / (float)HD + p.eps);
-#pragma unroll
-                for (int c = 0; c < 8; c++)
-#pragma unroll
-                    for (int j = 0; j < 8; j++) x[c][j] = x[c][j] * inv * w[c][j >> 2][j & 3];
-            }
-            if (p.n_rot) {
-#pragma unroll
-                for (int j = 0; j < 8; j++) {
-                    const float c = cs[j >> 1][2 * (j & 1)], s = cs[j >> 1][2 * (j & 1) + 1];
-                    const float x0 = x[0][j], x1 = x[1][j];
-                    x[0][j] = x0 * c - x1 * s;
-                    x[1][j] = x1 * c + x0 * s;
-                }
-            }
-            const float sl2 = p.scale * 1.4426950408889634f;
-#pragma unroll
-            for (int c = 0; c < 8; c++) {
-#pragma unroll
-                for (int j = 0; j < 8; j++) x[c][j] *= sl2;
-                amax = split32::split_amax(amax, x[c]);
-                const split32::Parts s = split32::split8(x[c], wt);
-                qh[c] = s.h; qm[c] = s.m; ql[c] = s.l;
+            for (int j = 0; j < 8; j++) {
+                const float c = cs[j >> 1][2 * (j & 1)], s = cs[j >> 1][2 * (j & 1) + 1];
+                const float x0 = x[0][j], x1 = x[1][j];
+                x[0][j] = x0 * c - x1 * s;
+                x[1][j] = x1 * c + x0 * s;
             }
         }
-        // the previous item's last reads are behind its closing barrier
-        put_k(0);
-        load_v(0);
+        const float sl2 = p.scale * 1.4426950408889634f;
+#pragma unroll
+        for (int c = 0; c < 8; c++) {
+#pragma unroll
+            for (int j = 0; j < 8; j++) x[c][j] *= sl2;
+            amax = split32::split_amax(amax, x[c]);
+            const split32::Parts s = split32::split8(x[c], wt);
+            qh[c] = s.h; qm[c] = s.m; ql[c] = s.l;
+        }
+    }
+    put_k(0);
+    load_v(0);
 
-        f32x4 o[16];
+    f32x4 o[16];
 #pragma unroll
-        for (int n = 0; n < 16; n++) o[n] = f32x4{0.f, 0.f, 0.f, 0.f};
-        // the running maximum starts at the lowest finite value: a row that has seen no key yet
-        // then needs no case of its own
-        float m_run = -3.4028235e38f, l_run = 0.f;
-        // every LDS access of the phase is done; the loads in flight stay so
-        auto phase_barrier = [&]() {
-            __builtin_amdgcn_sched_barrier(0);
-            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-            __builtin_amdgcn_sched_barrier(0);
-        };
-        for (int t = 0; t < n_tiles; t++) {
-            const int kb = t * BK;
-            const bool mine = kb < my_len;   // wave-uniform
-            phase_barrier();                 // K(t) is in place; V(t - 1) has been read
-            // S^T: two 16-key subtiles, eight 32-dim steps; the hh terms in one accumulator, the
-            // smaller ones in another
-            split32::Ring ring;
-            f32x4 s[2], sx[2];
+    for (int n = 0; n < 16; n++) o[n] = f32x4{0.f, 0.f, 0.f, 0.f};
+    // the running maximum starts at the lowest finite value: a row that has seen no key yet
+    // then needs no case of its own
+    float m_run = -3.4028235e38f, l_run = 0.f;
+    // every LDS access of the phase is done; the loads in flight stay so
+    auto phase_barrier = [&]() {
+        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    for (int t = 0; t < n_tiles; t++) {
+        const int kb = t * BK;
+        const bool mine = kb < my_len;   // wave-uniform
+        phase_barrier();                 // K(t) is in place; V(t - 1) has been read
+        // S^T: two 16-key subtiles, eight 32-dim steps; the hh terms in one accumulator, the
+        // smaller ones in another
+        split32::Ring ring;
+        f32x4 s[2], sx[2];
 #pragma unroll
-            for (int u = 0; u < 2; u++) s[u] = sx[u] = f32x4{0.f, 0.f, 0.f, 0.f};
-            if (mine) split32::ring_start<PL, 0, 4 * 2 * HD>(ring, ka[0], ka[0]);
-            const bool more = t + 1 < n_tiles;
-            put_v(kb);
-            if (more) load_k(kb + BK);
-            if (mine) {
-                split32::sfor<8>([&](auto I) {
-                    constexpr int i = decltype(I)::value, n = i + 1, o8 = 256 * (n / 4);
-                    split32::ring_step<PL, (n < 8), o8, o8 + 4 * 2 * HD>(ring, ka[n % 4], ka[n % 4], s[0], s[1], sx[0], sx[1], qh[i], qm[i], ql[i]);
-                });
-            }
-            phase_barrier();                 // V(t) is in place; K(t) has been read
-            if (mine) split32::ring_start<PL, 0, 0>(ring, va[0], va[1]);
-            if (more) {
-                put_k(kb + BK);
-                load_v(kb + BK);
-            }
-            if (mine) {
-                // x[4 u + v] is the score (exponent of 2) of key kb + 8g + 4u + v for row r16
-                float x[8], mx, rs = 0.f;
-#pragma unroll
-                for (int j = 0; j < 8; j++) x[j] = s[j >> 2][j & 3] + sx[j >> 2][j & 3];
-                if (kb + BK > k_len || (p.causal && kb + BK - 1 > q_pos0)) {
-                    const int lim = (p.causal ? min(k_len - 1, q_pos0 + r16) : k_len - 1) - kb - 8 * g;
-#pragma unroll
-                    for (int j = 0; j < 8; j++) x[j] = j <= lim ? x[j] : -INFINITY;
-                }
-                mx = x[0];
-#pragma unroll
-                for (int j = 1; j < 8; j++) mx = fmaxf(mx, x[j]);
-                const float mn = fmaxf(m_run, xrow_max(mx));
-                const float alpha = __builtin_amdgcn_exp2f(m_run - mn);
-#pragma unroll
-                for (int j = 0; j < 8; j++) {
-                    x[j] = split32::P_SCALE * __builtin_amdgcn_exp2f(x[j] - mn);   // a masked key's -inf gives 0
-                    rs += x[j];
-                }
-                m_run = mn;
-                l_run = l_run * alpha + rs;
-                if (__any(alpha != 1.f)) {   // in place (as plain C++ the other path copies the registers)
-#pragma unroll
-                    for (int n = 0; n < 16; n++)
-#pragma unroll
-                        for (int v = 0; v < 4; v++) {
-                            float d = o[n][v];
-                            asm("v_mul_f32 %0, %1, %0" : "+v"(d) : "v"(alpha));
-                            o[n][v] = d;
-                        }
-                }
-                const split32::Parts pp = split32::split8(x, wt);
-                // O^T += V^T . P^T: pairs of 16-dim tiles, the six terms smallest first
-                split32::sfor<8>([&](auto I) {
-                    constexpr int i = decltype(I)::value, o8 = 32 * (i + 1) * 2 * BK;
-                    split32::ring_step<PL, (i + 1 < 8), o8, o8>(ring, va[0], va[1], o[2 * i], o[2 * i + 1], o[2 * i], o[2 * i + 1], pp.h, pp.m, pp.l);
-                });
-            }
+        for (int u = 0; u < 2; u++) s[u] = sx[u] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (mine) split32::ring_start<PL, 0, 4 * 2 * HD>(ring, ka[0], ka[0]);
+        const bool more = t + 1 < n_tiles;
+        put_v(kb);
+        if (more) load_k(kb + BK);
+        if (mine) {
+            split32::sfor<8>([&](auto I) {
+                constexpr int i = decltype(I)::value, n = i + 1, o8 = 256 * (n / 4);
+                split32::ring_step<PL, (n < 8), o8, o8 + 4 * 2 * HD>(ring, ka[n % 4], ka[n % 4], s[0], s[1], sx[0], sx[1], qh[i], qm[i], ql[i]);
+            });
         }
-
-        // ---- epilogue: O = O^T / l, times sigmoid(gate). Tiles 2u, 2u + 1 of lane (g, r16) are
-        // dims 32 u + 8 g .. + 7 of row r16.
-        float l_row = l_run;
-        l_row += __shfl_xor(l_row, 16);
-        l_row += __shfl_xor(l_row, 32);
-        bool plain = false;
-        if (__syncthreads_or(!split32::split_fine(amax))) {   // also: the tiles' last reads are done
-            const int first = split32::first_bad_key<HD>(kbase, vbase, k_len, (int *)smem);
-            int own = 0;
-#pragma unroll
-            for (int c = 0; c < 8; c++) own |= split32::query_bad(qh[c]);
-            own |= __shfl_xor(own, 16);
-            own |= __shfl_xor(own, 32);
-            plain = q_valid && (own || first < (p.causal ? q_pos0 + r16 + 1 : k_len));
+        phase_barrier();                 // V(t) is in place; K(t) has been read
+        if (mine) split32::ring_start<PL, 0, 0>(ring, va[0], va[1]);
+        if (more) {
+            put_k(kb + BK);
+            load_v(kb + BK);
         }
-        if (q_valid && !plain) {
-            const float il = l_row > 0.f ? (1.0f / split32::V_SCALE) / l_row : 0.f;
-            const size_t t = (size_t)(q_row0 + r16);
-            const size_t obase = t * p.nh * HD + (size_t)h * HD + 8 * g;
-            if (p.gate) {   // every gate load goes out before the first store
-                const float *grow = p.qkv + t * p.row + (size_t)h * 2 * HD + HD + 8 * g;
-                f32x4 gv[16];
+        if (mine) {
+            // x[4 u + v] is the score (exponent of 2) of key kb + 8g + 4u + v for row r16
+            float x[8], mx, rs = 0.f;
 #pragma unroll
-                for (int n = 0; n < 16; n++) gv[n] = *(const f32x4 *)(grow + 32 * (n >> 1) + 4 * (n & 1));
+            for (int j = 0; j < 8; j++) x[j] = s[j >> 2][j & 3] + sx[j >> 2][j & 3];
+            if (kb + BK > k_len || (p.causal && kb + BK - 1 > q_pos0)) {
+                const int lim = (p.causal ? min(k_len - 1, q_pos0 + r16) : k_len - 1) - kb - 8 * g;
+#pragma unroll
+                for (int j = 0; j < 8; j++) x[j] = j <= lim ? x[j] : -INFINITY;
+            }
+            mx = x[0];
+#pragma unroll
+            for (int j = 1; j < 8; j++) mx = fmaxf(mx, x[j]);
+            const float mn = fmaxf(m_run, xrow_max(mx));
+            const float alpha = __builtin_amdgcn_exp2f(m_run - mn);
+#pragma unroll
+            for (int j = 0; j < 8; j++) {
+                x[j] = split32::P_SCALE * __builtin_amdgcn_exp2f(x[j] - mn);   // a masked key's -inf gives 0
+                rs += x[j];
+            }
+            m_run = mn;
+            l_run = l_run * alpha + rs;
+            if (__any(alpha != 1.f)) {   // in place (as plain C++ the other path copies the registers)
 #pragma unroll
                 for (int n = 0; n < 16; n++)
 #pragma unroll
-                    for (int v = 0; v < 4; v++) o[n][v] = o[n][v] * il * sigmoidf(gv[n][v]);
-            } else {
-#pragma unroll
-                for (int n = 0; n < 16; n++) o[n] *= il;
+                    for (int v = 0; v < 4; v++) {
+                        float d = o[n][v];
+                        asm("v_mul_f32 %0, %1, %0" : "+v"(d) : "v"(alpha));
+                        o[n][v] = d;
+                    }
             }
-            auto store = [&](const int type) {
-#pragma unroll
-                for (int u = 0; u < 8; u++) {
-                    float w[8];
-#pragma unroll
-                    for (int j = 0; j < 8; j++) w[j] = o[2 * u + (j >> 2)][j & 3];
-                    store_out8(p.out, obase + 32 * u, w, type, p.f16_lim, flag);
-                }
-            };
-            if (p.out_type == CLEF_HIP_OUT_F32) store(CLEF_HIP_OUT_F32);
-            else if (p.out_type == CLEF_HIP_OUT_BF16) store(CLEF_HIP_OUT_BF16);
-            else store(CLEF_HIP_OUT_F16);
+            const split32::Parts pp = split32::split8(x, wt);
+            // O^T += V^T . P^T: pairs of 16-dim tiles, the six terms smallest first
+            split32::sfor<8>([&](auto I) {
+                constexpr int i = decltype(I)::value, o8 = 32 * (i + 1) * 2 * BK;
+                split32::ring_step<PL, (i + 1 < 8), o8, o8>(ring, va[0], va[1], o[2 * i], o[2 * i + 1], o[2 * i], o[2 * i + 1], pp.h, pp.m, pp.l);
+            });
         }
-        const unsigned plain_rows = (unsigned)__ballot(plain) & 0xffffu;
-        if (plain_rows) text_rows_plain(p, plain_rows, q_row0, q_pos0, k_row0, k_len, h, kh, flag);
     }
+
+    // ---- epilogue: O = O^T / l, times sigmoid(gate). Tiles 2u, 2u + 1 of lane (g, r16) are
+    // dims 32 u + 8 g .. + 7 of row r16.
+    float l_row = l_run;
+    l_row += __shfl_xor(l_row, 16);
+    l_row += __shfl_xor(l_row, 32);
+    bool plain = false;
+    if (__syncthreads_or(!split32::split_fine(amax))) {   // also: the tiles' last reads are done
+        const int first = split32::first_bad_key<HD>(kbase, vbase, k_len, (int *)smem);
+        int own = 0;
+#pragma unroll
+        for (int c = 0; c < 8; c++) own |= split32::query_bad(qh[c]);
+        own |= __shfl_xor(own, 16);
+        own |= __shfl_xor(own, 32);
+        plain = q_valid && (own || first < (p.causal ? q_pos0 + r16 + 1 : k_len));
+    }
+    if (q_valid && !plain) {
+        const float il = l_row > 0.f ? (1.0f / split32::V_SCALE) / l_row : 0.f;
+        const size_t t = (size_t)(q_row0 + r16);
+        const size_t obase = t * p.nh * HD + (size_t)h * HD + 8 * g;
+        if (p.gate) {   // every gate load goes out before the first store
+            const float *grow = p.qkv + t * p.row + (size_t)h * 2 * HD + HD + 8 * g;
+            f32x4 gv[16];
+#pragma unroll
+            for (int n = 0; n < 16; n++) gv[n] = *(const f32x4 *)(grow + 32 * (n >> 1) + 4 * (n & 1));
+#pragma unroll
+            for (int n = 0; n < 16; n++)
+#pragma unroll
+                for (int v = 0; v < 4; v++) o[n][v] = o[n][v] * il * sigmoidf(gv[n][v]);
+        } else {
+#pragma unroll
+            for (int n = 0; n < 16; n++) o[n] *= il;
+        }
+        auto store = [&](const int type) {
+#pragma unroll
+            for (int u = 0; u < 8; u++) {
+                float w[8];
+#pragma unroll
+                for (int j = 0; j < 8; j++) w[j] = o[2 * u + (j >> 2)][j & 3];
+                store_out8(p.out, obase + 32 * u, w, type, p.f16_lim, flag);
+            }
+        };
+        if (p.out_type == CLEF_HIP_OUT_F32) store(CLEF_HIP_OUT_F32);
+        else if (p.out_type == CLEF_HIP_OUT_BF16) store(CLEF_HIP_OUT_BF16);
+        else store(CLEF_HIP_OUT_F16);
+    }
+    const unsigned plain_rows = (unsigned)__ballot(plain) & 0xffffu;
+    if (plain_rows) text_rows_plain(p, plain_rows, q_row0, q_pos0, k_row0, k_len, h, kh, flag);
 }
 
 }  // namespace text32
