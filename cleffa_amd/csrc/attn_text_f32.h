@@ -514,7 +514,14 @@ __global__ __launch_bounds__(64 * NW) void attn_text_f32_kernel(Params p) {
         if (mine) split32::ring_start<PL, 0, 4 * 2 * HD>(ring, ka[0], ka[0]);
         const bool more = t + 1 < n_tiles;
         put_v(kb);
-        if (more) load_k(kb + BK);
+        if (more) {
+            load_k(kb + BK);
+        } else {   // nothing: but a value that seemed to live on would be copied before its split
+#pragma unroll
+            for (int e = 0; e < 2; e++)
+#pragma unroll
+                for (int j = 0; j < 8; j++) asm volatile("" : "=v"(raw[e][j]));
+        }
         if (mine) {
             split32::sfor<8>([&](auto I) {
                 constexpr int i = decltype(I)::value, n = i + 1, o8 = 256 * (n / 4);
