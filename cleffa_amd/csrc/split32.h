@@ -50,21 +50,21 @@ __device__ __forceinline__ float minus_hi(unsigned pair, const Weights &w, float
     return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, pair), __builtin_bit_cast(bf16x2, w.hi), x, false);
 }
 
-// the parts of one pair of elements, as packed words
-__device__ __forceinline__ void split2(float a, float b, const Weights &w, unsigned &h, unsigned &m, unsigned &l) {
-    h = pack_bf16(a, b);
-    const float a1 = minus_lo(h, w, a), b1 = minus_hi(h, w, b);
-    m = pack_bf16(a1, b1);
-    l = pack_bf16(minus_lo(m, w, a1), minus_hi(m, w, b1));
-}
+// Part by part over the eight elements: pair by pair, each conversion waited for the differences ahead of it
+// (C1 FP32 303 -> 296 us, Omni 1 - 3%).
 __device__ __forceinline__ Parts split8(const float (&x)[8], const Weights &w) {
     u32x4 h, m, l;
+    float r[8];
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-        unsigned a, b, c;
-        split2(x[2 * i], x[2 * i + 1], w, a, b, c);
-        h[i] = a; m[i] = b; l[i] = c;
-    }
+    for (int i = 0; i < 4; i++) h[i] = pack_bf16(x[2 * i], x[2 * i + 1]);
+#pragma unroll
+    for (int i = 0; i < 4; i++) { r[2 * i] = minus_lo(h[i], w, x[2 * i]); r[2 * i + 1] = minus_hi(h[i], w, x[2 * i + 1]); }
+#pragma unroll
+    for (int i = 0; i < 4; i++) m[i] = pack_bf16(r[2 * i], r[2 * i + 1]);
+#pragma unroll
+    for (int i = 0; i < 4; i++) { r[2 * i] = minus_lo(m[i], w, r[2 * i]); r[2 * i + 1] = minus_hi(m[i], w, r[2 * i + 1]); }
+#pragma unroll
+    for (int i = 0; i < 4; i++) l[i] = pack_bf16(r[2 * i], r[2 * i + 1]);
     return {__builtin_bit_cast(bf16x8, h), __builtin_bit_cast(bf16x8, m), __builtin_bit_cast(bf16x8, l)};
 }
 
