@@ -83,7 +83,7 @@ __device__ __forceinline__ bool split_bad(float x) { return !(fabsf(x) < LIMIT);
 __device__ __forceinline__ float split_amax(float amax, const float (&x)[8]) {
     asm("v_maximum3_f32 %0, |%1|, |%2|, %0\n\tv_maximum3_f32 %0, |%3|, |%4|, %0\n\t"
         "v_maximum3_f32 %0, |%5|, |%6|, %0\n\tv_maximum3_f32 %0, |%7|, |%8|, %0"
-        : "+v"(amax) : "v"(x[0]), "v"(x[1]), "v"(x[2]), "v"(x[3]), "v"(x[4]), "v"(x[5]), "v"(x[6]), "v"(x[7]));
+        : "+&v"(amax) : "v"(x[0]), "v"(x[1]), "v"(x[2]), "v"(x[3]), "v"(x[4]), "v"(x[5]), "v"(x[6]), "v"(x[7]));
     return amax;
 }
 // (the margin: a bad query is told by its high parts, rounded)
