@@ -331,6 +331,22 @@ def test_fp32_rows_that_do_not_see_a_value_keep_their_bits(nh, nkv, which):
     assert torch.equal(got[~sees], clean[~sees])
 
 
+@pytest.mark.parametrize("gate", [True, False])
+def test_fp32_plain_rows_in_16_bits(gate):
+    """Rows on the plain path give bf16 and f16 outputs as the others do: the f32 output rounded, f16 saturated
+    and its record flagged, the other record's rows and flag untouched."""
+    _say(f"[fp32] plain rows in 16 bits, gate {gate}")
+    w = _fp32(dict(workloads.text_inputs([100, 70], 8, 2, seed=6), gate=gate, theta=1e7))
+    w, _ = _with_bad_value(w, "v_big", 60)
+    f32 = _run(w)[0]
+    assert (f32[60:100].abs() > 65504).any() and torch.isfinite(f32).all()
+    assert torch.equal(_run(w, out_dtype="bf16")[0].view(torch.int16), f32.to(torch.bfloat16).view(torch.int16))
+    ovf = torch.zeros(170, dtype=torch.int32, device="cuda")
+    f16 = _run(w, out_dtype="f16", ovf=ovf)[0]
+    assert torch.equal(f16.view(torch.int16), f32.clamp(-65504, 65504).to(torch.float16).view(torch.int16))
+    assert ovf.nonzero().flatten().tolist() == [0]
+
+
 @pytest.mark.parametrize("which", BAD_VALUES)
 def test_fp32_bad_values_agree_bitwise_over_item_sizes(which):
     """A record that holds such a value has the same bits alone (four-wave items), in a pass of eight-wave items,
