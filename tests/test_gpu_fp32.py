@@ -331,6 +331,26 @@ def test_fp32_rows_that_do_not_see_a_value_keep_their_bits(nh, nkv, which):
     assert torch.equal(got[~sees], clean[~sees])
 
 
+@pytest.mark.parametrize("which", ["v_inf", "v_big", "q_nan"])
+def test_fp32_bad_values_without_a_causal_mask(which):
+    """Without the mask every row of the record sees a bad key: the affected heads against float64, the
+    others with the bits of the clean pass."""
+    _say(f"[fp32] {which} without a causal mask")
+    nh, nkv, T = 6, 2, 110
+    w = _fp32(dict(workloads.text_inputs([70, 40], nh, nkv, seed=3), gate=False, theta=1e7))
+    bad, heads = _with_bad_value(w, which, 30)
+    plan = AttnPlan(w["cu_seqlens"], causal=False)
+    clean, got = (_run(x, plan=plan)[0].cpu().numpy().reshape(T, nh, 256) for x in (w, bad))
+    with np.errstate(all="ignore"):
+        want = oracle_text(bad, causal=False).reshape(T, nh, 256)
+    sees = np.zeros((T, nh), bool)
+    sees[(slice(30, 31) if which == "q_nan" else slice(0, 70)), list(heads)] = True
+    assert np.array_equal(got[~sees].view(np.uint32), clean[~sees].view(np.uint32))
+    fine = np.isfinite(want)
+    assert np.array_equal(got[~fine], want[~fine].astype(np.float32), equal_nan=True)
+    assert (np.abs(got[fine] - want[fine]) / np.maximum(np.abs(want[fine]), 1)).max() < 2e-5
+
+
 @pytest.mark.parametrize("gate", [True, False])
 def test_fp32_plain_rows_in_16_bits(gate):
     """Rows on the plain path give bf16 and f16 outputs as the others do: the f32 output rounded, f16 saturated
