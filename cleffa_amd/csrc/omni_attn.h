@@ -7,8 +7,8 @@
 // Both products run on the bf16 matrix cores with every FP32 operand split into three bf16 parts
 // and six products per pair (split32.h). Bounds of the item loop, per 32-key tile and SIMD: 192
 // matrix instructions of 16 cycles against 128 FP32 ones of 32 cycles and 128 FP64 ones of 64 for
-// the same work before. At 16,344 tokens, 32 / 4 heads: 27.9 -> 10.7 ms, 53% of the cycles on the matrix cores at
-// 2.1 GHz; relative error against float64 3.2e-7 -> 1.8e-7 (most of it the FP32 output's
+// the same work before. At 16,344 tokens, 32 / 4 heads: 27.85 -> 11.38 ms in turn on one box, 54% of the cycles on the
+// matrix cores at 2.04 GHz; relative error against float64 3.3e-7 -> 1.8e-7 (most of it the FP32 output's
 // rounding: the scores take 5 full-size roundings instead of 32). Where the scores do not matter, the FP32 sums
 // within a tile show: constant V over 200 random scores comes back within 0.5 x 2^-24 rms, with FP64 products 0.2.
 //
