@@ -55,7 +55,7 @@ def lds_wait_hazards(lines):
         if op == "s_waitcnt":
             if m:
                 keep = int(m.group(1))
-                pending = pending[len(pending) - keep:] if keep else []
+                pending = pending[max(len(pending) - keep, 0):]
             continue
         if op.startswith("ds_read") or op.startswith("ds_load"):
             srcs = set().union(*[_regs(a) for a in args[1:]])
@@ -80,9 +80,12 @@ def test_scanner_catches_a_copy_before_the_wait():
     ahead = ["\t;;#ASMSTART", "\tds_read_b128 v[8:11], v2", "\t;;#ASMEND", "\t;;#ASMSTART",
              "\tds_read_b128 v[12:15], v3", "\t;;#ASMEND", "\t;;#ASMSTART", "\ts_waitcnt lgkmcnt(1)",
              "\t;;#ASMEND", "\tv_mov_b32 v0, v8", "\tv_mov_b32 v1, v12"]
+    few = ["\t;;#ASMSTART", "\tds_read_b128 v[8:11], v2", "\t;;#ASMEND", "\t;;#ASMSTART", "\tds_read_b128 v[12:15], v3", "\t;;#ASMEND",
+           "\ts_waitcnt lgkmcnt(3)", "\tv_mov_b32 v0, v8"]   # waits for neither read
     assert lds_wait_hazards(good) == []
     assert len(lds_wait_hazards(bad)) == 1
     assert [t for _, t in lds_wait_hazards(ahead)] == ["v_mov_b32 v1, v12"]
+    assert [t for _, t in lds_wait_hazards(few)] == ["v_mov_b32 v0, v8"]
 
 
 @pytest.mark.skipif(not Path(HIPCC).exists(), reason="hipcc not found")
