@@ -196,9 +196,9 @@ def test_fp32_random_pass(seed):
 
 @pytest.mark.parametrize("which", ["v_inf", "v_big", "v_small", "q_big", "k_minus"])
 def test_fp32_values_without_bf16_parts(which):
-    """Infinities and magnitudes above bf16's overflow threshold (3.39e38) have no bf16 parts: items
-    that hold one run in plain FP32, against float64 (infinite and NaN outputs included); records
-    beside them stay bit for bit what they are alone. Values of 1e-28 keep their relative precision."""
+    """Infinities and magnitudes above bf16's overflow threshold (3.39e38) have no bf16 parts: rows
+    that see one run on the FP32 matrix instructions, against float64 (infinite and NaN outputs included); records
+    beside theirs stay bit for bit what they are alone. Values of 1e-28 keep their relative precision."""
     _say(f"[fp32] values {which}")
     lengths, nh, nkv, hd = [40, 70, 21], 8, 2, 256
     plain = which in ("q_big", "k_minus")

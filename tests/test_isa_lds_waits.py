@@ -30,8 +30,9 @@ def _regs(tok):
 
 def lds_wait_hazards(lines):
     """Linear scan of one kernel's assembly. LDS-counter operations (asm ds_reads with their
-    destination registers, compiler ds ops and scalar loads as placeholders) are queued in issue
-    order; `s_waitcnt lgkmcnt(N)` retires all but the newest N. Any other instruction that names a
+    destination registers, compiler ds ops as placeholders) are queued in issue
+    order; `s_waitcnt lgkmcnt(N)` retires all but the newest N. Scalar loads count too but may return before older
+    reads, so they stand for none. Any other instruction that names a
     register of a queued asm read is reported. Past an unconditional branch, the queue restarts at
     the next label (its predecessors are elsewhere in the listing)."""
     pending, found = [], []
@@ -63,7 +64,7 @@ def lds_wait_hazards(lines):
                 found.append((n, t))
             pending.append(_regs(args[0]) if in_asm else set())
             continue
-        if op.startswith("ds_") or op.startswith("s_load") or op.startswith("s_buffer_load"):
+        if op.startswith("ds_"):
             pending.append(set())
             continue
         used = set().union(*[_regs(a) for a in args])
@@ -82,10 +83,12 @@ def test_scanner_catches_a_copy_before_the_wait():
              "\t;;#ASMEND", "\tv_mov_b32 v0, v8", "\tv_mov_b32 v1, v12"]
     few = ["\t;;#ASMSTART", "\tds_read_b128 v[8:11], v2", "\t;;#ASMEND", "\t;;#ASMSTART", "\tds_read_b128 v[12:15], v3", "\t;;#ASMEND",
            "\ts_waitcnt lgkmcnt(3)", "\tv_mov_b32 v0, v8"]   # waits for neither read
+    scalar = few[:3] + ["\ts_load_dword s0, s[2:3], 0x0", "\ts_waitcnt lgkmcnt(1)", "\tv_mov_b32 v0, v8"]   # the load may be the one that came
     assert lds_wait_hazards(good) == []
     assert len(lds_wait_hazards(bad)) == 1
     assert [t for _, t in lds_wait_hazards(ahead)] == ["v_mov_b32 v1, v12"]
-    assert [t for _, t in lds_wait_hazards(few)] == ["v_mov_b32 v0, v8"]
+    for lines in (few, scalar):
+        assert [t for _, t in lds_wait_hazards(lines)] == ["v_mov_b32 v0, v8"]
 
 
 @pytest.mark.skipif(not Path(HIPCC).exists(), reason="hipcc not found")

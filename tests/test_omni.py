@@ -265,8 +265,8 @@ def test_omni_group_widths_and_tile_edges(nh, nkv):
 @pytest.mark.parametrize("nh,nkv", [(8, 1), (4, 1)])
 @pytest.mark.parametrize("which", ["v_inf", "v_big", "v_small", "k_minus", "q_big"])
 def test_omni_values_without_bf16_parts(nh, nkv, which):
-    """Infinities and magnitudes above bf16's overflow threshold (3.39e38) have no bf16 parts: such
-    items run in plain FP32, and records beside them stay bit for bit what they are alone."""
+    """Infinities and magnitudes above bf16's overflow threshold (3.39e38) have no bf16 parts: rows that
+    see one run on the FP32 and FP64 matrix instructions, and every record stays bit for bit what it is alone."""
     print(f"[omni] values {which} {nh}/{nkv}", flush=True)
     lens = [40, 70, 21]
     cu = np.concatenate([[0], np.cumsum(lens)])
