@@ -585,7 +585,9 @@ bool clef_hip_qkv_gemm(int H, const uint16_t *X, const uint16_t *W, const clef_h
     // round takes relative to one of 256 x 256 tiles (us at 14336 x 5120 with T = 61 / 512 / 1024):
     //   256 x 256 (111 / 137 / 138): the fewest operand bytes per product; 128-row tiles move 1.5 times as many
     //             and run fill-bound on whole rounds (0.59 against 0.53 ms at T = 4096).
-    //   128 x 256 (75 / 87 / 161): twice the tiles, for passes that leave half the CUs without a 256-row one.
+    //   128 x 256 (75 / 87 / 161): twice the tiles, for passes that leave half the CUs without a 256-row one. A round
+    //             behind two others costs more (0.69): the 256-row tiles' last round, part empty, runs faster than a full
+    //             one (T = 800, three rounds of theirs against four: 36864 x 8192 576 / 598, as halves 532).
     //   128 x 64, 64 x 64 (41, 38 / 154, 201 / -): few rows, where reading W is the work: 56 tiles of 256
     //             columns pull 147 MB through 56 CUs, 224 narrow ones, six to eight slices deep, at 4 TB/s.
     //   128 x 128 (52 / 108 / 194): in between, where it is one round and the others more or emptier (T = 160:
@@ -604,7 +606,8 @@ bool clef_hip_qkv_gemm(int H, const uint16_t *X, const uint16_t *W, const clef_h
     };
     const int most = (int)((N / 256 + 7) / 8 * ((a->T + 255L) / 256)), whole = gemm::whole_tiles(most);   // 256 x 256 tiles of an XCD
     const bool even = p.kv && most % gemm::XCD_CUS == gemm::XCD_CUS / 2 && whole > gemm::XCD_CUS && H < 5120;
-    const long cost[6] = {100 * rounds(256, 256), 63 * rounds(128, 256), 38 * rounds(128, 64), 33 * rounds(64, 64), 48 * rounds(128, 128),
+    const long tall = rounds(128, 256);
+    const long cost[6] = {100 * rounds(256, 256), (tall < 3 ? 63 : 69) * tall, 38 * rounds(128, 64), 33 * rounds(64, 64), 48 * rounds(128, 128),
                           whole == most || even ? LONG_MAX : 100L * (whole / gemm::XCD_CUS) + 63};
     const int best = (int)(std::min_element(cost, cost + 6) - cost);
     const bool kv = p.kv;
