@@ -196,16 +196,17 @@ bool core_f32(const clef_hip_attn_args *a, void *stream, char *err, size_t errle
     p.eps = a->eps; p.scale = a->scale; p.f16_lim = f16_limit(a->f16_lim);
     const int group = a->nh / a->nkv;
     const long cus = device_cus();
-    auto items = [&](int slots) {
+    auto items = [&](int slots) {   // of a block
         const text32::Shape f = text32::f32_shape(slots, group);
-        return (long)a->n_blk * (text32::BLK / (16 * f.R)) * (group / f.k) * a->nkv;
+        return (long)(text32::BLK / (16 * f.R)) * (group / f.k) * a->nkv;
     };
     // Eight waves of 16 rows share each K / V tile's split; a pass that gives them too few items to
     // fill the CUs runs items of four such waves, the others only helping with the splits.
-    p.slots = items(8) >= cus ? 8 : 4;
+    p.slots = a->n_blk * items(8) >= cus ? 8 : 4;
     // one workgroup per item, dispatched in the items' longest-first order: the hardware hands
     // each free CU the next item
-    const long n_items = items(p.slots);
+    p.stride = text32::f32_stride(a->n_blk, a->T, (int)items(p.slots), text32::BLK / (16 * text32::f32_shape(p.slots, group).R), cus);
+    const long n_items = (long)a->n_blk * p.stride;
     if (n_items > 0x7fffffffL) return fail(err, errlen, "grid too large");
     hipLaunchKernelGGL(text32::attn_text_f32_kernel, dim3((unsigned)n_items), dim3(64 * text32::NW), 0, (hipStream_t)stream, p);
     return launch_ok("attn_text_f32", err, errlen);

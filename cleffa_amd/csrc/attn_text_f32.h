@@ -58,6 +58,30 @@ __host__ __device__ inline int f32_heads(int slots, int rows, int group) {
     return 1;
 }
 
+// Workgroups of a block, for n_blk blocks of T rows in all with `items` items each in `subs` runs of rows, of which the
+// last ones hold a short block's rows and the others are empty. Workgroup i goes to shader engine i % 32 (eight XCDs of
+// four), busy or not: where the runs with rows fall on the same engines block after block, these take a second
+// round while the others idle. A block then gets idle workgroups up to the next count whose multiples bring the
+// items of the pass's blocks to all engines alike, at the latest the one that leaves the following block's items where
+// its own ended (modulo 32). That is done where
+//   the items with rows come unevenly, and the engines hit most get more than their CUs (records x tokens, us:
+//   16 / 8 heads, 12 x 64 43.4 -> 29.3; 32 / 4, 200 x 16 541 -> 141; 24 / 4, 200 x 16 164 -> 108), or
+//   the items with rows fit the CUs and all workgroups do not (15 / 3, 10 x 45 39.3 -> 25.7; 24 / 4,
+//   16 x 64 61.3 -> 37.8), unless they are of one key tile, where idle workgroups cost more (16 x 30 28.3 -> 29.1).
+__host__ inline int f32_stride(long n_blk, long T, int items, int subs, long cus) {
+    const int layer = items / subs, span = BLK / subs, turn = items & -items, step = turn < 32 ? turn : 32;
+    const long rows = n_blk > 0 ? (T + n_blk - 1) / n_blk : 0;   // of a block, rounded up
+    const long full = (rows + span - 1) / span * layer;           // its items with rows
+    const bool uneven = full % step && n_blk * ((full + step - 1) / step * step) > cus, spill = rows > BK && n_blk * full <= cus && n_blk * items > cus;
+    if (!uneven && !spill) return items;
+    int stride = items, turns;
+    do {
+        stride++;
+        turns = stride % 32 ? stride & -stride : 32;   // engines that one block's start moves on by at least
+    } while ((stride - layer) % 32 && (layer % turns || 32 / turns > n_blk));
+    return n_blk * stride < (1L << 32) / (64 * NW) ? stride : items;
+}
+
 struct PrepParams {
     const float *qkv;           // [T][row]
     const float *k_norm;        // [256] or NULL
@@ -82,6 +106,7 @@ struct Params {
     int32_t *ovf;
     int row, kvT, nh, nkv, n_rot, causal, gate, out_type;
     int slots;                  // waves of an item that hold rows: 8, or 4 (the others only stage tiles)
+    int stride;                 // workgroups of a block: its items, and idle ones behind them (core_f32)
     float eps, scale, f16_lim;
 };
 
@@ -300,7 +325,7 @@ __device__ __forceinline__ void text_rows_plain(const Params &p, unsigned rows, 
 // Work items are (block, R x 16 rows of it, k heads of a kv group, kv head), the plan's longest-first
 // blocks outermost, each block's last rows first, kv heads innermost (an XCD then streams the K / V
 // of few of them), one workgroup each. An item of few rows runs more heads (f32_heads), and the
-// items of the heads it took are empty.
+// items of the heads it took are empty, as are those past a block's rows.
 //
 // Per 32-key tile: barrier; S(t) while V(t) is split into LDS; barrier; softmax; P.V(t) while
 // K(t + 1) is split. The operand staged beside a product is the one the product does not read, so
@@ -325,11 +350,11 @@ __global__ __launch_bounds__(64 * NW) void attn_text_f32_kernel(Params p) {
     for (int w = 0; w < 2; w++)
         va[w] = lds0 + KV + (8 * (r16 >> 2) + 4 * w + (r16 & 3)) * (2 * BK) + ((g ^ (-(r16 >> 2) & 3) ^ w) * 16);
 
-    const int item = blockIdx.x;
-    const int kh = item % p.nkv, ic = item / p.nkv % n_ch, ib = item / p.nkv / n_ch;
-    const int32_t *blk = p.blocks + 8 * (ib / n_sub);
-    const int r0 = span * (n_sub - 1 - ib % n_sub), rows = min(span, blk[1] - r0);
-    if (rows <= 0) return;
+    const int bi = blockIdx.x / p.stride, item = blockIdx.x - bi * p.stride;
+    const int kh = item % p.nkv, ic = item / p.nkv % n_ch, sub = item / p.nkv / n_ch;
+    const int32_t *blk = p.blocks + 8 * bi;
+    const int r0 = span * (n_sub - 1 - sub), rows = min(span, blk[1] - r0);
+    if (sub >= n_sub || rows <= 0) return;
     const int kk = f32_heads(p.slots, rows, group), wph = (rows + 15) / 16;
     if (ic * kk >= group) return;
     const int slot = wave / wph;

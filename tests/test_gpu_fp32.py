@@ -414,3 +414,19 @@ def test_fp32_without_rope_table():
     without = att.forward(*d, plan, stage="core", **kw)
     torch.cuda.synchronize()
     assert torch.equal(with_table.view(torch.int32), without.view(torch.int32))
+
+
+@pytest.mark.parametrize("nh,nkv,lengths", [(16, 8, [64] * 12), (16, 4, [64] * 7 + [1] * 13), (32, 4, [9] * 40 + [130, 33]), (15, 3, [45] * 10),
+                                            (24, 4, [64] * 16), (3, 1, [40] * 45), (2, 1, [70] * 150)])
+def test_fp32_short_records_with_idle_workgroups(nh, nkv, lengths):
+    """Passes of short records, whose blocks are followed by idle workgroups: every row is written, and each record
+    has the bits it has alone."""
+    _say(f"[fp32] short records {nh}/{nkv} {len(lengths)} x {lengths[0]}")
+    w = _fp32(dict(workloads.text_inputs(lengths, nh, nkv, seed=8), gate=True, theta=1e7))
+    got = _run(w, out=torch.full((sum(lengths), nh * 256), float("nan"), device="cuda"))[0].view(torch.int32)
+    cu = w["cu_seqlens"]
+    for r in sorted({0, 1, len(lengths) // 2, len(lengths) - 1}):
+        a, b = int(cu[r]), int(cu[r + 1])
+        alone, _ = _run(dict(w, qkv=w["qkv"][a:b].clone(), pos3=w["pos3"][a:b].clone(), cu_seqlens=np.array([0, b - a], np.int32)))
+        assert torch.equal(alone.view(torch.int32), got[a:b])
+    assert torch.isfinite(got.view(torch.float32)).all()
